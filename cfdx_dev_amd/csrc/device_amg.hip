@@ -39,25 +39,20 @@ constexpr uint32_t kRestartMax = 120;  // largest FGMRES restart
 constexpr uint32_t kGsCoefSlot = 512; // Gram-Schmidt update coefficients (2 * kRestartMax + 2 slots)
 constexpr uint32_t kPcgScalars = 8;   // scalar slots the PCG uses
 
-// Row blocks of the CSR-stream SpMV: consecutive rows up to kStreamNnz
-// entries (and kMaxRowsPerBlock rows); a longer row is a block of its own.
-std::vector<uint32_t> row_blocks(const std::vector<uint32_t>& rowp, uint32_t kStreamNnz) {
+// Row blocks of the CSR-stream SpMV: consecutive rows up to a target of
+// entries (and kMaxRowsPerBlock rows); a row longer than the target is a
+// block of its own. The target is the kernel's LDS capacity `cap`, less on
+// the small coarse levels so that they keep about 1024 workgroups: a level of
+// 42K entries in 11 blocks of 4096 left 245 of the 256 CUs idle.
+std::vector<uint2> row_blocks(const std::vector<uint32_t>& rowp, uint32_t cap) {
     const uint32_t n = uint32_t(rowp.size() - 1);
-    std::vector<uint32_t> b{0};
+    const uint32_t target = std::clamp<uint32_t>(rowp[n] / 1024, 512, cap);
+    std::vector<uint2> b{make_uint2(0, 0)};
     uint32_t row = 0;
     while (row < n) {
-        const uint32_t start = row;
-        if (rowp[row + 1] - rowp[row] > kStreamNnz) {
-            ++row;
-        } else {
-            uint32_t acc = 0;
-            while (row < n && row - start < uint32_t(kMaxRowsPerBlock) &&
-                   acc + (rowp[row + 1] - rowp[row]) <= kStreamNnz) {
-                acc += rowp[row + 1] - rowp[row];
-                ++row;
-            }
-        }
-        b.push_back(row);
+        const uint32_t start = row++;
+        while (row < n && row - start < uint32_t(kMaxRowsPerBlock) && rowp[row + 1] - rowp[start] <= target) ++row;
+        b.push_back(make_uint2(row, rowp[row]));
     }
     return b;
 }

@@ -17,9 +17,9 @@ struct DevCsr {
     uint64_t nnz = 0;
     uint32_t* rowp = nullptr;
     uint32_t* cols = nullptr;
-    uint32_t* blocks = nullptr;  // CSR-stream row blocks of FP64 launches (nblocks + 1 boundaries)
+    uint2* blocks = nullptr;  // CSR-stream row blocks of FP64 launches (nblocks + 1 boundaries: row, first entry)
     uint32_t nblocks = 0;
-    uint32_t* blocks32 = nullptr;  // the same for FP32 launches (smaller blocks)
+    uint2* blocks32 = nullptr;  // the same for FP32 launches (smaller blocks)
     uint32_t nblocks32 = 0;
     double* v64 = nullptr;
     float* v32 = nullptr;

@@ -90,19 +90,37 @@ static __global__ __launch_bounds__(1024) void reduce_partials_kernel(const doub
 
 // ------------------------------------------------------------------ SpMV --
 
-// s + p[b] + p[b+1] + ... + p[e-1], added strictly left to right; the LDS
-// reads of each group of eight are issued together so their latency overlaps
-// while the dependent additions keep the sequential order.
+// s + p[b] + p[b+1] + ... + p[e-1], added strictly left to right. The sum of
+// a long row is a chain of dependent additions, so eight LDS reads are always
+// in flight ahead of the eight additions that use the previous ones.
 template <class T>
 __device__ __forceinline__ T ordered_sum(const T* p, uint32_t b, uint32_t e, T s) {
 #pragma clang fp contract(off)
     uint32_t k = b;
-    for (; k + 8 <= e; k += 8) {
-        T v[8];
+    if (k + 8 <= e) {
+        T v[8], w[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = p[k + j];
+        k += 8;
+        for (; k + 16 <= e; k += 16) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[j] = p[k + j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s += v[j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = p[k + 8 + j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s += w[j];
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) s += v[j];
+    }
+    for (; k + 4 <= e; k += 4) {
+        T v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = p[k + j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s += v[j];
     }
     for (; k < e; ++k) s += p[k];
     return s;
@@ -124,8 +142,33 @@ struct OrderedSum<float> {
 constexpr uint32_t kGroupRowNnz = 12;                // FP32: lanes per row above this mean row length
 constexpr uint32_t kGroupLanes = CFDX_GROUP_LANES;   // power of two, at most 64
 
+// FP32 rows of a block that one lane (16 lanes in a block of long rows) would
+// sum for longer than the whole wavefront: the coarse levels mix rows of a few
+// entries with rows that span the level, and such a row summed by one lane
+// kept a launch of seven workgroups waiting 12 us.
+constexpr uint32_t kWaveRowNnz = 24;
+constexpr uint32_t kGroupRowMax = 128;
+
+// Sums of the rows [b, e) of the lanes with `mine`, one row after the other
+// by the whole wavefront (strided partial sums, fixed butterfly): each such
+// lane receives its row's sum. Collective over the wavefront.
+template <class T>
+__device__ __forceinline__ T wave_row_sums(const T* p, uint32_t b, uint32_t e, bool mine) {
+    const uint32_t lane = threadIdx.x & 63u;
+    T out = T(0);
+    for (uint64_t m = __ballot(mine); m; m &= m - 1) {
+        const int src = __builtin_ctzll(m);
+        const uint32_t rb = __shfl(b, src, 64), re = __shfl(e, src, 64);
+        T s = T(0);
+        for (uint32_t k = rb + lane; k < re; k += 64) s += p[k];
+        s = wave_sum(s);
+        if (int(lane) == src) out = s;
+    }
+    return out;
+}
+
 template <class T, class Init, class Epi, int kStreamNnz = StreamNnz<T>::value>
-__global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint32_t* __restrict__ blocks, uint32_t nb,
+__global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint2* __restrict__ blocks, uint32_t nb,
                                                              const uint32_t* __restrict__ rowp,
                                                              const uint32_t* __restrict__ cols,
                                                              const T* __restrict__ vals, const T* __restrict__ x,
@@ -135,8 +178,8 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint32_t* __r
     __shared__ T prod[kStreamNnz];
     __shared__ double red[4];
     const uint32_t b = xcd_block(blockIdx.x, nb);
-    const uint32_t r0 = blocks[b], r1 = blocks[b + 1];
-    const uint32_t k0 = rowp[r0], k1 = rowp[r1];
+    const uint2 lo = blocks[b], hi = blocks[b + 1];
+    const uint32_t r0 = lo.x, r1 = hi.x, k0 = lo.y, k1 = hi.y;
     double part = 0.0;
     if (k1 - k0 <= uint32_t(kStreamNnz)) {
         // The epilogue inputs of this thread's first row (its offsets, the
@@ -183,15 +226,27 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint32_t* __r
         bool grouped = false;
         if constexpr (!kOrdered) grouped = (k1 - k0) >= kGroupRowNnz * (r1 - r0);
         if (!grouped) {
-            for (uint32_t row = row1; row < r1; row += kBlock) {
+            // Loop bounds uniform in a wavefront (wave_row_sums is collective).
+            for (uint32_t row = row1; row - (threadIdx.x & 63u) < r1; row += kBlock) {
+                const bool live = row < r1;
                 if (row != row1) {
-                    rb = rowp[row];
-                    re = rowp[row + 1];
-                    pre = epi.load(row);
-                    ini = init(row);
+                    rb = live ? rowp[row] : 0u;
+                    re = live ? rowp[row + 1] : 0u;
+                    if (live) {
+                        pre = epi.load(row);
+                        ini = init(row);
+                    }
                 }
-                const T s = ordered_sum(prod, rb - k0, re - k0, ini);
-                part += epi.apply(row, s, pre);
+                T s;
+                if constexpr (kOrdered) {
+                    s = live ? ordered_sum(prod, rb - k0, re - k0, ini) : ini;
+                } else {
+                    const bool longer = live && re - rb > kWaveRowNnz;
+                    s = live && !longer ? ordered_sum(prod, rb - k0, re - k0, ini) : ini;
+                    const T t = wave_row_sums(prod, rb - k0, re - k0, longer);
+                    if (longer) s = ini + t;
+                }
+                if (live) part += epi.apply(row, s, pre);
             }
         } else {
             if constexpr (!kOrdered) {
@@ -205,7 +260,7 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint32_t* __r
                 for (uint32_t row0 = r0; row0 < r1; row0 += kBlock / kGroupLanes) {
                     const uint32_t row = row0 + g;
                     T s = T(0);
-                    if (row < r1)
+                    if (row < r1 && rowp[row + 1] - rowp[row] <= kGroupRowMax)
                         for (uint32_t k = rowp[row] - k0 + lane; k < rowp[row + 1] - k0; k += kGroupLanes)
                             s += prod[k];
 #pragma unroll
@@ -213,24 +268,55 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint32_t* __r
                     if (row < r1 && lane == 0) rsum[row - r0] = s;
                 }
                 __syncthreads();
-                for (uint32_t row = row1; row < r1; row += kBlock) {
+                for (uint32_t row = row1; row - (threadIdx.x & 63u) < r1; row += kBlock) {
+                    const bool live = row < r1;
                     if (row != row1) {
-                        pre = epi.load(row);
-                        ini = init(row);
+                        rb = live ? rowp[row] : 0u;
+                        re = live ? rowp[row + 1] : 0u;
+                        if (live) {
+                            pre = epi.load(row);
+                            ini = init(row);
+                        }
                     }
-                    part += epi.apply(row, ini + rsum[row - r0], pre);
+                    const bool longer = live && re - rb > kGroupRowMax;
+                    const T t = wave_row_sums(prod, rb - k0, re - k0, longer);
+                    if (live) part += epi.apply(row, ini + (longer ? t : rsum[row - r0]), pre);
                 }
             }
         }
     } else if (kOrdered) {
-        // One long row: stream it in chunks, a single thread keeps the
-        // sequential sum.
+        // One long row: streamed in chunks, a single thread keeps the
+        // sequential sum while the other wavefronts fill the next chunk.
+        constexpr uint32_t kHalf = uint32_t(kStreamNnz) / 2;
         T s = init(r0);
-        for (uint32_t base = k0; base < k1; base += kStreamNnz) {
-            const uint32_t len = (k1 - base) < uint32_t(kStreamNnz) ? (k1 - base) : uint32_t(kStreamNnz);
-            for (uint32_t k = threadIdx.x; k < len; k += kBlock) prod[k] = vals[base + k] * x[cols[base + k]];
-            __syncthreads();
-            if (threadIdx.x == 0) s = ordered_sum(prod, 0u, len, s);
+        auto fill = [&](uint32_t base, T* dst, uint32_t first, uint32_t step) {
+            const uint32_t len = min(k1 - base, kHalf);
+            for (uint32_t k = first; k < len; k += 4 * step) {
+                T v[4];
+                uint32_t c[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint32_t kk = k + uint32_t(u) * step;
+                    c[u] = kk < len ? cols[base + kk] : 0u;
+                    v[u] = kk < len ? vals[base + kk] : T(0);
+                }
+                T xv[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) xv[u] = x[c[u]];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (k + uint32_t(u) * step < len) dst[k + uint32_t(u) * step] = v[u] * xv[u];
+            }
+        };
+        fill(k0, prod, threadIdx.x, kBlock);
+        __syncthreads();
+        uint32_t h = 0;
+        for (uint32_t base = k0; base < k1; base += kHalf, h ^= 1u) {
+            if (threadIdx.x >= 64) {
+                if (base + kHalf < k1) fill(base + kHalf, prod + (h ^ 1u) * kHalf, threadIdx.x - 64, kBlock - 64);
+            } else if (threadIdx.x == 0) {
+                s = ordered_sum(prod + h * kHalf, 0u, min(k1 - base, kHalf), s);
+            }
             __syncthreads();
         }
         if (threadIdx.x == 0) part = epi(r0, s);
@@ -836,33 +922,55 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(uint32_t n, const T* __res
 // -------------------------------------------------------- coarse solve --
 
 // Replays the dense partial-pivot elimination of the coarsest level
-// (amg_preconditioner.h:2603-2663) with factors computed once at setup.
-// One thread; n <= 16.
+// (amg_preconditioner.h:2603-2663) with factors computed once at setup. One
+// wavefront, order n <= 17 (16 unknowns, bordered); nr unknowns (n or n - 1),
+// the border's right-hand side is 0. Lane i owns component i: a forward step
+// updates every component at once, each with the operations of the sequential
+// elimination. The back substitution subtracts a row's terms in ascending
+// column order, a chain that only lane ii can follow, so its products are
+// formed by the lanes and read in order. 24 us with one lane and its arrays in
+// scratch memory, see coarse_lu_solve.
 template <class T>
-__global__ void coarse_lu_kernel(uint32_t n, uint32_t nr, const uint32_t* __restrict__ piv,
+__device__ __forceinline__ void coarse_lu_solve(uint32_t n, uint32_t nr, const uint32_t* __restrict__ piv,
+                                                const double* __restrict__ factor, const double* __restrict__ upper,
+                                                const T* r, T* x, double* sm /* 2 * 17 * 17 */) {
+#pragma clang fp contract(off)
+    const uint32_t lane = threadIdx.x & 63u;
+    double* F = sm;
+    double* U = sm + 17 * 17;
+    for (uint32_t k = lane; k < n * n; k += 64) {
+        F[k] = factor[k];
+        U[k] = upper[k];
+    }
+    double b = lane < nr ? double(r[lane]) : 0.0;
+    const uint32_t pv = lane < n ? piv[lane] : 0u;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint32_t p = __shfl(pv, int(k), 64);
+        const double bk = __shfl(b, int(k), 64), bp = __shfl(b, int(p), 64);
+        if (lane == k) b = bp;
+        else if (lane == p) b = bk;
+        if (lane > k && lane < n) b -= F[k * n + lane] * bp;
+    }
+    double s = 0.0;  // lane i: component i of the solution once it is known
+    for (uint32_t ii = n; ii-- > 0;) {
+        // Products of row ii, lane j holds upper[ii][j] s[j].
+        const double t = lane > ii && lane < n ? U[ii * n + lane] * s : 0.0;
+        double sum = __shfl(b, int(ii), 64);
+        for (uint32_t j = ii + 1; j < n; ++j) sum -= __shfl(t, int(j), 64);
+        if (lane == ii) s = sum / U[ii * n + ii];
+    }
+    if (lane < nr) x[lane] = T(s);
+}
+
+template <class T>
+__global__ __launch_bounds__(64) void coarse_lu_kernel(uint32_t n, uint32_t nr, const uint32_t* __restrict__ piv,
                                  const double* __restrict__ factor, const double* __restrict__ upper,
                                  const T* __restrict__ r, T* __restrict__ x) {
-#pragma clang fp contract(off)
-    // n: order of the factored system (at most 17: 16 unknowns, bordered);
-    // nr: unknowns of the level (n or n - 1); the border's right-hand side is 0.
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double b[17], s[17];
-    for (uint32_t i = 0; i < n; ++i) b[i] = i < nr ? double(r[i]) : 0.0;
-    for (uint32_t k = 0; k < n; ++k) {
-        const uint32_t p = piv[k];
-        if (p != k) {
-            const double t = b[k];
-            b[k] = b[p];
-            b[p] = t;
-        }
-        for (uint32_t i = k + 1; i < n; ++i) b[i] -= factor[k * n + i] * b[k];
-    }
-    for (uint32_t ii = n; ii-- > 0;) {
-        double sum = b[ii];
-        for (uint32_t j = ii + 1; j < n; ++j) sum -= upper[ii * n + j] * s[j];
-        s[ii] = sum / upper[ii * n + ii];
-    }
-    for (uint32_t i = 0; i < nr; ++i) x[i] = T(s[i]);
+    __shared__ double sm[2 * 17 * 17];
+    coarse_lu_solve<T>(n, nr, piv, factor, upper, r, x, sm);
 }
 
 // Partial sums of v over grid-stride chunks (the mean of the constant null
