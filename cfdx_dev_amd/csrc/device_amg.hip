@@ -16,6 +16,7 @@
 #include "device_amg.hpp"
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -26,6 +27,7 @@
 #include <numeric>
 #include <stdexcept>
 
+#include "coarse_tail.hpp"
 #include "device_util.hpp"
 #include "kernels.hpp"
 
@@ -33,6 +35,7 @@ namespace cfdxhip {
 
 namespace {
 
+constexpr uint32_t kLastSweeps = 24;  // Jacobi sweeps of a coarsest level without dense factors
 constexpr uint32_t kGsStride = 4096;  // partial stride (and grid cap) of the Gram-Schmidt reductions
 constexpr uint32_t kScalars = 1024;   // device scalar slots
 constexpr uint32_t kRestartMax = 120;  // largest FGMRES restart
@@ -214,6 +217,8 @@ void DeviceAmg::release() {
     dfree(lu_.factor);
     dfree(lu_.upper);
     lu_ = DevCoarseLU{};
+    for (void* p : tail_.mem) (void)hipFree(p);
+    tail_ = Tail{};
     dfree(d_perm0_);
     dfree(partials_);
     dfree(aux_part_);
@@ -384,6 +389,7 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
             lu_.upper = upload(lu.upper, stream_);
         }
     }
+    build_tail();
     const uint32_t n0 = lv_[0].n;
     d_perm0_ = upload(lv_[0].new_of_old, stream_);
     partial_stride_ = std::max<uint64_t>({spmv_groups<double>(lv_[0].A), spmv_groups<float>(lv_[0].A), 4096});
@@ -522,6 +528,7 @@ void DeviceAmg::set_chebyshev_lambda(const std::vector<double>& lambda_max) {
         if (l > 0 && cheb_degree_coarse_ > 0) cheb_deg_[l] = cheb_degree_coarse_;
         chebyshev_coefficients(lambda_max[l], cheb_ratio_, cheb_deg_[l], cheb_c1_[l], cheb_c2_[l]);
     }
+    upload_tail();
 }
 
 template <class T>
@@ -649,11 +656,217 @@ void DeviceAmg::smooth(uint32_t l, const T* b, T*& x, uint32_t sweeps, bool from
         spmv_jacobi_sweeps<T>(lv_[l], b, x, sweeps, from_zero);
 }
 
+namespace {
+
+// A matrix packed for the coarse end: rows of at most kTailLaneRow entries in
+// lanes, longer ones listed. src: the CSR entry of each stored value (lane
+// slots, then the long rows' entries).
+struct TailPack {
+    uint32_t first[kTailWaves], count[kTailWaves];
+    std::vector<uint32_t> ctl, src;
+    std::vector<uint16_t> cols, lcols;
+    std::vector<uint4> groups, lrows;
+    uint32_t lane_values = 0;
+};
+
+// False when a lane would hold more than kTailBatches.
+bool pack_tail(const std::vector<uint32_t>& rowp, const std::vector<uint32_t>& cols, uint32_t ncols, TailPack& t) {
+    const uint32_t n = uint32_t(rowp.size() - 1);
+    auto len = [&](uint32_t r) { return rowp[r + 1] - rowp[r]; };
+    std::vector<uint32_t> rows, longs;
+    uint64_t grouped = 0;  // entries of rows that share a group
+    for (uint32_t r = 0; r < n; ++r) {
+        (len(r) <= kTailLaneRow ? rows : longs).push_back(r);
+        if (len(r) > kTailLaneRow && len(r) < kTailChunk / 2) grouped += len(r);
+    }
+    // Groups of longer rows, about one for each wavefront; a row of half a
+    // chunk and more is alone.
+    std::stable_sort(longs.begin(), longs.end(), [&](uint32_t a, uint32_t b) { return len(a) > len(b); });
+    const uint32_t target = uint32_t(std::min<uint64_t>(kTailChunk, grouped / kTailWaves + kTailLaneRow));
+    for (size_t i = 0; i < longs.size();) {
+        uint4 g = make_uint4(uint32_t(t.lcols.size()), 0, uint32_t(t.lrows.size()), 0);
+        do {
+            const uint32_t r = longs[i];
+            t.lrows.push_back(make_uint4(r, g.y, g.y + len(r), 0));
+            t.lcols.insert(t.lcols.end(), cols.begin() + rowp[r], cols.begin() + rowp[r + 1]);
+            g.y += len(r);
+            ++g.w;
+            ++i;
+        } while (i < longs.size() && g.w < 64 && len(longs[i - g.w]) < kTailChunk / 2 &&
+                 g.y + len(longs[i]) <= target);
+        t.groups.push_back(g);
+    }
+    auto need = [&](uint32_t r) { return std::max<uint32_t>(1, (len(r) + 7) / 8); };
+    std::stable_sort(rows.begin(), rows.end(), [&](uint32_t a, uint32_t b) { return need(a) > need(b); });
+    // Longest first over the lanes, back and forth: neighbouring lanes, and
+    // so the lanes of a wavefront, end up with like counts.
+    std::vector<std::vector<uint32_t>> lane(kTailThreads);
+    for (size_t i = 0; i < rows.size(); ++i) {
+        const uint32_t pos = uint32_t(i % kTailThreads);
+        lane[(i / kTailThreads) % 2 ? kTailThreads - 1 - pos : pos].push_back(rows[i]);
+    }
+    uint32_t total = 0;
+    for (uint32_t w = 0; w < kTailWaves; ++w) {
+        uint32_t most = 0;
+        for (uint32_t l = 0; l < 64; ++l) {
+            uint32_t c = 0;
+            for (uint32_t r : lane[w * 64 + l]) c += need(r);
+            most = std::max(most, c);
+        }
+        if (most > kTailBatches) return false;
+        t.first[w] = total;
+        t.count[w] = most;
+        total += most;
+    }
+    t.lane_values = total * 512;
+    t.ctl.assign(size_t(total) * 64, 0);
+    t.cols.assign(t.lane_values, uint16_t(ncols));
+    t.src.assign(t.lane_values, kTailPad);
+    for (uint32_t w = 0; w < kTailWaves; ++w)
+        for (uint32_t l = 0; l < 64; ++l) {
+            uint32_t at = t.first[w];
+            for (uint32_t r : lane[w * 64 + l])
+                for (uint32_t q = 0; q < need(r); ++q, ++at) {
+                    t.ctl[size_t(at) * 64 + l] = r | (q == 0 ? kTailStart : 0u) | (q + 1 == need(r) ? kTailEnd : 0u);
+                    for (uint32_t j = 0; j < 8 && 8 * q + j < len(r); ++j) {
+                        const uint32_t k = rowp[r] + 8 * q + j;
+                        t.cols[(size_t(at) * 64 + l) * 8 + j] = uint16_t(cols[k]);
+                        t.src[((size_t(at) * 4 + j / 2) * 64 + l) * 2 + j % 2] = k;
+                    }
+                }
+        }
+    for (const uint4& m : t.lrows)
+        for (uint32_t k = rowp[m.x]; k < rowp[m.x + 1]; ++k) t.src.push_back(k);
+    return true;
+}
+
+}  // namespace
+
+// The levels one workgroup runs: the longest run of levels down to the
+// coarsest, at least two, whose matrices fit its lanes and whose vectors fit
+// LDS (160 KiB). Mean removals of the constant null space are launches
+// between the sweeps: such hierarchies keep the launches.
+void DeviceAmg::build_tail() {
+    Tail& t = tail_;
+    const uint32_t L = uint32_t(lv_.size());
+    t.first = L;
+    if (cns_ || !has64_) return;
+    constexpr uint32_t kLds = 160 * 1024;
+    constexpr uint32_t stage_cells = kTailWaves * kTailChunk;  // the coarsest factors use it too
+    static_assert(stage_cells >= 2 * 17 * 17, "coarse_lu_solve's arrays");
+    std::vector<std::array<TailPack, 3>> packs;  // A, R, P of the levels, coarsest first
+    uint32_t cells = 0;
+    while (t.first > 0 && L - t.first < kTailMaxLevels) {
+        const DevLevel& D = lv_[t.first - 1];
+        const uint32_t more = 2 * D.n + 2;
+        if (D.n > kTailMaxRows || D.A.nnz > 4 * uint64_t(kTailThreads) * kTailLaneRow) break;
+        if ((cells + more + 3 * (D.n + 1) + stage_cells) * sizeof(double) > kLds) break;
+        std::array<TailPack, 3> p;
+        bool ok = true;
+        for (int m = 0; ok && m < (t.first == L ? 1 : 3); ++m) {
+            const DevCsr& M = m == 0 ? D.A : m == 1 ? D.R : D.P;
+            std::vector<uint32_t> rowp(size_t(M.n) + 1), cols(M.nnz);
+            HIP_OK(hipMemcpyAsync(rowp.data(), M.rowp, rowp.size() * 4, hipMemcpyDeviceToHost, stream_));
+            HIP_OK(hipMemcpyAsync(cols.data(), M.cols, cols.size() * 4, hipMemcpyDeviceToHost, stream_));
+            HIP_OK(hipStreamSynchronize(stream_));
+            ok = pack_tail(rowp, cols, M.ncols, p[m]);
+        }
+        if (!ok) break;
+        packs.push_back(std::move(p));
+        cells += more;
+        --t.first;
+    }
+    if (L - t.first < 2) {
+        t.first = L;
+        return;
+    }
+    auto put = [&](const auto& v) {
+        auto* d = upload(v, stream_);
+        t.mem.push_back(d);
+        return d;
+    };
+    t.host.resize(L - t.first);
+    uint32_t at = 0;
+    for (uint32_t k = 0; k < t.host.size(); ++k) {
+        const uint32_t l = t.first + k;
+        DevLevel& D = lv_[l];
+        TailLevel& H = t.host[k];
+        std::memset(&H, 0, sizeof(H));
+        H.inv = D.inv64;
+        H.x = at;
+        H.b = at + D.n + 1;
+        at += 2 * D.n + 2;
+        auto& p = packs[t.host.size() - 1 - k];
+        for (int m = 0; m < (l + 1 == L ? 1 : 3); ++m) {
+            const DevCsr& M = m == 0 ? D.A : m == 1 ? D.R : D.P;
+            TailMat& X = m == 0 ? H.A : m == 1 ? H.R : H.P;
+            X.n = M.n;
+            X.ngroups = uint32_t(p[m].groups.size());
+            std::copy(p[m].first, p[m].first + kTailWaves, X.first);
+            std::copy(p[m].count, p[m].count + kTailWaves, X.count);
+            X.ctl = put(p[m].ctl);
+            X.cols = reinterpret_cast<const uint4*>(put(p[m].cols));
+            X.groups = put(p[m].groups);
+            X.lrows = put(p[m].lrows);
+            X.lcols = put(p[m].lcols);
+            double* v = dalloc<double>(p[m].src.size());
+            t.mem.push_back(v);
+            X.vals = v;
+            X.lvals = v + p[m].lane_values;
+            const uint32_t n = uint32_t(p[m].src.size());
+            const uint32_t* src = put(p[m].src);
+            tail_values_kernel<<<grid_for(n), kBlock, 0, stream_>>>(n, src, M.v64, v);
+            if (m == 0) t.refill.push_back({l, n, src, v});
+        }
+    }
+    t.cells = at;
+    t.stage = at + 3 * (lv_[t.first].n + 1);
+    t.lds_bytes = (t.stage + stage_cells) * sizeof(double);
+    t.dev = dalloc<TailLevel>(t.host.size());
+    t.mem.push_back(t.dev);
+    for (const auto kernel : {coarse_tail_kernel<false>, coarse_tail_kernel<true>})
+        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   int(kLds)));
+    upload_tail();
+}
+
+// The level descriptors, which carry the Chebyshev coefficients.
+void DeviceAmg::upload_tail() {
+    Tail& t = tail_;
+    if (!t.dev) return;
+    for (size_t k = 0; k < t.host.size() && t.first + k < cheb_deg_.size(); ++k) {
+        const size_t l = t.first + k;
+        TailLevel& H = t.host[k];
+        H.degree = cheb_deg_[l];
+        std::copy(cheb_c1_[l].begin(), cheb_c1_[l].end(), H.c1);
+        std::copy(cheb_c2_[l].begin(), cheb_c2_[l].end(), H.c2);
+    }
+    HIP_OK(hipMemcpyAsync(t.dev, t.host.data(), t.host.size() * sizeof(t.host[0]), hipMemcpyHostToDevice, stream_));
+    HIP_OK(hipStreamSynchronize(stream_));
+}
+
+void DeviceAmg::refill_tail() {
+    for (const auto& f : tail_.refill)
+        tail_values_kernel<<<grid_for(f.n), kBlock, 0, stream_>>>(f.n, f.src, lv_[f.level].A.v64, f.dst);
+}
+
 template <class T>
 bool DeviceAmg::vcycle_t(uint32_t l, const T* b, T*& x) {
     DevLevel& L = lv_[l];
     T* const* xs = x_of<T>(L);
     x = xs[0];
+    if constexpr (sizeof(T) == 8) {
+        if (l == tail_.first) {
+            const bool dense = lv_.back().n <= 16;
+            if (dense && !lu_.ok) return false;
+            const auto kernel =
+                smoother64_ == SMOOTHER_CHEBYSHEV ? coarse_tail_kernel<true> : coarse_tail_kernel<false>;
+            kernel<<<1, kTailThreads, tail_.lds_bytes, stream_>>>(
+                tail_.dev, uint32_t(tail_.host.size()), tail_.cells, tail_.stage, omega_, pre_, post_, kLastSweeps,
+                TailLu{dense ? lu_.n : 0u, lu_.piv, lu_.factor, lu_.upper}, b, x);
+            return true;
+        }
+    }
     if (l + 1 == lv_.size()) {
         if (L.n <= 16) {
             if (!lu_.ok) return false;
@@ -661,7 +874,7 @@ bool DeviceAmg::vcycle_t(uint32_t l, const T* b, T*& x) {
             if (cns_) remove_mean<T>(x, L.n);
             return true;
         }
-        spmv_jacobi_sweeps<T>(L, b, x, 24, true);
+        spmv_jacobi_sweeps<T>(L, b, x, kLastSweeps, true);
         return true;
     }
     const bool cheb = (sizeof(T) == 8 ? smoother64_ : smoother32_) == SMOOTHER_CHEBYSHEV;

@@ -62,6 +62,34 @@ struct DevLevel {
     std::vector<uint32_t> new_of_old;
 };
 
+// Levels of the FP64 V-cycle's single-launch coarse end (layout:
+// coarse_tail.hpp).
+constexpr int kTailWaves = 8;
+
+struct TailMat {
+    uint32_t n;                  // rows
+    uint32_t ngroups;            // groups of longer rows
+    uint32_t first[kTailWaves];  // first batch of each wavefront
+    uint32_t count[kTailWaves];
+    const uint32_t* ctl;         // [batch][lane]
+    const uint4* cols;           // [batch][lane]: eight 16-bit columns
+    const double* vals;          // [batch][pair of slots][lane]
+    const uint4* groups;         // first entry, entries, first row in lrows, rows
+    const uint4* lrows;          // row, first and end product in its group
+    const uint16_t* lcols;
+    const double* lvals;
+};
+
+// x and b: offsets of the level's vectors in LDS (n + 1 cells each, the last
+// one of x holds 1.0). R and P lead to the next level; the last has none.
+struct TailLevel {
+    TailMat A, R, P;
+    const double* inv;
+    uint32_t x, b;
+    uint32_t degree;       // Chebyshev degree
+    double c1[16], c2[16];  // its coefficients
+};
+
 struct DevCoarseLU {
     bool ok = false;
     uint32_t n = 0;
@@ -324,6 +352,27 @@ private:
     // stride 0: the hierarchy's own partial-sum stride; src null: scal_.
     void reduce(const double* partials, uint32_t n, uint32_t count, double* out, uint64_t stride = 0);
     bool fetch_scalars(uint32_t count, const double* src = nullptr);
+
+    // The FP64 V-cycle's single-launch coarse end (coarse_tail.hpp): its
+    // first level (the number of levels: none), the level descriptors on the
+    // host and the device, the LDS layout, and what refills the packed
+    // matrices from the levels' CSR values.
+    struct Tail {
+        struct Refill {
+            uint32_t level, n;
+            const uint32_t* src;
+            double* dst;
+        };
+        uint32_t first = 0, cells = 0, stage = 0, lds_bytes = 0;
+        std::vector<TailLevel> host;
+        TailLevel* dev = nullptr;
+        std::vector<Refill> refill;
+        std::vector<void*> mem;  // its device arrays
+    };
+    void build_tail();
+    void upload_tail();  // after new Chebyshev coefficients
+    void refill_tail();  // after new values of the levels' CSR copies
+    Tail tail_;
 
     std::vector<DevLevel> lv_;
     std::vector<RefreshLevel> rf_;

@@ -1240,6 +1240,7 @@ bool DeviceAmg::refresh_device(const double* d_vals, const AmgConfig& cfg, doubl
                                                                              D.A.hvals);
         }
     }
+    refill_tail();
     rf_cur_ = stg;
     omega_ = wv;
     omega = wv;

@@ -1,0 +1,52 @@
+"""The coarse end of the FP64 V-cycle, run by one workgroup from the first
+level that fits it (cfdx_dev_amd/csrc/coarse_tail.hpp), against the oracle bit
+for bit, where it can go wrong:
+* the whole hierarchy in one launch, and only its end;
+* rows of more than 64 entries in groups (classical C/F on the 2-D Poisson
+  square) and alone in their group (arrow rows of the filtered channel
+  hierarchy, longer than one staged chunk);
+* a coarsest level without dense factors (24 sweeps), policies of 2 and 6
+  sweeps, Chebyshev smoothing with a recurrence;
+* after a numeric refresh (packed values, damping and coefficients renewed).
+"""
+import numpy as np
+import pytest
+
+import cfdx_dev_amd as cx
+from systems import box_mesh, channel_system, pressure_system
+from test_poisson_mms import mms_system
+
+pytestmark = pytest.mark.gpu
+
+FILTER = dict(prolongator_filter=0.2, filter_keeps_aggregate=True)
+CASES = {
+    "whole_box": ("sa", "balanced", {}, lambda o: pressure_system(o, box_mesh(8, 7, 6, seed=5), seed=5)),
+    "end_of_box": ("sa", "low", {}, lambda o: pressure_system(o, box_mesh(24, 23, 22, seed=5), seed=5)),
+    "grouped_rows": ("boomer", "balanced", {}, lambda o: mms_system(o, 128)),
+    "grouped_rows_small": ("boomer", "balanced", {}, lambda o: mms_system(o, 50)),
+    "arrow_rows": ("sa", "balanced", FILTER, lambda o: channel_system(o, (80, 32, 30), 3, 1)),
+    "chebyshev": ("sa", "balanced", dict(FILTER, smoother="chebyshev"),
+                  lambda o: channel_system(o, (40, 16, 14), 3, 2)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_coarse_end_bit_identical(oracle, name):
+    method, policy, opt, make = CASES[name]
+    s = make(oracle)
+    ao = oracle.amg(method, policy=policy, **opt)
+    assert ao.setup(s["n"], s["rowp"], s["cols"], s["vals"])
+    ap = cx.NativeAMGPreconditioner(method=method, policy=policy, **opt)
+    assert ap.setup(s["n"], s["rowp"], s["cols"], s["vals"]), ap.last_error()
+    assert ap.num_levels() > 2
+    rng = np.random.default_rng(11)
+    for refresh in (False, True):
+        if refresh:
+            # S A S with powers of two keeps every pruning decision.
+            d = np.exp2(np.arange(s["n"]) % 2)
+            rows = np.repeat(np.arange(s["n"]), np.diff(s["rowp"].astype(np.int64)))
+            vals = s["vals"] * d[rows] * d[s["cols"]]
+            assert ao.update_values(vals) == ap.update_values(vals)
+        for _ in range(2):
+            r = rng.normal(size=s["n"])
+            assert np.array_equal(ao.apply(r), ap.apply(r))
