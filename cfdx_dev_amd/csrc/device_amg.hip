@@ -120,7 +120,7 @@ void build_sell(DevCsr& D, const std::vector<uint32_t>& rowp, hipStream_t s) {
                                                                                 D.scols32);
         D.s32 = dalloc<float>(slots);
     }
-    sell_values(D, s);
+    sell_values(D, s, true);
 }
 
 // Relabels a CSR: row i -> rp[i], column j -> cp[j], entry order kept.
@@ -143,16 +143,17 @@ void permute_csr(const HCsr& A, const std::vector<uint32_t>& rp, const std::vect
 
 }  // namespace
 
-// Fills the SELL values of D from its CSR values (padding slots hold 0).
-void sell_values(DevCsr& D, hipStream_t s) {
+// Fills the SELL values of D from its CSR values (padding slots hold 0, from
+// the first fill on).
+void sell_values(DevCsr& D, hipStream_t s, bool first) {
     if (!D.nslices) return;
     const uint32_t slots = uint32_t(D.sell_entries);
     if (D.s64) {
-        fill_kernel<double><<<grid_for(slots), kBlock, 0, s>>>(slots, 0.0, D.s64);
+        if (first) fill_kernel<double><<<grid_for(slots), kBlock, 0, s>>>(slots, 0.0, D.s64);
         sell_scatter_kernel<double><<<grid_for(D.n), kBlock, 0, s>>>(D.n, D.rowp, D.soff, D.v64, D.s64);
     }
     if (D.s32) {
-        fill_kernel<float><<<grid_for(slots), kBlock, 0, s>>>(slots, 0.0f, D.s32);
+        if (first) fill_kernel<float><<<grid_for(slots), kBlock, 0, s>>>(slots, 0.0f, D.s32);
         sell_scatter_sorted_kernel<float><<<grid_for(D.n), kBlock, 0, s>>>(D.n, D.rowp, D.cols, D.soff, D.v32,
                                                                              D.s32);
     }

@@ -111,8 +111,8 @@ struct SolveStats {
 };
 
 // Fills the SELL-64 values of a matrix from its CSR values (no-op without a
-// SELL copy; padding slots hold 0).
-void sell_values(DevCsr& D, hipStream_t s);
+// SELL copy); first: the padding slots too.
+void sell_values(DevCsr& D, hipStream_t s, bool first);
 
 // Caller <-> solve ordering moves on the device (new_of_old on the device).
 void scatter_d2d(uint32_t n, const uint32_t* perm, const double* src, double* dst, hipStream_t s);
@@ -129,6 +129,35 @@ constexpr uint64_t kNoAllocAlign = 256;
 bool noalloc_scratch(int device, unsigned char*& ptr, std::string& err);
 
 class DeviceAmg;
+
+// One level as the refresh's batched kernels see it: a launch covers all
+// levels, each with a range of workgroups (first_* of the next entry ends it).
+struct RefreshView {
+    uint32_t n;
+    uint32_t first_wg;     // 256-row workgroups (elementwise kernels, 256-row tiles)
+    uint32_t first_block;  // CSR-stream row blocks
+    uint32_t row0;         // offset of the level's rows in the work vectors
+    // solve ordering
+    const uint2* blocks;
+    const uint32_t* rowp;
+    const uint32_t* cols;
+    const double* vals;
+    const double* inv;
+    const uint32_t* perm;  // new_of_old
+    // reference ordering, current and staged values
+    const uint32_t* arow;
+    const uint32_t* acol;
+    const double* aval[2];
+    const double* rinv[2];
+};
+
+// Lanczos scalars of a level.
+constexpr uint32_t kLanczosMax = 32;
+struct LanczosState {
+    double norm, a, bprev, b;
+    uint32_t count, stop;
+    double alpha[kLanczosMax], beta[kLanczosMax];
+};
 
 // A preconditioner stage run ahead of (and around) the FP32 V-cycle inside
 // mixed FGMRES: z = stage(r) on FP32 vectors in the solve ordering.
@@ -190,8 +219,11 @@ public:
         double* apv = nullptr;
         uint32_t* c_off = nullptr;
         uint32_t* c_col = nullptr;
-        uint32_t* c_row = nullptr;  // row of each unpruned coarse entry
-        uint32_t c_maxrow = 0;      // longest unpruned coarse row
+        // Coarse rows the Galerkin product gives a wavefront or a workgroup
+        // (row, tile of columns) each; the others share a wavefront.
+        uint32_t* c_mid = nullptr;
+        uint2* c_heavy = nullptr;
+        uint32_t c_nmid = 0, c_nheavy = 0;
         double* cv = nullptr;
         uint32_t* t_off = nullptr;
         uint32_t* t_row = nullptr;
@@ -344,7 +376,10 @@ private:
     bool build_refresh(const HostHierarchy& h, std::string& err, std::vector<RefreshLevel>* adopt = nullptr);
     // Normalised Gershgorin bound over all levels of the refresh state's
     // values `slot` (the damping certificate's input).
-    bool gershgorin_bound(uint32_t slot, bool& certified, double& mb);
+    // Launches it for all levels (results in rf_host_ after read_refresh).
+    void launch_gershgorin(uint32_t slot);
+    void read_refresh(bool coarsest, uint32_t slot);
+    bool gershgorin_bound(bool& certified, double& mb) const;
     // Lanczos eigenvalue estimates of every level's committed matrix.
     std::vector<double> lanczos_bounds(const AmgConfig& cfg);
     void release_refresh();
@@ -377,8 +412,15 @@ private:
     std::vector<DevLevel> lv_;
     std::vector<RefreshLevel> rf_;
     uint32_t rf_cur_ = 0;        // which aval holds the committed values
-    int* rf_flags_ = nullptr;    // refresh error flags
-    double* rf_work_ = nullptr;  // Lanczos vectors, block partials, maxima, scalars
+    int* rf_flags_ = nullptr;    // refresh error flags, per level
+    double* rf_work_ = nullptr;  // Lanczos vectors and tile sums, Gershgorin rows
+    RefreshView* rf_view_ = nullptr;  // the levels as the batched kernels see them
+    std::vector<RefreshView> rf_view_host_;
+    LanczosState* rf_lz_ = nullptr;
+    double* rf_ub_ = nullptr;        // Gershgorin bound per level
+    std::vector<int> rf_host_flags_;
+    std::vector<double> rf_host_ub_;
+    HCsr rf_coarsest_;               // pattern and fetched values of the coarsest level
     DevCoarseLU lu_;
     double omega_ = 0.7;
     uint32_t pre_ = 6, post_ = 6;

@@ -68,27 +68,6 @@ __global__ __launch_bounds__(kBlock) void finite_check_kernel(uint64_t n, const 
     if (i < n && !isfinite(v[i])) flags[kBadInput] = 1;
 }
 
-// build_diagonal: inv[i] = 1 / a_ii, failing on |a_ii| <= 1e-30.
-__global__ __launch_bounds__(kBlock) void inv_diag_kernel(uint32_t n, const uint32_t* __restrict__ rowp,
-                                                          const uint32_t* __restrict__ cols,
-                                                          const double* __restrict__ vals, double* __restrict__ inv,
-                                                          int* __restrict__ flags) {
-#pragma clang fp contract(off)
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    double d = 0.0;
-    for (uint32_t k = rowp[i]; k < rowp[i + 1]; ++k)
-        if (cols[k] == i) d += vals[k];
-    if (!isfinite(d) || fabs(d) <= 1e-30) {
-        flags[kBadDiagonal] = 1;
-        inv[i] = 0.0;
-        return;
-    }
-    const double r = 1.0 / d;
-    if (!isfinite(r)) flags[kBadDiagonal] = 1;
-    inv[i] = r;
-}
-
 __device__ __forceinline__ uint32_t lower_bound_u32(const uint32_t* __restrict__ a, uint32_t lo, uint32_t hi,
                                                     uint32_t key) {
     while (lo < hi) {
@@ -99,107 +78,319 @@ __device__ __forceinline__ uint32_t lower_bound_u32(const uint32_t* __restrict__
     return lo;
 }
 
-// Galerkin numeric products (galerkin_csr_product.h's numeric pass), one
-// thread per output entry. The reference accumulates row by row: for AP,
-// apv[i, c] += a_ij p_jc over A's entries (i, j) in row order; for P^T AP,
-// cv[c, k] += p_ic apv[i, k] over the fine rows i of the transpose plan in
-// ascending order. A given output entry receives its contributions in that
-// same order (each A entry matches at most one P entry of the column, each
-// fine row at most one AP entry), so summing them per entry from 0 gives the
-// reference's values bit for bit, with a long row's work spread over its
-// entries.
+// build_diagonal: inv[i] = 1 / a_ii, failing on |a_ii| <= 1e-30. Columns
+// ascend strictly, so the diagonal is found by bisection: a scan of the rows
+// that span a coarse level took one lane 340 us.
+__global__ __launch_bounds__(kBlock) void inv_diag_kernel(uint32_t n, const uint32_t* __restrict__ rowp,
+                                                          const uint32_t* __restrict__ cols,
+                                                          const double* __restrict__ vals, double* __restrict__ inv,
+                                                          int* __restrict__ flags) {
+#pragma clang fp contract(off)
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t e = rowp[i + 1], k = lower_bound_u32(cols, rowp[i], e, i);
+    const double d = k < e && cols[k] == i ? vals[k] : 0.0;
+    if (!isfinite(d) || fabs(d) <= 1e-30) {
+        flags[kBadDiagonal] = 1;
+        inv[i] = 0.0;
+        return;
+    }
+    const double r = 1.0 / d;
+    if (!isfinite(r)) flags[kBadDiagonal] = 1;
+    inv[i] = r;
+}
+
+// Lane `src`'s value (src uniform).
+__device__ __forceinline__ double lane_value(double v, int src) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
+                            __builtin_amdgcn_readlane(__double2loint(v), src));
+}
+
+// acc + the values of the lanes in `m`, in lane order.
+__device__ __forceinline__ double add_lanes(double acc, double v, uint64_t m) {
+#pragma clang fp contract(off)
+    for (; m; m &= m - 1) acc += lane_value(v, __builtin_ctzll(m));
+    return acc;
+}
+
+// Galerkin numeric products (galerkin_csr_product.h's numeric pass). The
+// reference accumulates row by row: for AP, apv[i, c] += a_ij p_jc over A's
+// entries (i, j) in row order; for P^T AP, cv[c, k] += p_ic apv[i, k] over the
+// fine rows i of the transpose plan in ascending order. A given output entry
+// receives its contributions in that same order (each A entry matches at most
+// one P entry of the column, each fine row at most one AP entry), so summing
+// them per entry from 0 gives the reference's values bit for bit.
+//
+// AP: one thread per output entry (i, c). Its contributions are the j common
+// to A's row i and to the fine rows of c (column c of P), both ascending: the
+// thread walks the shorter list and looks each j up in the other. On the
+// coarse levels some rows of A span the level: walking those for each of their
+// AP entries took 1.24 ms on a level of 4.6K rows. Entries where both lists
+// are long are walked by the whole wavefront, 64 candidates at a time, the
+// hits added in order.
 __global__ __launch_bounds__(kBlock) void galerkin_ap_entries_kernel(
     uint64_t m, const uint32_t* __restrict__ ap_row, const uint32_t* __restrict__ ap_col,
     const uint32_t* __restrict__ arow, const uint32_t* __restrict__ acol, const double* __restrict__ aval,
     const uint32_t* __restrict__ prow, const uint32_t* __restrict__ pcol, const double* __restrict__ pval,
+    const uint32_t* __restrict__ t_off, const uint32_t* __restrict__ t_row, const uint32_t* __restrict__ t_pos,
     double* __restrict__ apv, int* __restrict__ flags) {
 #pragma clang fp contract(off)
     const uint64_t p = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (p >= m) return;
-    const uint32_t i = ap_row[p], col = ap_col[p];
-    double acc = 0.0;
-    for (uint32_t k = arow[i]; k < arow[i + 1]; ++k) {
-        const uint32_t j = acol[k];
-        const uint32_t e = prow[j + 1];
-        const uint32_t q = lower_bound_u32(pcol, prow[j], e, col);
-        if (q < e && pcol[q] == col) acc += aval[k] * pval[q];
+    const bool live = p < m;
+    uint32_t col = 0, a0 = 0, a1 = 0, t0 = 0, t1 = 0;
+    if (live) {
+        const uint32_t i = ap_row[p];
+        col = ap_col[p];
+        a0 = arow[i];
+        a1 = arow[i + 1];
+        t0 = t_off[col];
+        t1 = t_off[col + 1];
     }
-    apv[p] = acc;
-    if (!isfinite(acc)) flags[kBadProduct] = 1;
+    // Dependent steps of the two walks: a row's P entries are few, a lookup in
+    // A's row halves it.
+    const uint32_t by_a = 2 * (a1 - a0), by_t = (t1 - t0) * (33u - __clz(a1 - a0));
+    const bool walk_t = by_t < by_a;
+    const bool heavy = (walk_t ? by_t : by_a) > 512;
+    double acc = 0.0;
+    if (live && !heavy) {
+        if (walk_t) {
+            for (uint32_t t = t0; t < t1; ++t) {
+                const uint32_t j = t_row[t], k = lower_bound_u32(acol, a0, a1, j);
+                if (k < a1 && acol[k] == j) acc += aval[k] * pval[prow[j] + t_pos[t]];
+            }
+        } else {
+            for (uint32_t k = a0; k < a1; ++k) {
+                const uint32_t j = acol[k], e = prow[j + 1];
+                const uint32_t q = lower_bound_u32(pcol, prow[j], e, col);
+                if (q < e && pcol[q] == col) acc += aval[k] * pval[q];
+            }
+        }
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint64_t hm = __ballot(live && heavy); hm; hm &= hm - 1) {
+        const int src = __builtin_ctzll(hm);
+        const uint32_t c = __builtin_amdgcn_readlane(col, src), b0 = __builtin_amdgcn_readlane(a0, src),
+                       b1 = __builtin_amdgcn_readlane(a1, src), u0 = __builtin_amdgcn_readlane(t0, src),
+                       u1 = __builtin_amdgcn_readlane(t1, src);
+        const bool wt = __builtin_amdgcn_readlane(uint32_t(walk_t), src) != 0;
+        double s = 0.0;
+        for (uint32_t base = wt ? u0 : b0, end = wt ? u1 : b1; base < end; base += 64) {
+            const uint32_t x = base + lane;
+            bool hit = false;
+            double v = 0.0;
+            if (x < end) {
+                if (wt) {
+                    const uint32_t j = t_row[x], k = lower_bound_u32(acol, b0, b1, j);
+                    hit = k < b1 && acol[k] == j;
+                    if (hit) v = aval[k] * pval[prow[j] + t_pos[x]];
+                } else {
+                    const uint32_t j = acol[x], e = prow[j + 1];
+                    const uint32_t q = lower_bound_u32(pcol, prow[j], e, c);
+                    hit = q < e && pcol[q] == c;
+                    if (hit) v = aval[x] * pval[q];
+                }
+            }
+            s = add_lanes(s, v, __ballot(hit));
+        }
+        if (int(lane) == src) acc = s;
+    }
+    if (live) {
+        apv[p] = acc;
+        if (!isfinite(acc)) flags[kBadProduct] = 1;
+    }
 }
 
-__global__ __launch_bounds__(kBlock) void galerkin_c_entries_kernel(
-    uint64_t m, const uint32_t* __restrict__ c_row, const uint32_t* __restrict__ c_col,
-    const uint32_t* __restrict__ t_off, const uint32_t* __restrict__ t_row, const uint32_t* __restrict__ t_pos,
-    const uint32_t* __restrict__ prow, const double* __restrict__ pval, const uint32_t* __restrict__ ap_off,
-    const uint32_t* __restrict__ ap_col, const double* __restrict__ apv, double* __restrict__ cv,
-    const uint8_t* __restrict__ keep_mask, int* __restrict__ flags, const uint32_t* __restrict__ c_off,
-    uint32_t skip_len) {
-#pragma clang fp contract(off)
-    const uint64_t p = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (p >= m) return;
-    const uint32_t c = c_row[p], col = c_col[p];
-    if (c_off[c + 1] - c_off[c] <= skip_len) return;
-    double acc = 0.0;
-    for (uint32_t t = t_off[c]; t < t_off[c + 1]; ++t) {
-        const uint32_t i = t_row[t];
-        const uint32_t e = ap_off[i + 1];
-        const uint32_t q = lower_bound_u32(ap_col, ap_off[i], e, col);
-        if (q < e && ap_col[q] == col) acc += pval[prow[i] + t_pos[t]] * apv[q];
-    }
-    cv[p] = acc;
-    if (!isfinite(acc)) flags[kBadProduct] = 1;
-    if (keep_mask && ((fabs(acc) > 1e-30) != (keep_mask[p] != 0))) flags[kPatternChanged] = 1;
+// P^T (AP), three kinds of coarse row by their length and their count of fine
+// rows. Each kind takes the fine rows in order and adds their AP entries
+// (distinct columns) into the row's slots in LDS, so each slot receives its
+// terms in the reference's order.
+//   * up to kLightRow entries and kLightFine fine rows (nearly all): 16 lanes,
+//     sixteen rows a workgroup;
+//   * up to kTileCols entries and kMidFine fine rows: a wavefront;
+//   * the rest, rows that span a coarse level: a workgroup for every
+//     kTileCols columns, 32 fine rows at a time. Each wavefront writes the
+//     products of two of them into a 32 x kTileCols table and marks them in
+//     the columns' masks; then a thread a column adds the marked ones in order.
+//     One wavefront a row, fine row after fine row, took 7 ms on a level of 2K
+//     coarse rows.
+constexpr uint32_t kLightRow = 64, kLightFine = 24, kTileCols = 512, kMidFine = 64, kTileFine = 32;
+constexpr uint32_t kTileBytes = kTileFine * kTileCols * 8 + kTileCols * 16 + 2 * kTileFine * 16;
+
+__device__ __forceinline__ int c_row_kind(uint32_t len, uint32_t fine) {
+    return len <= kLightRow && fine <= kLightFine ? 0 : len <= kTileCols && fine <= kMidFine ? 1 : 2;
 }
 
-// The same P^T (AP) values, one 64-lane workgroup per coarse row of at most
-// kCRowCap entries: the row accumulates in LDS; the transpose plan's fine
-// rows are taken in order, and for each one the lanes add its AP entries
-// (distinct columns) into the row's slots, so each slot receives its terms in
-// the reference's order. Longer rows are left to galerkin_c_entries_kernel.
-constexpr uint32_t kCRowCap = 8192;  // 64 KiB of LDS at most
+// Counts (null lists) or lists the mid rows and the heavy rows' tiles; their
+// order does not matter.
+__global__ __launch_bounds__(kBlock) void c_row_kinds_kernel(uint32_t nc, const uint32_t* __restrict__ c_off,
+                                                             const uint32_t* __restrict__ t_off,
+                                                             uint32_t* __restrict__ cnt, uint32_t* __restrict__ mid,
+                                                             uint2* __restrict__ heavy) {
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= nc) return;
+    const uint32_t len = c_off[c + 1] - c_off[c];
+    const int kind = c_row_kind(len, t_off[c + 1] - t_off[c]);
+    if (kind == 1) {
+        const uint32_t at = atomicAdd(&cnt[0], 1u);
+        if (mid) mid[at] = c;
+    } else if (kind == 2) {
+        const uint32_t tiles = max(1u, (len + kTileCols - 1) / kTileCols), at = atomicAdd(&cnt[1], tiles);
+        if (heavy)
+            for (uint32_t t = 0; t < tiles; ++t) heavy[at + t] = make_uint2(c, t);
+    }
+}
 
-__global__ __launch_bounds__(64) void galerkin_c_rows_kernel(
-    const uint32_t* __restrict__ t_off, const uint32_t* __restrict__ t_row, const uint32_t* __restrict__ t_pos,
-    const uint32_t* __restrict__ prow, const double* __restrict__ pval, const uint32_t* __restrict__ ap_off,
-    const uint32_t* __restrict__ ap_col, const double* __restrict__ apv, const uint32_t* __restrict__ c_off,
-    const uint32_t* __restrict__ c_col, double* __restrict__ cv, const uint8_t* __restrict__ keep_mask,
-    int* __restrict__ flags) {
+struct CProduct {
+    const uint32_t *t_off, *t_row, *t_pos, *prow;
+    const double* pval;
+    const uint32_t *ap_off, *ap_col;
+    const double* apv;
+    const uint32_t *c_off, *c_col;
+    double* cv;
+    const uint8_t* keep_mask;  // null at setup
+    int* flags;
+};
+
+// Position of col in the ascending cols[0, n) (LDS), or n.
+__device__ __forceinline__ uint32_t find_col(const uint32_t* cols, uint32_t n, uint32_t col) {
+    uint32_t lo = 0, hi = n;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (cols[mid] < col) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo < n && cols[lo] == col ? lo : n;
+}
+
+__device__ __forceinline__ void store_c(const CProduct& g, uint32_t at, double v) {
+    g.cv[at] = v;
+    if (!isfinite(v)) g.flags[kBadProduct] = 1;
+    if (g.keep_mask && (fabs(v) > 1e-30) != (g.keep_mask[at] != 0)) g.flags[kPatternChanged] = 1;
+}
+
+// kLanes lanes a row of at most kLen entries; rows from `list`, or the light
+// ones of all rows.
+template <uint32_t kLanes, uint32_t kLen>
+__global__ __launch_bounds__(kBlock) void galerkin_c_rows_kernel(uint32_t count, const uint32_t* __restrict__ list,
+                                                                 CProduct g) {
 #pragma clang fp contract(off)
-    extern __shared__ double acc[];
-    const uint32_t c = blockIdx.x, lane = threadIdx.x;
-    const uint32_t rb = c_off[c], re = c_off[c + 1], len = re - rb;
-    if (len > kCRowCap) return;
-    for (uint32_t k = lane; k < len; k += 64) acc[k] = 0.0;
-    __syncthreads();
+    constexpr uint32_t kGroups = kBlock / kLanes;
+    __shared__ double accs[kGroups][kLen];
+    __shared__ uint32_t colss[kGroups][kLen];
+    const uint32_t grp = threadIdx.x / kLanes, lane = threadIdx.x % kLanes;
+    const uint32_t q = blockIdx.x * kGroups + grp;
+    if (q >= count) return;
+    const uint32_t c = list ? list[q] : q;
+    const uint32_t rb = g.c_off[c], len = g.c_off[c + 1] - rb, t0 = g.t_off[c], t1 = g.t_off[c + 1];
+    if (!list && c_row_kind(len, t1 - t0) != 0) return;
+    double* acc = accs[grp];
+    uint32_t* cols = colss[grp];
+    for (uint32_t k = lane; k < len; k += kLanes) {
+        acc[k] = 0.0;
+        cols[k] = g.c_col[rb + k];
+    }
+    wave_fence();
     bool missing = false;
-    for (uint32_t t = t_off[c]; t < t_off[c + 1]; ++t) {
-        const uint32_t i = t_row[t];
-        const double wgt = pval[prow[i] + t_pos[t]];
-        for (uint32_t p = ap_off[i] + lane; p < ap_off[i + 1]; p += 64) {
-            const uint32_t col = ap_col[p];
-            const uint32_t pos = lower_bound_u32(c_col, rb, re, col);
-            if (pos < re && c_col[pos] == col) acc[pos - rb] += wgt * apv[p];
+    // The next fine row's offsets are loaded while the current one is added.
+    uint32_t p0 = 0, p1 = 0;
+    double wgt = 0.0;
+    auto fetch = [&](uint32_t t) {
+        const uint32_t i = g.t_row[t];
+        p0 = g.ap_off[i];
+        p1 = g.ap_off[i + 1];
+        wgt = g.pval[g.prow[i] + g.t_pos[t]];
+    };
+    if (t0 < t1) fetch(t0);
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t b = p0, e = p1;
+        const double w = wgt;
+        if (t + 1 < t1) fetch(t + 1);
+        for (uint32_t p = b + lane; p < e; p += kLanes) {
+            const double v = g.apv[p];
+            const uint32_t pos = find_col(cols, len, g.ap_col[p]);
+            if (pos < len) acc[pos] += w * v;
             else missing = true;
         }
-        __syncthreads();
+        wave_fence();
     }
-    bool bad = missing, changed = false;
-    for (uint32_t k = lane; k < len; k += 64) {
-        const double v = acc[k];
-        cv[rb + k] = v;
-        bad = bad || !isfinite(v);
-        if (keep_mask) changed = changed || ((fabs(v) > 1e-30) != (keep_mask[rb + k] != 0));
-    }
-    if (bad) flags[kBadProduct] = 1;
-    if (changed) flags[kPatternChanged] = 1;
+    if (missing) g.flags[kBadProduct] = 1;
+    for (uint32_t k = lane; k < len; k += kLanes) store_c(g, rb + k, acc[k]);
 }
 
-// Longest row of a CSR pattern (integer maximum: any order).
-__global__ __launch_bounds__(kBlock) void max_row_len_kernel(uint32_t n, const uint32_t* __restrict__ off,
-                                                             uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) atomicMax(out, off[i + 1] - off[i]);
+__global__ __launch_bounds__(1024) void galerkin_c_tiles_kernel(const uint2* __restrict__ list, CProduct g) {
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    double* table = reinterpret_cast<double*>(tile_lds);  // [fine][column]
+    double* acc = table + kTileFine * kTileCols;
+    uint32_t* cols = reinterpret_cast<uint32_t*>(acc + kTileCols);
+    uint32_t* mask = cols + kTileCols;
+    uint4* meta = reinterpret_cast<uint4*>(mask + kTileCols);  // two sets: AP row begin, end, weight
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+    const uint32_t c = list[blockIdx.x].x, tile = list[blockIdx.x].y;
+    const uint32_t row0 = g.c_off[c], row1 = g.c_off[c + 1];
+    const uint32_t rb = row0 + tile * kTileCols, len = min(row1 - rb, kTileCols);
+    const uint32_t t0 = g.t_off[c], t1 = g.t_off[c + 1];
+    if (tid < len) {
+        cols[tid] = g.c_col[rb + tid];
+        acc[tid] = 0.0;
+        mask[tid] = 0u;
+    }
+    // Columns this tile answers for: up to the next tile's first.
+    const bool first = tile == 0, last = rb + len == row1;
+    const uint32_t lo = first || len == 0 ? 0u : g.c_col[rb], hi = last ? 0xffffffffu : g.c_col[rb + len];
+    auto fetch = [&](uint32_t t) {
+        uint4 m = make_uint4(0, 0, 0, 0);
+        if (t < t1) {
+            const uint32_t i = g.t_row[t];
+            const double w = g.pval[g.prow[i] + g.t_pos[t]];
+            m = make_uint4(g.ap_off[i], g.ap_off[i + 1], uint32_t(__double2loint(w)), uint32_t(__double2hiint(w)));
+        }
+        return m;
+    };
+    if (tid < kTileFine) meta[tid] = fetch(t0 + tid);
+    __syncthreads();
+    bool missing = false;
+    uint32_t set = 0;
+    for (uint32_t r = t0; r < t1; r += kTileFine, set ^= 1u) {
+        uint4 next = make_uint4(0, 0, 0, 0);
+        if (tid < kTileFine) next = fetch(r + kTileFine + tid);
+        for (uint32_t f = wave; f < kTileFine && r + f < t1; f += 16) {
+            const uint4 m = meta[set * kTileFine + f];
+            const double w = __hiloint2double(int(m.w), int(m.z));
+            uint32_t b = __builtin_amdgcn_readfirstlane(m.x);
+            const uint32_t e = __builtin_amdgcn_readfirstlane(m.y);
+            if (!first && e - b > 128) b = lower_bound_u32(g.ap_col, b, e, lo);
+            for (uint32_t p = b; p < e; p += 64) {
+                const bool in = p + lane < e;
+                const uint32_t col = in ? g.ap_col[p + lane] : 0xffffffffu;
+                if (in && col >= lo && (last || col < hi)) {
+                    const double v = g.apv[p + lane];
+                    const uint32_t pos = find_col(cols, len, col);
+                    if (pos < len) {
+                        table[f * kTileCols + pos] = w * v;
+                        atomicOr(&mask[pos], 1u << f);
+                    } else {
+                        missing = true;
+                    }
+                }
+                if (!last && __ballot(in && col >= hi)) break;
+            }
+        }
+        __syncthreads();
+        if (tid < len) {
+            uint32_t m = mask[tid];
+            if (m) {
+                double a = acc[tid];
+                for (; m; m &= m - 1) a += table[__builtin_ctz(m) * kTileCols + tid];
+                acc[tid] = a;
+                mask[tid] = 0u;
+            }
+        }
+        if (tid < kTileFine) meta[(set ^ 1u) * kTileFine + tid] = next;
+        __syncthreads();
+    }
+    if (missing) g.flags[kBadProduct] = 1;
+    if (tid < len) store_c(g, rb + tid, acc[tid]);
 }
 
 // Row index of every entry of a CSR pattern.
@@ -210,46 +401,91 @@ __global__ __launch_bounds__(kBlock) void row_index_kernel(uint32_t n, const uin
     for (uint32_t k = off[i]; k < off[i + 1]; ++k) row[k] = i;
 }
 
-// Normalised Gershgorin row sums sum_j |a_ij| / (sqrt(d_i) sqrt(d_j)),
-// d = 1 / inv; per-block maxima.
-__global__ __launch_bounds__(kBlock) void gershgorin_sd_kernel(uint32_t n, const double* __restrict__ inv,
-                                                               double* __restrict__ sd, int* __restrict__ flags) {
-#pragma clang fp contract(off)
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const double v = inv[i];
-    double s = 0.0;
-    if (!(v > 0.0) || !isfinite(v)) {
-        flags[kBadGershgorin] = 1;
-    } else {
-        const double d = 1.0 / v;
-        if (!(d > 0.0) || !isfinite(d)) flags[kBadGershgorin] = 1;
-        else s = sqrt(d);
-    }
-    sd[i] = s;
+// ---- Damping certificate and Lanczos bounds, all levels in one launch: a
+// level is a few microseconds of work, and a launch each (with a scalar sent
+// back to the host after every dot product) made 1800 launches of a refresh.
+
+// The level of workgroup wg: views[l].*first <= wg < views[l + 1].*first.
+__device__ __forceinline__ uint32_t level_of(const RefreshView* __restrict__ views, uint32_t wg) {
+    uint32_t l = 0;
+    while (wg >= views[l + 1].first_wg) ++l;
+    return l;
 }
 
-__global__ __launch_bounds__(kBlock) void gershgorin_rows_kernel(uint32_t n, const uint32_t* __restrict__ rowp,
-                                                                 const uint32_t* __restrict__ cols,
-                                                                 const double* __restrict__ vals,
-                                                                 const double* __restrict__ sd,
+// Normalised Gershgorin row sums sum_j |a_ij| / (sqrt(d_i) sqrt(d_j)),
+// d = 1 / inv; per-workgroup maxima. flags: kFlagCount per level.
+__global__ __launch_bounds__(kBlock) void gershgorin_sd_kernel(const RefreshView* __restrict__ views, uint32_t slot,
+                                                               double* __restrict__ sd, int* __restrict__ flags) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    if (i >= L.n) return;
+    const double v = L.rinv[slot][i];
+    double s = 0.0;
+    if (!(v > 0.0) || !isfinite(v)) {
+        flags[l * kFlagCount + kBadGershgorin] = 1;
+    } else {
+        const double d = 1.0 / v;
+        if (!(d > 0.0) || !isfinite(d)) flags[l * kFlagCount + kBadGershgorin] = 1;
+        else s = sqrt(d);
+    }
+    sd[L.row0 + i] = s;
+}
+
+// Rows above kGershgorinRow entries are summed by the wavefront, 64 terms
+// formed at a time and added in order.
+constexpr uint32_t kGershgorinRow = 48;
+__global__ __launch_bounds__(kBlock) void gershgorin_rows_kernel(const RefreshView* __restrict__ views, uint32_t slot,
+                                                                 const double* __restrict__ sd_all,
                                                                  double* __restrict__ block_max,
                                                                  int* __restrict__ flags) {
 #pragma clang fp contract(off)
     __shared__ double sm[kBlock];
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t l = level_of(views, blockIdx.x);
+    const RefreshView& L = views[l];
+    const double* sd = sd_all + L.row0;
+    const uint32_t* cols = L.acol;
+    const double* vals = L.aval[slot];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    const bool live = i < L.n;
+    const uint32_t b = live ? L.arow[i] : 0u, e = live ? L.arow[i + 1] : 0u;
+    const double si = live ? sd[i] : 0.0;
+    const bool longer = e - b > kGershgorinRow;
     double rs = 0.0;
-    if (i < n) {
-        bool bad = false;
-        for (uint32_t k = rowp[i]; k < rowp[i + 1]; ++k) {
-            const double sc = sd[i] * sd[cols[k]];
+    bool bad = false;
+    if (!longer)
+        for (uint32_t k = b; k < e; ++k) {
+            const double sc = si * sd[cols[k]];
             if (!(sc > 0.0) || !isfinite(sc)) bad = true;
             rs += fabs(vals[k]) / sc;
         }
-        if (bad || !isfinite(rs)) {
-            flags[kBadGershgorin] = 1;
-            rs = 0.0;
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint64_t m = __ballot(longer); m; m &= m - 1) {
+        const int src = __builtin_ctzll(m);
+        const uint32_t rb = __builtin_amdgcn_readlane(b, src), re = __builtin_amdgcn_readlane(e, src);
+        const double s0 = lane_value(si, src);
+        double s = 0.0;
+        bool wrong = false;
+        for (uint32_t k = rb; k < re; k += 64) {
+            double t = 0.0;
+            const bool in = k + lane < re;
+            if (in) {
+                const double sc = s0 * sd[cols[k + lane]];
+                if (!(sc > 0.0) || !isfinite(sc)) wrong = true;
+                t = fabs(vals[k + lane]) / sc;
+            }
+            s = add_lanes(s, t, __ballot(in));
         }
+        wrong = __ballot(wrong) != 0;
+        if (int(lane) == src) {
+            rs = s;
+            bad = wrong;
+        }
+    }
+    if (live && (bad || !isfinite(rs))) {
+        flags[l * kFlagCount + kBadGershgorin] = 1;
+        rs = 0.0;
     }
     sm[threadIdx.x] = rs;
     __syncthreads();
@@ -260,105 +496,231 @@ __global__ __launch_bounds__(kBlock) void gershgorin_rows_kernel(uint32_t n, con
     if (threadIdx.x == 0) block_max[blockIdx.x] = sm[0];
 }
 
-__global__ __launch_bounds__(1024) void max_reduce_kernel(uint32_t n, const double* __restrict__ v,
-                                                          double* __restrict__ out) {
+// out[l] = maximum over level l's workgroups.
+__global__ __launch_bounds__(1024) void max_reduce_kernel(const RefreshView* __restrict__ views,
+                                                          const double* __restrict__ v, double* __restrict__ out) {
     __shared__ double sm[1024];
     double m = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += 1024) m = fmax(m, v[i]);
+    for (uint32_t i = views[blockIdx.x].first_wg + threadIdx.x; i < views[blockIdx.x + 1].first_wg; i += 1024)
+        m = fmax(m, v[i]);
     sm[threadIdx.x] = m;
     __syncthreads();
     for (uint32_t s = 512; s > 0; s >>= 1) {
         if (threadIdx.x < s) sm[threadIdx.x] = fmax(sm[threadIdx.x], sm[threadIdx.x + s]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = sm[0];
+    if (threadIdx.x == 0) out[blockIdx.x] = sm[0];
 }
 
 // ---- Lanczos on D^-1/2 A D^-1/2, the host estimate's arithmetic. Vectors
 // live in the solve ordering next to the committed solve-ordered matrix
 // (rows keep the reference's entry order, so each row sum is the host's);
-// the dot products visit rows in the reference order through new_of_old.
+// the dot products visit rows in the reference order through new_of_old, in
+// 256-row tiles (tile_tree_sum) whose sums lanczos_total_kernel adds in the
+// host's blocks of 8192 rows. A level whose recurrence has ended (stop) skips
+// the launches that remain.
 
 __device__ __forceinline__ double lanczos_start(uint32_t i) {
     const uint32_t h = i * 2654435761u + 0x9e3779b9u;
     return double(h >> 8) * (1.0 / 16777216.0) - 0.5;
 }
 
-__global__ __launch_bounds__(kBlock) void lanczos_init_kernel(uint32_t n, const uint32_t* __restrict__ perm,
-                                                              const double* __restrict__ inv,
-                                                              double* __restrict__ sq, double* __restrict__ v,
-                                                              double* __restrict__ vp) {
+struct LanczosVectors {
+    double *sq, *v, *vp, *w, *u, *tile;
+};
+
+// The workgroup's tile sum of x (one value a thread).
+__device__ __forceinline__ void store_tile(double x, double* __restrict__ tile) {
+#pragma clang fp contract(off)
+    __shared__ double red[4];
+    x = wave_sum(x);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) tile[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+__global__ __launch_bounds__(kBlock) void lanczos_init_kernel(const RefreshView* __restrict__ views,
+                                                              LanczosState* __restrict__ st, LanczosVectors z) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    double x = 0.0;
+    if (i < L.n) {
+        const uint32_t p = L.perm[i];
+        const double v = lanczos_start(i);
+        z.v[L.row0 + p] = v;
+        z.sq[L.row0 + i] = sqrt(L.inv[i]);
+        z.vp[L.row0 + i] = 0.0;
+        x = v * v;
+    }
+    if (blockIdx.x == L.first_wg && threadIdx.x == 0) {
+        st[l].count = st[l].stop = 0;
+        st[l].beta[0] = 0.0;
+    }
+    store_tile(x, z.tile);
+}
+
+// The ordered total of a level's tile sums, then what the host's loop does
+// with it. kWhat 0: |v| at the start; 1: alpha; 2: beta and the stop rule.
+template <int kWhat>
+__global__ __launch_bounds__(1024) void lanczos_total_kernel(const RefreshView* __restrict__ views, uint32_t steps,
+                                                             LanczosState* __restrict__ states,
+                                                             const double* __restrict__ tile) {
+#pragma clang fp contract(off)
+    constexpr uint32_t kTiles = kLanczosRows / kBlock;
+    const RefreshView& L = views[blockIdx.x];
+    LanczosState& S = states[blockIdx.x];
+    if (S.stop) return;
+    const uint32_t nt = views[blockIdx.x + 1].first_wg - L.first_wg, nb = (nt + kTiles - 1) / kTiles;
+    const double* t = tile + L.first_wg;
+    __shared__ double sm[1024];
+    double total = 0.0;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 1024) {
+        const uint32_t b = b0 + threadIdx.x;
+        double acc = 0.0;
+        if (b < nb) {
+            double v[kTiles];
+#pragma unroll
+            for (uint32_t k = 0; k < kTiles; ++k) v[k] = b * kTiles + k < nt ? t[b * kTiles + k] : 0.0;
+#pragma unroll
+            for (uint32_t k = 0; k < kTiles; ++k)
+                if (b * kTiles + k < nt) acc += v[k];
+        }
+        sm[threadIdx.x] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) total = ordered_sum<false>(sm, 0u, min(nb - b0, 1024u), total);
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    if (kWhat == 0) {
+        S.norm = sqrt(total);
+    } else if (kWhat == 1) {
+        S.a = total;
+        S.alpha[S.count] = total;
+        S.bprev = S.beta[S.count];
+        ++S.count;
+    } else {
+        const double bn = sqrt(total);
+        if (!(bn > 1e-14 * fabs(S.a)) || S.count == min(steps, L.n)) {
+            S.stop = 1;
+        } else {
+            S.beta[S.count] = bn;
+            S.b = bn;
+        }
+    }
+}
+
+// v /= |v| and u = sq v.
+__global__ __launch_bounds__(kBlock) void lanczos_scale_kernel(const RefreshView* __restrict__ views,
+                                                               const LanczosState* __restrict__ st,
+                                                               LanczosVectors z) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    if (i >= L.n) return;
+    const double v = z.v[L.row0 + i] / st[l].norm;
+    z.v[L.row0 + i] = v;
+    z.u[L.row0 + i] = z.sq[L.row0 + i] * v;
+}
+
+// w = sq (A u): w_i = sq_i sum_q a_iq (sq_j v_j) in each row's entry order.
+struct EpiScaled {
+    static constexpr bool kPartial = false;
+    struct Pre {
+        double d;
+    };
+    const double* d;
+    double* y;
+    __device__ Pre load(uint32_t row) const { return {d[row]}; }
+    __device__ double apply(uint32_t row, double s, const Pre& p) const {
+        y[row] = p.d * s;
+        return 0.0;
+    }
+    __device__ double operator()(uint32_t row, double s) const { return apply(row, s, load(row)); }
+};
+__global__ __launch_bounds__(kBlock) void lanczos_spmv_kernel(const RefreshView* __restrict__ views,
+                                                              const LanczosState* __restrict__ st,
+                                                              LanczosVectors z) {
+    uint32_t l = 0;
+    while (blockIdx.x >= views[l + 1].first_block) ++l;
+    if (st[l].stop) return;
+    const RefreshView& L = views[l];
+    const uint32_t b = xcd_block(blockIdx.x - L.first_block, views[l + 1].first_block - L.first_block);
+    stream_rows<double>(L.blocks[b], L.blocks[b + 1], L.rowp, L.cols, L.vals, z.u + L.row0, InitZero<double>{},
+                        EpiScaled{z.sq + L.row0, z.w + L.row0});
+}
+
+// Tile sums of w v.
+__global__ __launch_bounds__(kBlock) void lanczos_dot_kernel(const RefreshView* __restrict__ views,
+                                                             const LanczosState* __restrict__ st, LanczosVectors z) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    if (st[l].stop) return;
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    double x = 0.0;
+    if (i < L.n) {
+        const uint32_t p = L.row0 + L.perm[i];
+        x = z.w[p] * z.v[p];
+    }
+    store_tile(x, z.tile);
+}
+
+// w = (w - a v) - b_prev vp, and the tile sums of w w.
+__global__ __launch_bounds__(kBlock) void lanczos_update_kernel(const RefreshView* __restrict__ views,
+                                                                const LanczosState* __restrict__ st,
+                                                                LanczosVectors z) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    if (st[l].stop) return;
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    double x = 0.0;
+    if (i < L.n) {
+        const uint32_t p = L.row0 + L.perm[i];
+        const double w = (z.w[p] - st[l].a * z.v[p]) - st[l].bprev * z.vp[p];
+        z.w[p] = w;
+        x = w * w;
+    }
+    store_tile(x, z.tile);
+}
+
+// vp = v, v = w / b, u = sq v.
+__global__ __launch_bounds__(kBlock) void lanczos_next_kernel(const RefreshView* __restrict__ views,
+                                                              const LanczosState* __restrict__ st, LanczosVectors z) {
+#pragma clang fp contract(off)
+    const uint32_t l = level_of(views, blockIdx.x);
+    if (st[l].stop) return;
+    const RefreshView& L = views[l];
+    const uint32_t i = (blockIdx.x - L.first_wg) * kBlock + threadIdx.x;
+    if (i >= L.n) return;
+    const uint32_t p = L.row0 + i;
+    z.vp[p] = z.v[p];
+    const double v = z.w[p] / st[l].b;
+    z.v[p] = v;
+    z.u[p] = z.sq[p] * v;
+}
+
+// Committed values in the solve ordering: CSR copies of either precision.
+__global__ __launch_bounds__(kBlock) void commit_values_kernel(uint64_t n, const uint32_t* __restrict__ idx,
+                                                               const double* __restrict__ src,
+                                                               double* __restrict__ v64, float* __restrict__ v32) {
+    const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const double v = src[idx[i]];
+    if (v64) v64[i] = v;
+    if (v32) v32[i] = float(v);
+}
+__global__ __launch_bounds__(kBlock) void commit_diagonal_kernel(uint32_t n, const uint32_t* __restrict__ perm,
+                                                                 const double* __restrict__ src,
+                                                                 double* __restrict__ d64, float* __restrict__ d32) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const uint32_t p = perm[i];
-    v[p] = lanczos_start(i);
-    sq[i] = sqrt(inv[i]);
-    vp[i] = 0.0;
-}
-
-// u = sq v and w = sq y: the two diagonal scalings around the level's FP64
-// SpMV y = A u, so w_i = sq_i sum_q a_iq (sq_j v_j) in each row's entry order.
-__global__ __launch_bounds__(kBlock) void diag_mul_kernel(uint32_t n, const double* __restrict__ d,
-                                                          const double* __restrict__ x, double* __restrict__ y) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) y[i] = d[i] * x[i];
-}
-
-// part[b] = the 8192-row block b's sum of a_i b_i (rows in the reference
-// order, entry perm[i] of the solve-ordered vectors): its 256-row tiles in
-// order, each tile the workgroup's butterfly tree (tile_tree_sum).
-__global__ __launch_bounds__(kBlock) void block_dot_kernel(uint32_t n, const uint32_t* __restrict__ perm,
-                                                           const double* __restrict__ a,
-                                                           const double* __restrict__ b,
-                                                           double* __restrict__ part) {
-#pragma clang fp contract(off)
-    __shared__ double red[4];
-    const uint32_t r0 = blockIdx.x * kLanczosRows;
-    double acc = 0.0;
-    for (uint32_t t0 = r0; t0 < r0 + kLanczosRows && t0 < n; t0 += kBlock) {
-        const uint32_t i = t0 + threadIdx.x;
-        double x = 0.0;
-        if (i < n) {
-            const uint32_t p = perm[i];
-            x = a[p] * b[p];
-        }
-        x = wave_sum(x);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
-        __syncthreads();
-        if (threadIdx.x == 0) acc += ((red[0] + red[1]) + red[2]) + red[3];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
-}
-
-__global__ void ordered_total_kernel(uint32_t nb, const double* __restrict__ part, double* __restrict__ out) {
-#pragma clang fp contract(off)
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double t = 0.0;
-    for (uint32_t b = 0; b < nb; ++b) t += part[b];
-    *out = t;
-}
-
-__global__ __launch_bounds__(kBlock) void scale_div_kernel(uint32_t n, double s, double* __restrict__ v) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) v[i] /= s;
-}
-
-__global__ __launch_bounds__(kBlock) void lanczos_update_kernel(uint32_t n, double a, double bprev,
-                                                                const double* __restrict__ v,
-                                                                const double* __restrict__ vp,
-                                                                double* __restrict__ w) {
-#pragma clang fp contract(off)
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) w[i] = (w[i] - a * v[i]) - bprev * vp[i];
-}
-
-__global__ __launch_bounds__(kBlock) void lanczos_next_kernel(uint32_t n, double bn, double* __restrict__ v,
-                                                              double* __restrict__ vp, const double* __restrict__ w) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    vp[i] = v[i];
-    v[i] = w[i] / bn;
+    if (d64) d64[p] = src[i];
+    if (d32) d32[p] = float(src[i]);
 }
 
 template <class T>
@@ -907,30 +1269,43 @@ __global__ __launch_bounds__(kBlock) void prune_fill_kernel(uint32_t nc, const u
 
 }  // namespace
 
-// P^T (AP) numeric of a transfer: rows up to kCRowCap in LDS (one workgroup
-// each), longer rows one thread per entry.
-static void launch_galerkin_c(const DeviceAmg::RefreshLevel& R, const uint8_t* keep_mask, int* flags,
-                              hipStream_t s) {
-    const uint32_t lds_rows = std::min(R.c_maxrow, kCRowCap);
-    galerkin_c_rows_kernel<<<R.nc, 64, size_t(std::max(1u, lds_rows)) * 8, s>>>(
-        R.t_off, R.t_row, R.t_pos, R.prow, R.pval, R.ap_off, R.ap_col, R.apv, R.c_off, R.c_col, R.cv, keep_mask,
-        flags);
-    if (R.c_maxrow > kCRowCap)
-        galerkin_c_entries_kernel<<<grid64(R.cnnz), kBlock, 0, s>>>(R.cnnz, R.c_row, R.c_col, R.t_off, R.t_row,
-                                                                    R.t_pos, R.prow, R.pval, R.ap_off, R.ap_col,
-                                                                    R.apv, R.cv, keep_mask, flags, R.c_off,
-                                                                    kCRowCap);
+// A P numeric of a transfer.
+static void launch_galerkin_ap(const DeviceAmg::RefreshLevel& R, const double* aval, int* flags, hipStream_t s) {
+    galerkin_ap_entries_kernel<<<grid64(R.apnnz), kBlock, 0, s>>>(R.apnnz, R.ap_row, R.ap_col, R.arow, R.acol, aval,
+                                                                  R.prow, R.pcol, R.pval, R.t_off, R.t_row, R.t_pos,
+                                                                  R.apv, flags);
 }
 
-static uint32_t max_row_len(const uint32_t* off, uint32_t n, hipStream_t s) {
-    uint32_t* d = dalloc<uint32_t>(1);
-    HIP_OK(hipMemsetAsync(d, 0, 4, s));
-    max_row_len_kernel<<<grid64(n), kBlock, 0, s>>>(n, off, d);
-    uint32_t h = 0;
-    HIP_OK(hipMemcpyAsync(&h, d, 4, hipMemcpyDeviceToHost, s));
+// P^T (AP) numeric of a transfer.
+static void launch_galerkin_c(const DeviceAmg::RefreshLevel& R, const uint8_t* keep_mask, int* flags,
+                              hipStream_t s) {
+    const CProduct g{R.t_off, R.t_row, R.t_pos, R.prow, R.pval, R.ap_off, R.ap_col, R.apv,
+                     R.c_off, R.c_col, R.cv,    keep_mask, flags};
+    galerkin_c_rows_kernel<16, kLightRow><<<(R.nc + 15) / 16, kBlock, 0, s>>>(R.nc, nullptr, g);
+    if (R.c_nmid) galerkin_c_rows_kernel<64, kTileCols><<<(R.c_nmid + 3) / 4, kBlock, 0, s>>>(R.c_nmid, R.c_mid, g);
+    if (R.c_nheavy) galerkin_c_tiles_kernel<<<R.c_nheavy, 1024, kTileBytes, s>>>(R.c_heavy, g);
+}
+
+// Lists of the mid and heavy coarse rows of a transfer.
+static void list_c_rows(DeviceAmg::RefreshLevel& R, hipStream_t s) {
+    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(galerkin_c_tiles_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kTileBytes)));
+    uint32_t* cnt = dalloc<uint32_t>(2);
+    uint32_t h[2] = {0, 0};
+    HIP_OK(hipMemsetAsync(cnt, 0, 8, s));
+    c_row_kinds_kernel<<<grid64(R.nc), kBlock, 0, s>>>(R.nc, R.c_off, R.t_off, cnt, nullptr, nullptr);
+    HIP_OK(hipMemcpyAsync(h, cnt, 8, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
-    dfree(d);
-    return h;
+    R.c_nmid = h[0];
+    R.c_nheavy = h[1];
+    R.c_mid = dalloc<uint32_t>(R.c_nmid);
+    R.c_heavy = dalloc<uint2>(R.c_nheavy);
+    if (h[0] || h[1]) {
+        HIP_OK(hipMemsetAsync(cnt, 0, 8, s));
+        c_row_kinds_kernel<<<grid64(R.nc), kBlock, 0, s>>>(R.nc, R.c_off, R.t_off, cnt, R.c_mid, R.c_heavy);
+        HIP_OK(hipStreamSynchronize(s));
+    }
+    dfree(cnt);
 }
 
 void DeviceAmg::release_refresh() {
@@ -938,15 +1313,21 @@ void DeviceAmg::release_refresh() {
     rf_.clear();
     dfree(rf_flags_);
     dfree(rf_work_);
+    dfree(rf_view_);
+    dfree(rf_lz_);
+    dfree(rf_ub_);
+    rf_view_host_.clear();
     rf_cur_ = 0;
 }
 
 void DeviceAmg::free_refresh_level(RefreshLevel& R) {
     for (uint32_t** p : {&R.arow, &R.acol, &R.src, &R.perm, &R.prow, &R.pcol, &R.ap_off, &R.ap_col, &R.ap_row,
-                         &R.c_off, &R.c_col, &R.c_row, &R.t_off, &R.t_row, &R.t_pos, &R.keep})
+                         &R.c_off, &R.c_col, &R.t_off, &R.t_row, &R.t_pos, &R.keep})
         dfree(*p);
     for (double** p : {&R.aval[0], &R.aval[1], &R.inv[0], &R.inv[1], &R.pval, &R.apv, &R.cv}) dfree(*p);
     dfree(R.keep_mask);
+    dfree(R.c_mid);
+    dfree(R.c_heavy);
 }
 
 bool DeviceAmg::build_refresh(const HostHierarchy& h, std::string& err, std::vector<RefreshLevel>* adopt) {
@@ -1006,11 +1387,7 @@ bool DeviceAmg::build_refresh(const HostHierarchy& h, std::string& err, std::vec
                 R.ap_row = dalloc<uint32_t>(R.apnnz);
                 row_index_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.ap_off, R.ap_row);
             }
-            if (!R.c_row) {
-                R.c_row = dalloc<uint32_t>(R.cnnz);
-                row_index_kernel<<<grid64(R.nc), kBlock, 0, stream_>>>(R.nc, R.c_off, R.c_row);
-            }
-            R.c_maxrow = max_row_len(R.c_off, R.nc, stream_);
+            if (!R.c_mid) list_c_rows(R, stream_);
         }
         // src: solve-ordered CSR position -> reference entry (rows relabelled
         // by the solve ordering, entry order kept).
@@ -1026,39 +1403,84 @@ bool DeviceAmg::build_refresh(const HostHierarchy& h, std::string& err, std::vec
         R.src = upload(src, stream_);
         R.perm = upload(perm, stream_);
     }
-    rf_flags_ = dalloc<int>(kFlagCount);
-    const uint32_t n0 = rf_[0].n;
-    const uint64_t nb = (n0 + kLanczosRows - 1) / kLanczosRows;
-    // Lanczos vectors sq, v, vp, w, u, y (n0 each), block partials,
-    // Gershgorin block maxima (n0 / 256) and 8 scalar slots.
-    rf_work_ = dalloc<double>(6 * uint64_t(n0) + nb + grid64(n0) + 8);
+    // What the batched kernels see of the levels.
+    rf_view_host_.assign(L + 1, RefreshView{});
+    uint32_t wg = 0, blk = 0, rows = 0;
+    for (size_t l = 0; l <= L; ++l) {
+        RefreshView& V = rf_view_host_[l];
+        V.first_wg = wg;
+        V.first_block = blk;
+        V.row0 = rows;
+        if (l == L) break;
+        const RefreshLevel& R = rf_[l];
+        const DevLevel& D = lv_[l];
+        V.n = R.n;
+        V.blocks = D.A.blocks;
+        V.rowp = D.A.rowp;
+        V.cols = D.A.cols;
+        V.vals = D.A.v64;
+        V.inv = D.inv64;
+        V.perm = R.perm;
+        V.arow = R.arow;
+        V.acol = R.acol;
+        for (int k = 0; k < 2; ++k) {
+            V.aval[k] = R.aval[k];
+            V.rinv[k] = R.inv[k];
+        }
+        wg += grid64(R.n);
+        blk += D.A.nblocks;
+        rows += R.n;
+    }
+    rf_view_ = upload(rf_view_host_, stream_);
+    rf_flags_ = dalloc<int>(kFlagCount * L);
+    rf_lz_ = dalloc<LanczosState>(L);
+    rf_ub_ = dalloc<double>(L);
+    // Five Lanczos vectors over all rows, tile sums (Gershgorin: row scales
+    // and workgroup maxima).
+    rf_work_ = dalloc<double>(5 * uint64_t(rows) + wg);
     rf_cur_ = 0;
+    const RefreshLevel& C = rf_.back();
+    rf_coarsest_ = HCsr{};
+    if (C.n <= 16) {
+        const HCsr& A = h.lv.back().A;
+        rf_coarsest_.n = rf_coarsest_.ncols = A.n;
+        rf_coarsest_.rowp = A.rowp;
+        rf_coarsest_.cols = A.cols;
+        rf_coarsest_.vals = A.vals;
+    }
     HIP_OK(hipStreamSynchronize(stream_));
     return true;
 }
 
-bool DeviceAmg::gershgorin_bound(uint32_t slot, bool& certified, double& mb) {
-    const size_t L = rf_.size();
-    const uint32_t n0 = rf_[0].n;
-    const uint64_t nb0 = (n0 + kLanczosRows - 1) / kLanczosRows;
+void DeviceAmg::launch_gershgorin(uint32_t slot) {
+    const RefreshView& end = rf_view_host_.back();
     double* sd = rf_work_;
-    double* bmax = rf_work_ + 6 * uint64_t(n0) + nb0;
-    double* scal = bmax + grid64(n0);
-    int hflags[kFlagCount];
+    double* bmax = rf_work_ + 5 * uint64_t(end.row0);
+    gershgorin_sd_kernel<<<end.first_wg, kBlock, 0, stream_>>>(rf_view_, slot, sd, rf_flags_);
+    gershgorin_rows_kernel<<<end.first_wg, kBlock, 0, stream_>>>(rf_view_, slot, sd, bmax, rf_flags_);
+    max_reduce_kernel<<<uint32_t(rf_.size()), 1024, 0, stream_>>>(rf_view_, bmax, rf_ub_);
+}
+
+// Fetches the levels' flags and Gershgorin bounds and, for a dense coarsest
+// level, its values of `slot`.
+void DeviceAmg::read_refresh(bool coarsest, uint32_t slot) {
+    rf_host_flags_.resize(kFlagCount * rf_.size());
+    rf_host_ub_.resize(rf_.size());
+    HIP_OK(hipMemcpyAsync(rf_host_flags_.data(), rf_flags_, rf_host_flags_.size() * sizeof(int),
+                          hipMemcpyDeviceToHost, stream_));
+    HIP_OK(hipMemcpyAsync(rf_host_ub_.data(), rf_ub_, rf_host_ub_.size() * 8, hipMemcpyDeviceToHost, stream_));
+    if (coarsest)
+        HIP_OK(hipMemcpyAsync(rf_coarsest_.vals.data(), rf_.back().aval[slot], rf_coarsest_.vals.size() * 8,
+                              hipMemcpyDeviceToHost, stream_));
+    HIP_OK(hipStreamSynchronize(stream_));
+}
+
+bool DeviceAmg::gershgorin_bound(bool& certified, double& mb) const {
     mb = 0.0;
     certified = true;
-    for (size_t l = 0; l < L && certified; ++l) {
-        RefreshLevel& R = rf_[l];
-        HIP_OK(hipMemsetAsync(rf_flags_ + kBadGershgorin, 0, sizeof(int), stream_));
-        gershgorin_sd_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.inv[slot], sd, rf_flags_);
-        gershgorin_rows_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.arow, R.acol, R.aval[slot], sd, bmax,
-                                                                    rf_flags_);
-        max_reduce_kernel<<<1, 1024, 0, stream_>>>(grid64(R.n), bmax, scal);
-        double ub = 0.0;
-        HIP_OK(hipMemcpyAsync(&ub, scal, 8, hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipMemcpyAsync(hflags, rf_flags_, sizeof(hflags), hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipStreamSynchronize(stream_));
-        if (hflags[kBadGershgorin] || !std::isfinite(ub) || !(ub > 0.0)) certified = false;
+    for (size_t l = 0; l < rf_.size() && certified; ++l) {
+        const double ub = rf_host_ub_[l];
+        if (rf_host_flags_[l * kFlagCount + kBadGershgorin] || !std::isfinite(ub) || !(ub > 0.0)) certified = false;
         else mb = std::max(mb, ub);
     }
     return true;
@@ -1067,52 +1489,31 @@ bool DeviceAmg::gershgorin_bound(uint32_t slot, bool& certified, double& mb) {
 std::vector<double> DeviceAmg::lanczos_bounds(const AmgConfig& cfg) {
     // Lanczos estimate of lambda_max(D^-1 A) per level on the committed
     // solve-ordered FP64 matrices (the host estimate's arithmetic).
-    const size_t L = lv_.size();
-    const uint32_t n0 = lv_[0].n;
-    const uint64_t nb0 = (n0 + kLanczosRows - 1) / kLanczosRows;
-    double* sq = rf_work_;
-    double* v = sq + n0;
-    double* vp = v + n0;
-    double* w = vp + n0;
-    double* u = w + n0;
-    double* y = u + n0;
-    double* part = y + n0;
-    double* scal = part + nb0 + grid64(n0);
-    std::vector<double> lambda;
-    for (size_t l = 0; l < L; ++l) {
-        const DevLevel& D = lv_[l];
-        const uint32_t n = D.n;
-        const uint32_t* perm = rf_[l].perm;
-        const uint32_t nb = uint32_t((n + kLanczosRows - 1) / kLanczosRows);
-        auto total = [&](const double* a, const double* b) {
-            block_dot_kernel<<<nb, kBlock, 0, stream_>>>(n, perm, a, b, part);
-            ordered_total_kernel<<<1, 1, 0, stream_>>>(nb, part, scal);
-            double t = 0.0;
-            HIP_OK(hipMemcpyAsync(&t, scal, 8, hipMemcpyDeviceToHost, stream_));
-            HIP_OK(hipStreamSynchronize(stream_));
-            return t;
-        };
-        lanczos_init_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, perm, D.inv64, sq, v, vp);
-        const double nv = std::sqrt(total(v, v));
-        scale_div_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, nv, v);
-        std::vector<double> alpha, beta(1, 0.0);
-        const uint32_t steps = std::min<uint32_t>(cfg.lambda_iterations, n);
-        for (uint32_t k = 0; k < steps; ++k) {
-            diag_mul_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, sq, v, u);
-            spmv64_level(uint32_t(l), u, y);
-            diag_mul_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, sq, y, w);
-            const double a = total(w, v);
-            alpha.push_back(a);
-            const double bprev = beta.back();
-            lanczos_update_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, a, bprev, v, vp, w);
-            const double bn = std::sqrt(total(w, w));
-            if (!(bn > 1e-14 * std::abs(a)) || k + 1 == steps) break;
-            beta.push_back(bn);
-            lanczos_next_kernel<<<grid64(n), kBlock, 0, stream_>>>(n, bn, v, vp, w);
-        }
-        beta.resize(alpha.size());
-        lambda.push_back(tridiag_max_eigenvalue(alpha, beta));
+    const uint32_t steps = cfg.lambda_iterations;
+    if (steps > kLanczosMax) throw std::runtime_error("too many Lanczos steps");
+    const RefreshView& end = rf_view_host_.back();
+    const uint32_t L = uint32_t(lv_.size()), g = end.first_wg;
+    const uint64_t n = end.row0;
+    double* q = rf_work_;
+    const LanczosVectors z{q, q + n, q + 2 * n, q + 3 * n, q + 4 * n, q + 5 * n};
+    lanczos_init_kernel<<<g, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
+    lanczos_total_kernel<0><<<L, 1024, 0, stream_>>>(rf_view_, steps, rf_lz_, z.tile);
+    lanczos_scale_kernel<<<g, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
+    for (uint32_t k = 0; k < steps; ++k) {
+        lanczos_spmv_kernel<<<end.first_block, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
+        lanczos_dot_kernel<<<g, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
+        lanczos_total_kernel<1><<<L, 1024, 0, stream_>>>(rf_view_, steps, rf_lz_, z.tile);
+        lanczos_update_kernel<<<g, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
+        lanczos_total_kernel<2><<<L, 1024, 0, stream_>>>(rf_view_, steps, rf_lz_, z.tile);
+        if (k + 1 < steps) lanczos_next_kernel<<<g, kBlock, 0, stream_>>>(rf_view_, rf_lz_, z);
     }
+    std::vector<LanczosState> st(L);
+    HIP_OK(hipMemcpyAsync(st.data(), rf_lz_, L * sizeof(LanczosState), hipMemcpyDeviceToHost, stream_));
+    HIP_OK(hipStreamSynchronize(stream_));
+    std::vector<double> lambda;
+    for (const LanczosState& S : st)
+        lambda.push_back(tridiag_max_eigenvalue(std::vector<double>(S.alpha, S.alpha + S.count),
+                                                std::vector<double>(S.beta, S.beta + S.count)));
     return lambda;
 }
 
@@ -1120,7 +1521,10 @@ bool DeviceAmg::finish_setup(const AmgConfig& cfg, double& omega, std::vector<do
     bool certified = false;
     double mb = 0.0;
     const auto t0 = std::chrono::steady_clock::now();
-    gershgorin_bound(rf_cur_, certified, mb);
+    HIP_OK(hipMemsetAsync(rf_flags_, 0, sizeof(int) * kFlagCount * rf_.size(), stream_));
+    launch_gershgorin(rf_cur_);
+    read_refresh(false, rf_cur_);
+    gershgorin_bound(certified, mb);
     lambda.clear();
     if (cfg.wants_lambda()) lambda = lanczos_bounds(cfg);
     if (std::getenv("CFDXHIP_SETUP_TRACE"))
@@ -1153,44 +1557,44 @@ bool DeviceAmg::refresh_device(const double* d_vals, const AmgConfig& cfg, doubl
     }
     const uint32_t stg = rf_cur_ ^ 1u;
     const size_t L = rf_.size();
-    int hflags[kFlagCount];
-    auto check = [&](size_t level) -> bool {
-        HIP_OK(hipMemcpyAsync(hflags, rf_flags_, sizeof(hflags), hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipStreamSynchronize(stream_));
-        if (hflags[kBadInput]) err = "non-finite matrix value";
-        else if (hflags[kBadDiagonal]) err = "invalid or zero diagonal at level " + std::to_string(level);
-        else if (hflags[kBadProduct]) err = "non-finite Galerkin product at level " + std::to_string(level);
-        else if (hflags[kPatternChanged]) {
-            err = "Galerkin pattern changed at level " + std::to_string(level + 1);
-            pattern_changed = true;
-        } else {
-            return true;
-        }
-        return false;
-    };
-    HIP_OK(hipMemsetAsync(rf_flags_, 0, sizeof(int) * kFlagCount, stream_));
+    // Every level is recomputed into the staged slot; the error flags, the
+    // Gershgorin bounds and the coarsest values come back together. A level
+    // that follows a failed one computes on what it finds (patterns are
+    // fixed), and the first failure in the order of the checks is reported.
+    HIP_OK(hipMemsetAsync(rf_flags_, 0, sizeof(int) * kFlagCount * L, stream_));
     // Level 0 values come in the caller's (reference) order.
     HIP_OK(hipMemcpyAsync(rf_[0].aval[stg], d_vals, rf_[0].nnz * 8, hipMemcpyDeviceToDevice, stream_));
     finite_check_kernel<<<grid64(rf_[0].nnz), kBlock, 0, stream_>>>(rf_[0].nnz, rf_[0].aval[stg], rf_flags_);
-    if (!check(0)) return false;
     for (size_t l = 0; l < L; ++l) {
         RefreshLevel& R = rf_[l];
-        inv_diag_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.arow, R.acol, R.aval[stg], R.inv[stg],
-                                                             rf_flags_);
-        if (!check(l)) return false;
+        int* flags = rf_flags_ + l * kFlagCount;
+        inv_diag_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.arow, R.acol, R.aval[stg], R.inv[stg], flags);
         if (l + 1 == L) break;
-        galerkin_ap_entries_kernel<<<grid64(R.apnnz), kBlock, 0, stream_>>>(
-            R.apnnz, R.ap_row, R.ap_col, R.arow, R.acol, R.aval[stg], R.prow, R.pcol, R.pval, R.apv, rf_flags_);
-        if (!check(l)) return false;
-        launch_galerkin_c(R, R.keep_mask, rf_flags_, stream_);
-        if (!check(l)) return false;
+        launch_galerkin_ap(R, R.aval[stg], flags, stream_);
+        launch_galerkin_c(R, R.keep_mask, flags, stream_);
         RefreshLevel& N = rf_[l + 1];
         gather_idx_kernel<double><<<grid64(N.nnz), kBlock, 0, stream_>>>(N.nnz, R.keep, R.cv, N.aval[stg]);
+    }
+    launch_gershgorin(stg);
+    const bool dense = rf_.back().n <= 16;
+    read_refresh(dense, stg);
+    for (size_t l = 0; l < L; ++l) {
+        const int* f = rf_host_flags_.data() + l * kFlagCount;
+        if (f[kBadInput]) err = "non-finite matrix value";
+        else if (f[kBadDiagonal]) err = "invalid or zero diagonal at level " + std::to_string(l);
+        else if (f[kBadProduct]) err = "non-finite Galerkin product at level " + std::to_string(l);
+        else if (f[kPatternChanged]) {
+            err = "Galerkin pattern changed at level " + std::to_string(l + 1);
+            pattern_changed = true;
+        } else {
+            continue;
+        }
+        return false;
     }
     // Damping certificate on the staged values.
     bool certified = false;
     double mb = 0.0;
-    gershgorin_bound(stg, certified, mb);
+    gershgorin_bound(certified, mb);
     double wv = 0.0;
     if (certified) {
         wv = std::min(cfg.omega, 1.8 / mb);
@@ -1206,34 +1610,15 @@ bool DeviceAmg::refresh_device(const double* d_vals, const AmgConfig& cfg, doubl
     // Coarsest dense LU from the refreshed coarsest values (at most 16 rows).
     CoarseLU lu;
     bool lu_ok = false;
-    const RefreshLevel& C = rf_.back();
-    const bool dense = C.n <= 16;
-    if (dense) {
-        HCsr A;
-        A.n = A.ncols = C.n;
-        A.rowp.resize(size_t(C.n) + 1);
-        A.cols.resize(C.nnz);
-        A.vals.resize(C.nnz);
-        HIP_OK(hipMemcpyAsync(A.rowp.data(), C.arow, A.rowp.size() * 4, hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipMemcpyAsync(A.cols.data(), C.acol, C.nnz * 4, hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipMemcpyAsync(A.vals.data(), C.aval[stg], C.nnz * 8, hipMemcpyDeviceToHost, stream_));
-        HIP_OK(hipStreamSynchronize(stream_));
-        lu_ok = factor_coarsest(A, lu, cns_);
-    }
+    if (dense) lu_ok = factor_coarsest(rf_coarsest_, lu, cns_);
     // Commit: values into the solve-ordered CSR / SELL copies, inverse
     // diagonals, damping, Chebyshev coefficients, coarsest factors.
     for (size_t l = 0; l < L; ++l) {
         RefreshLevel& R = rf_[l];
         DevLevel& D = lv_[l];
-        if (has64_) {
-            gather_idx_kernel<double><<<grid64(R.nnz), kBlock, 0, stream_>>>(R.nnz, R.src, R.aval[stg], D.A.v64);
-            scatter_d2d(R.n, R.perm, R.inv[stg], D.inv64, stream_);
-        }
-        if (has32_) {
-            gather_idx_kernel<float><<<grid64(R.nnz), kBlock, 0, stream_>>>(R.nnz, R.src, R.aval[stg], D.A.v32);
-            scatter_d2f(R.n, R.perm, R.inv[stg], D.inv32, stream_);
-        }
-        sell_values(D.A, stream_);
+        commit_values_kernel<<<grid64(R.nnz), kBlock, 0, stream_>>>(R.nnz, R.src, R.aval[stg], D.A.v64, D.A.v32);
+        commit_diagonal_kernel<<<grid64(R.n), kBlock, 0, stream_>>>(R.n, R.perm, R.inv[stg], D.inv64, D.inv32);
+        sell_values(D.A, stream_, false);
         if (D.A.hvals) {
             const uint32_t rows = D.A.nslices * kSellRows;
             sell_half_values_kernel<<<grid_for(rows), kBlock, 0, stream_>>>(D.n, rows, D.A.soff, D.A.s32, D.inv32,
@@ -1253,14 +1638,16 @@ bool DeviceAmg::refresh_device(const double* d_vals, const AmgConfig& cfg, doubl
         set_chebyshev_lambda(lambda);
     }
     if (dense) {
-        dfree(lu_.piv);
-        dfree(lu_.factor);
-        dfree(lu_.upper);
         lu_.ok = lu_ok;
         if (lu_ok) {
-            lu_.piv = upload(lu.piv, stream_);
-            lu_.factor = upload(lu.factor, stream_);
-            lu_.upper = upload(lu.upper, stream_);
+            if (!lu_.piv) {
+                lu_.piv = dalloc<uint32_t>(lu.piv.size());
+                lu_.factor = dalloc<double>(lu.factor.size());
+                lu_.upper = dalloc<double>(lu.upper.size());
+            }
+            HIP_OK(hipMemcpyAsync(lu_.piv, lu.piv.data(), lu.piv.size() * 4, hipMemcpyHostToDevice, stream_));
+            HIP_OK(hipMemcpyAsync(lu_.factor, lu.factor.data(), lu.factor.size() * 8, hipMemcpyHostToDevice, stream_));
+            HIP_OK(hipMemcpyAsync(lu_.upper, lu.upper.data(), lu.upper.size() * 8, hipMemcpyHostToDevice, stream_));
         }
     }
     HIP_OK(hipStreamSynchronize(stream_));
@@ -1507,13 +1894,9 @@ bool DeviceAmg::build_sa_device(const uint32_t* d_rowp, const uint32_t* d_cols, 
         R.apv = dalloc<double>(apnnz);
         R.cv = dalloc<double>(cnnz);
         R.ap_row = dalloc<uint32_t>(apnnz);
-        R.c_row = dalloc<uint32_t>(cnnz);
         row_index_kernel<<<g, kBlock, 0, stream>>>(nl, R.ap_off, R.ap_row);
-        row_index_kernel<<<gc, kBlock, 0, stream>>>(nc, R.c_off, R.c_row);
-        galerkin_ap_entries_kernel<<<grid64(apnnz), kBlock, 0, stream>>>(apnnz, R.ap_row, R.ap_col, R.arow, R.acol,
-                                                                         R.aval[0], R.prow, R.pcol, R.pval, R.apv,
-                                                                         flags);
-        R.c_maxrow = max_row_len(R.c_off, nc, stream);
+        launch_galerkin_ap(R, R.aval[0], flags, stream);
+        list_c_rows(R, stream);
         launch_galerkin_c(R, nullptr, flags, stream);
         if (flagged(kBadProduct))
             return fail("invalid Galerkin coarse matrix from level " + std::to_string(levels.size() - 1));
@@ -1552,14 +1935,16 @@ bool DeviceAmg::build_sa_device(const uint32_t* d_rowp, const uint32_t* d_cols, 
             }
             free_refresh_level(N);
             RefreshLevel& T = levels.back();
-            for (uint32_t** p : {&T.prow, &T.pcol, &T.ap_off, &T.ap_col, &T.ap_row, &T.c_off, &T.c_col, &T.c_row,
+            for (uint32_t** p : {&T.prow, &T.pcol, &T.ap_off, &T.ap_col, &T.ap_row, &T.c_off, &T.c_col,
                                  &T.t_off, &T.t_row, &T.t_pos, &T.keep})
                 dfree(*p);
             for (double** p : {&T.pval, &T.apv, &T.cv}) dfree(*p);
             dfree(T.keep_mask);
             T.nc = 0;
             T.pnnz = T.apnnz = T.cnnz = 0;
-            T.c_maxrow = 0;
+            dfree(T.c_mid);
+            dfree(T.c_heavy);
+            T.c_nmid = T.c_nheavy = 0;
             host.lv.pop_back();
             break;
         }

@@ -181,18 +181,15 @@ __device__ __forceinline__ T wave_row_sums(const T* p, uint32_t b, uint32_t e, b
     return out;
 }
 
+// The rows of one row block [lo, hi) (row, first entry), summed by the
+// workgroup and handed to the epilogue; returns this thread's partial.
 template <class T, class Init, class Epi, int kStreamNnz = StreamNnz<T>::value>
-__global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint2* __restrict__ blocks, uint32_t nb,
-                                                             const uint32_t* __restrict__ rowp,
-                                                             const uint32_t* __restrict__ cols,
-                                                             const T* __restrict__ vals, const T* __restrict__ x,
-                                                             Init init, Epi epi) {
+__device__ __forceinline__ double stream_rows(uint2 lo, uint2 hi, const uint32_t* __restrict__ rowp,
+                                              const uint32_t* __restrict__ cols, const T* __restrict__ vals,
+                                              const T* __restrict__ x, const Init& init, const Epi& epi) {
 #pragma clang fp contract(off)
     constexpr bool kOrdered = OrderedSum<T>::value;
     __shared__ T prod[kStreamNnz];
-    __shared__ double red[4];
-    const uint32_t b = xcd_block(blockIdx.x, nb);
-    const uint2 lo = blocks[b], hi = blocks[b + 1];
     const uint32_t r0 = lo.x, r1 = hi.x, k0 = lo.y, k1 = hi.y;
     double part = 0.0;
     if (k1 - k0 <= uint32_t(kStreamNnz)) {
@@ -356,7 +353,19 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint2* __rest
         __syncthreads();
         if (threadIdx.x == 0) part = epi(r0, init(r0) + (((tred[0] + tred[1]) + tred[2]) + tred[3]));
     }
+    return part;
+}
+
+template <class T, class Init, class Epi>
+__global__ __launch_bounds__(kBlock) void spmv_stream_kernel(const uint2* __restrict__ blocks, uint32_t nb,
+                                                             const uint32_t* __restrict__ rowp,
+                                                             const uint32_t* __restrict__ cols,
+                                                             const T* __restrict__ vals, const T* __restrict__ x,
+                                                             Init init, Epi epi) {
+    const uint32_t b = xcd_block(blockIdx.x, nb);
+    const double part = stream_rows<T>(blocks[b], blocks[b + 1], rowp, cols, vals, x, init, epi);
     if (Epi::kPartial) {
+        __shared__ double red[4];
         const double bs = block_sum(part, red);
         if (threadIdx.x == 0) epi.store_partial(blockIdx.x, bs);
     }
