@@ -2079,6 +2079,89 @@ void FvMesh::rhie_chow_flux_device(const uint8_t* h_vbt, const double* h_vbv, co
 
 namespace {
 
+// Per-cell accumulation of a chunk of faces. Face lists come grouped by owner
+// as a rule, so a chunk's owners, and its neighbours one cell or one row of
+// cells away, lie in a window of cells that fits LDS: those contributions are
+// added there and reach memory as one atomic a cell and component, 64
+// consecutive cells an instruction. Contributions outside the window, and the
+// chunks whose owners spread over more than the window (an ungrouped list), go
+// to memory one by one. On a 160^3 lattice (12.4M faces; every contribution a
+// global atomic took 1369 us for the gradient, 489 us for the divergence) the
+// atomics to memory fall from 18 to about 7 a cell.
+constexpr uint32_t kFacePer = 8;                       // faces a thread
+constexpr uint32_t kFaceChunk = kFacePer * kBlock;
+template <int C>
+struct FaceWindow {
+    static constexpr uint32_t kCells = C == 3 ? 1280 : 4096;
+};
+
+// term(f, o, nb, add): calls add(cell, c, value) for the face's contributions.
+template <int C, class Term>
+__device__ __forceinline__ void accumulate_faces(uint64_t nf, uint64_t nc, const uint32_t* __restrict__ owner,
+                                                 const int64_t* __restrict__ neighbour, double* const (&out)[C],
+                                                 int* bad, Term term) {
+    constexpr uint32_t kW = FaceWindow<C>::kCells;
+    __shared__ double win[C][kW];
+    __shared__ uint32_t range[2];
+    const uint64_t f0 = uint64_t(blockIdx.x) * kFaceChunk;
+    uint32_t ow[kFacePer];
+    uint32_t lo = 0xffffffffu, hi = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kFacePer; ++k) {
+        const uint64_t f = f0 + k * kBlock + threadIdx.x;
+        ow[k] = f < nf ? owner[f] : 0xffffffffu;
+        if (ow[k] < nc) {
+            lo = min(lo, ow[k]);
+            hi = max(hi, ow[k]);
+        }
+    }
+    if (threadIdx.x == 0) {
+        range[0] = 0xffffffffu;
+        range[1] = 0;
+    }
+    for (uint32_t w = threadIdx.x; w < kW; w += kBlock)
+#pragma unroll
+        for (int c = 0; c < C; ++c) win[c][w] = 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, uint32_t(__shfl_xor(int(lo), off, 64)));
+        hi = max(hi, uint32_t(__shfl_xor(int(hi), off, 64)));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin(&range[0], lo);
+        atomicMax(&range[1], hi);
+    }
+    __syncthreads();
+    const uint32_t base = range[0];
+    // Nothing valid: base stays above every cell and no contribution arises.
+    const uint32_t width = range[1] >= base && range[1] - base < kW ? kW : 0;
+    auto add = [&](uint64_t cell, int c, double v) {
+        const uint64_t w = cell - base;
+        if (w < width) unsafeAtomicAdd(&win[c][w], v);
+        else unsafeAtomicAdd(out[c] + cell, v);
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < kFacePer; ++k) {
+        const uint64_t f = f0 + k * kBlock + threadIdx.x;
+        if (f >= nf) break;
+        const uint64_t o = ow[k];
+        const int64_t nb = neighbour[f];
+        if (o >= nc || nb >= int64_t(nc)) {
+            atomicOr(bad, 1);
+            continue;
+        }
+        term(f, o, nb, add);
+    }
+    __syncthreads();
+    for (uint32_t w = threadIdx.x; w < width; w += kBlock)
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const double v = win[c][w];
+            if (v != 0.0) unsafeAtomicAdd(out[c] + base + w, v);
+        }
+}
+
 __global__ __launch_bounds__(kBlock) void face_gradient_kernel(uint64_t nf, uint64_t nc, const double* __restrict__ phi,
                                                                const double* __restrict__ sx,
                                                                const double* __restrict__ sy,
@@ -2087,24 +2170,16 @@ __global__ __launch_bounds__(kBlock) void face_gradient_kernel(uint64_t nf, uint
                                                                const int64_t* __restrict__ neighbour, double* gx,
                                                                double* gy, double* gz, int* bad) {
 #pragma clang fp contract(off)
-    for (uint64_t f = blockIdx.x * uint64_t(kBlock) + threadIdx.x; f < nf; f += uint64_t(gridDim.x) * kBlock) {
-        const uint64_t o = owner[f];
-        const int64_t nb = neighbour[f];
-        if (o >= nc || nb >= int64_t(nc)) {
-            atomicOr(bad, 1);
-            continue;
-        }
+    double* const out[3] = {gx, gy, gz};
+    accumulate_faces<3>(nf, nc, owner, neighbour, out, bad, [&](uint64_t f, uint64_t o, int64_t nb, auto add) {
         const double vf = nb >= 0 ? 0.5 * (phi[o] + phi[nb]) : phi[o];
-        const double cx = vf * sx[f], cy = vf * sy[f], cz = vf * sz[f];
-        atomicAdd(gx + o, cx);
-        atomicAdd(gy + o, cy);
-        atomicAdd(gz + o, cz);
-        if (nb >= 0) {
-            atomicAdd(gx + nb, -cx);
-            atomicAdd(gy + nb, -cy);
-            atomicAdd(gz + nb, -cz);
+        const double t[3] = {vf * sx[f], vf * sy[f], vf * sz[f]};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            add(o, c, t[c]);
+            if (nb >= 0) add(uint64_t(nb), c, -t[c]);
         }
-    }
+    });
 }
 
 __global__ __launch_bounds__(kBlock) void inverse_volume_scale_kernel(uint64_t nc, const double* __restrict__ vol,
@@ -2123,26 +2198,31 @@ __global__ __launch_bounds__(kBlock) void face_divergence_kernel(uint64_t nf, ui
                                                                  const uint32_t* __restrict__ owner,
                                                                  const int64_t* __restrict__ neighbour, double* div,
                                                                  int* bad) {
-    for (uint64_t f = blockIdx.x * uint64_t(kBlock) + threadIdx.x; f < nf; f += uint64_t(gridDim.x) * kBlock) {
-        const uint64_t o = owner[f];
-        const int64_t nb = neighbour[f];
-        if (o >= nc || nb >= int64_t(nc)) {
-            atomicOr(bad, 1);
-            continue;
-        }
-        atomicAdd(div + o, phi_face[f]);
-        if (nb >= 0) atomicAdd(div + nb, -phi_face[f]);
+    double* const out[1] = {div};
+    accumulate_faces<1>(nf, nc, owner, neighbour, out, bad, [&](uint64_t f, uint64_t o, int64_t nb, auto add) {
+        const double v = phi_face[f];
+        add(o, 0, v);
+        if (nb >= 0) add(uint64_t(nb), 0, -v);
+    });
+}
+
+// Clears the outputs (null: absent) and the index flag.
+__global__ __launch_bounds__(kBlock) void face_clear_kernel(uint64_t n, double* a, double* b, double* c, int* bad) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
+    for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * kBlock) {
+        a[i] = 0.0;
+        if (b) b[i] = 0.0;
+        if (c) c[i] = 0.0;
     }
 }
 
-__global__ __launch_bounds__(kBlock) void zero_f64_kernel(uint64_t n, double* a) {
-    for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * kBlock)
-        a[i] = 0.0;
-}
-
-__global__ void zero_i32_kernel(int* a) { *a = 0; }
-
 uint32_t face_grid(uint64_t n) { return uint32_t(std::min<uint64_t>((n + kBlock - 1) / kBlock, 1u << 20)) + (n == 0); }
+
+uint32_t chunks(uint64_t n_faces) {
+    const uint64_t c = (n_faces + kFaceChunk - 1) / kFaceChunk;
+    if (c > 0x7fffffffu) throw std::invalid_argument("face list too long");
+    return uint32_t(c);
+}
 
 // Stream-ordered flag for one call; false when any face index was out of
 // range.
@@ -2150,7 +2230,6 @@ template <class F>
 bool with_index_flag(hipStream_t s, F launch) {
     int* bad = nullptr;
     HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&bad), sizeof(int), s));
-    zero_i32_kernel<<<1, 1, 0, s>>>(bad);
     launch(bad);
     HIP_OK(hipGetLastError());
     int h = 0;
@@ -2166,9 +2245,9 @@ bool face_gradient_gauss(const double* phi, const double* sx, const double* sy, 
                          const uint32_t* owner, const int64_t* neighbour, const double* volume, uint64_t n_faces,
                          uint64_t n_cells, double* gx, double* gy, double* gz, hipStream_t s) {
     return with_index_flag(s, [&](int* bad) {
-        for (double* g : {gx, gy, gz}) zero_f64_kernel<<<face_grid(n_cells), kBlock, 0, s>>>(n_cells, g);
+        face_clear_kernel<<<face_grid(n_cells), kBlock, 0, s>>>(n_cells, gx, gy, gz, bad);
         if (n_faces)
-            face_gradient_kernel<<<face_grid(n_faces), kBlock, 0, s>>>(n_faces, n_cells, phi, sx, sy, sz, owner,
+            face_gradient_kernel<<<chunks(n_faces), kBlock, 0, s>>>(n_faces, n_cells, phi, sx, sy, sz, owner,
                                                                        neighbour, gx, gy, gz, bad);
         inverse_volume_scale_kernel<<<face_grid(n_cells), kBlock, 0, s>>>(n_cells, volume, gx, gy, gz);
     });
@@ -2177,9 +2256,9 @@ bool face_gradient_gauss(const double* phi, const double* sx, const double* sy, 
 bool face_divergence(const double* phi_face, const uint32_t* owner, const int64_t* neighbour, uint64_t n_faces,
                      uint64_t n_cells, double* div, hipStream_t s) {
     return with_index_flag(s, [&](int* bad) {
-        zero_f64_kernel<<<face_grid(n_cells), kBlock, 0, s>>>(n_cells, div);
+        face_clear_kernel<<<face_grid(n_cells), kBlock, 0, s>>>(n_cells, div, nullptr, nullptr, bad);
         if (n_faces)
-            face_divergence_kernel<<<face_grid(n_faces), kBlock, 0, s>>>(n_faces, n_cells, phi_face, owner,
+            face_divergence_kernel<<<chunks(n_faces), kBlock, 0, s>>>(n_faces, n_cells, phi_face, owner,
                                                                          neighbour, div, bad);
     });
 }
