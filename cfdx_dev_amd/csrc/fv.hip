@@ -184,10 +184,13 @@ __global__ __launch_bounds__(kBlock) void cell_volume_kernel(uint32_t nc, const 
 // instead of gathering the face and neighbour-cell arrays face by face.
 //   other: the cell across an internal face, -1 for a boundary face, -2 for
 //          an EMPTY face or an unused slot;
-//   face:  the face;
+//   face:  the face; the top bit is set on the neighbour's side of an internal
+//          face (a boundary face's entry is the plain id; 2^31 faces are
+//          beyond what the slots of a mesh could be stored for);
 //   w:     the distance weight dn / (dc + dn) of an internal face (the
 //          Green-Gauss face interpolation);
 //   s:     the face area vector oriented out of the cell.
+constexpr uint32_t kFaceReversed = 0x80000000u;
 struct Slots {
     int32_t* other;
     uint32_t* face;
@@ -201,12 +204,15 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
                                                            const int32_t* __restrict__ neigh,
                                                            const uint32_t* __restrict__ patch, uint32_t npatch,
                                                            const uint8_t* __restrict__ kind, Soa3 fc, Soa3 fs,
-                                                           Soa3 cc, Slots sl, int* __restrict__ err) {
+                                                           Soa3 cc, const double* __restrict__ vol,
+                                                           double4* __restrict__ cell, Slots sl,
+                                                           int* __restrict__ err) {
 #pragma clang fp contract(off)
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= nc) return;
     const uint32_t deg = coff[c + 1] - coff[c];
     const D3 centre = cc.get(c);
+    cell[c] = make_double4(centre.x, centre.y, centre.z, vol[c]);
     for (uint32_t q = 0; q < D; ++q) {
         const size_t idx = size_t(q) * nc + c;
         if (q >= deg) {
@@ -218,7 +224,7 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
         }
         const uint32_t f = cf[coff[c] + q];
         const bool own = owner[f] == c;
-        sl.face[idx] = f;
+        sl.face[idx] = own ? f : f | kFaceReversed;
         sl.s.set(idx, own ? fs.get(f) : mul3(fs.get(f), -1.0));
         if (neigh[f] >= 0) {
             const uint32_t other = own ? uint32_t(neigh[f]) : owner[f];
@@ -235,45 +241,78 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
     }
 }
 
+// The cell block of a launch's workgroup: each XCD takes one contiguous range
+// of cells (workgroups go to the XCDs in turn), so that the records a cell and
+// its neighbours share are fetched into one L2 rather than into most of them.
+__device__ __forceinline__ uint32_t xcd_block() {
+    const uint32_t nb = gridDim.x, b = blockIdx.x, x = b & 7u;
+    return x * (nb >> 3) + min(x, nb & 7u) + (b >> 3);
+}
+
+// Slots a thread loads together: the loads of one slot depend on each other
+// (cell id, then that cell's record), so a thread that walks them one by one
+// waits for two round trips a face. Enough waves are resident to hide most of
+// it: the gradient of a 128^3 box takes 157 us one by one, 151 by threes, 146
+// by sixes, which cost half again the registers.
+constexpr uint32_t kSlotBatch = 3, kRowBatch = 2;
+
 // gauss_gradient_with_boundary over the slot stencils. bc arrays are per
-// patch: type 0 none/zero-gradient, 1 fixed value, 2 fixed gradient.
+// patch: type 0 none/zero-gradient, 1 fixed value, 2 fixed gradient. The field
+// value of cell i is p[i * ps]; kRec writes one record (gx, gy, gz, 0) a cell,
+// else three arrays. Bound by the slots' 36 bytes a face and side.
+template <bool kRec>
 __global__ __launch_bounds__(kBlock) void gauss_gradient_kernel(
-    uint32_t nc, const uint32_t* __restrict__ coff, Slots sl, const uint32_t* __restrict__ patch, uint32_t npatch,
+    uint32_t nc, uint32_t D, Slots sl, const uint32_t* __restrict__ patch, uint32_t npatch,
     const uint8_t* __restrict__ bct, const double* __restrict__ bcv, Soa3 fc, Soa3 cc, const double* __restrict__ vol,
-    const double* __restrict__ p, double* __restrict__ grad) {
+    const double* __restrict__ p, uint32_t ps, double* __restrict__ grad) {
 #pragma clang fp contract(off)
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t c = xcd_block() * kBlock + threadIdx.x;
     if (c >= nc) return;
-    const uint32_t deg = coff[c + 1] - coff[c];
-    const double pc = p[c];
+    const double pc = p[size_t(c) * ps];
     D3 sum = d3(0.0, 0.0, 0.0);
-    for (uint32_t q = 0; q < deg; ++q) {
-        const size_t idx = size_t(q) * nc + c;
-        const int32_t o = sl.other[idx];
-        if (o == -2) continue;
-        const D3 Sf = sl.s.get(idx);
-        double vf = pc;
-        if (o >= 0) {
-            const double w = sl.w[idx];
-            vf = w * pc + (1.0 - w) * p[o];
-        } else {
-            const uint32_t f = sl.face[idx];
-            const uint32_t pp = patch[f];
-            if (pp < npatch) {
-                if (bct[pp] == 1) {
-                    vf = bcv[pp];
-                } else if (bct[pp] == 2) {
-                    const D3 out = mul3(Sf, 1.0 / mag3(Sf));
-                    vf += bcv[pp] * dot3(sub3(fc.get(f), cc.get(c)), out);
+    for (uint32_t q0 = 0; q0 < D; q0 += kSlotBatch) {
+        int32_t o[kSlotBatch];
+        double po[kSlotBatch], w[kSlotBatch];
+        D3 S[kSlotBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kSlotBatch; ++j) {
+            const size_t idx = size_t(min(q0 + j, D - 1)) * nc + c;
+            o[j] = q0 + j < D ? sl.other[idx] : -2;
+            w[j] = sl.w[idx];
+            S[j] = sl.s.get(idx);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kSlotBatch; ++j) po[j] = p[size_t(o[j] >= 0 ? uint32_t(o[j]) : c) * ps];
+#pragma unroll
+        for (uint32_t j = 0; j < kSlotBatch; ++j) {
+            if (o[j] == -2) continue;
+            const D3 Sf = S[j];
+            double vf = pc;
+            if (o[j] >= 0) {
+                vf = w[j] * pc + (1.0 - w[j]) * po[j];
+            } else {
+                const uint32_t f = sl.face[size_t(q0 + j) * nc + c];
+                const uint32_t pp = patch[f];
+                if (pp < npatch) {
+                    if (bct[pp] == 1) {
+                        vf = bcv[pp];
+                    } else if (bct[pp] == 2) {
+                        const D3 out = mul3(Sf, 1.0 / mag3(Sf));
+                        vf += bcv[pp] * dot3(sub3(fc.get(f), cc.get(c)), out);
+                    }
                 }
             }
+            sum = add3(sum, mul3(Sf, vf));
         }
-        sum = add3(sum, mul3(Sf, vf));
     }
     const double invV = 1.0 / vol[c];
-    grad[c] = sum.x * invV;
-    grad[nc + c] = sum.y * invV;
-    grad[2 * size_t(nc) + c] = sum.z * invV;
+    if (kRec) {
+        reinterpret_cast<double4*>(grad)[c] = make_double4(sum.x * invV, sum.y * invV, sum.z * invV, 0.0);
+    } else {
+        grad[c] = sum.x * invV;
+        grad[nc + c] = sum.y * invV;
+        grad[2 * size_t(nc) + c] = sum.z * invV;
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void mass_flux_kernel(uint32_t nf, uint32_t nc, const uint32_t* __restrict__ owner,
@@ -305,7 +344,10 @@ __global__ __launch_bounds__(kBlock) void mass_flux_kernel(uint32_t nf, uint32_t
 
 // ---------------------------------------------------------- pressure ----
 
-__device__ __forceinline__ bool ortho_coeff(D3 Sf, D3 dv, D3 dAU, double& out) {
+// Orthogonal coefficient (S.e)(dAU e.e)/|d| of a face and the flux of the
+// gradient g beyond its orthogonal part; false when the geometry does not
+// admit them.
+__device__ __forceinline__ bool face_pressure_terms(D3 Sf, D3 dv, D3 dAU, D3 g, double& coeff, double& flux) {
 #pragma clang fp contract(off)
     const double d = mag3(dv);
     const double area = mag3(Sf);
@@ -314,136 +356,236 @@ __device__ __forceinline__ bool ortho_coeff(D3 Sf, D3 dv, D3 dAU, double& out) {
     const double oa = dot3(Sf, e);
     if (!(oa > 0.0) || !isfinite(oa)) return false;
     const double rfn = dAU.x * e.x * e.x + dAU.y * e.y * e.y + dAU.z * e.z * e.z;
-    out = rfn * oa / d;
-    return isfinite(out);
-}
-
-__device__ __forceinline__ bool nonortho_flux(D3 Sf, D3 dv, D3 dAU, D3 g, double& out) {
-#pragma clang fp contract(off)
-    const double d = mag3(dv);
-    if (!(d > 0.0) || !isfinite(d)) return false;
-    const D3 e = d3(dv.x / d, dv.y / d, dv.z / d);
-    const double oa = dot3(Sf, e);
-    const double rfn = dAU.x * e.x * e.x + dAU.y * e.y * e.y + dAU.z * e.z * e.z;
+    coeff = rfn * oa / d;
     const double full = dAU.x * g.x * Sf.x + dAU.y * g.y * Sf.y + dAU.z * g.z * Sf.z;
     const double impl = rfn * dot3(g, e) * oa;
-    out = full - impl;
-    return isfinite(out);
+    flux = full - impl;
+    return isfinite(coeff) && isfinite(flux);
 }
 
-// Per face: internal -> coeff (rho * orthogonal coefficient) and the
-// Rhie-Chow pressure flux; fixed-pressure boundary -> boundary coefficient
-// and source. Weights are the default w = 1/2.
-__global__ __launch_bounds__(kBlock) void pressure_face_kernel(
-    uint32_t nf, uint32_t nc, const uint32_t* __restrict__ owner, const int32_t* __restrict__ neigh,
-    const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ pbt,
-    const double* __restrict__ pbv, double rho, Soa3 fc, Soa3 fs, Soa3 cc, const double* __restrict__ vol,
-    const double* __restrict__ rAU, const double* __restrict__ p, const double* __restrict__ grad,
-    double* __restrict__ coeff, double* __restrict__ bsrc, const double* __restrict__ phi,
-    const uint8_t* __restrict__ slot_o, const uint8_t* __restrict__ slot_n, double* __restrict__ s_phi,
-    double* __restrict__ s_rc, double* __restrict__ s_coeff, int* __restrict__ err) {
-#pragma clang fp contract(off)
-    const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nf) return;
-    const uint32_t o = owner[f];
-    const int32_t nb = neigh[f];
-    const size_t n2 = 2 * size_t(nc);
-    // Continuity terms of this face in its cells' slots (EMPTY faces too: the
-    // reference's continuity loop visits every face of the cell).
-    const size_t io = size_t(slot_o[f]) * nc + o;
-    const double ph = phi[f];
-    s_phi[io] = ph;
-    double cf = 0.0, bs = 0.0;
-    if (nb >= 0) {
-        const uint32_t n = uint32_t(nb);
-        const double wn = 0.5, wo = 1.0 - wn;
-        const D3 dAU = d3(wo * vol[o] * rAU[o] + wn * vol[n] * rAU[n],
-                          wo * vol[o] * rAU[nc + o] + wn * vol[n] * rAU[nc + n],
-                          wo * vol[o] * rAU[n2 + o] + wn * vol[n] * rAU[n2 + n]);
-        const D3 gp = d3(wo * grad[o] + wn * grad[n], wo * grad[nc + o] + wn * grad[nc + n],
-                         wo * grad[n2 + o] + wn * grad[n2 + n]);
-        const D3 Sf = fs.get(f);
-        const D3 dv = sub3(cc.get(n), cc.get(o));
-        double ic = 0.0, nof = 0.0;
-        if (!ortho_coeff(Sf, dv, dAU, ic) || !nonortho_flux(Sf, dv, dAU, gp, nof)) {
-            err[0] = 3;
-            coeff[f] = 0.0;
-            bsrc[f] = 0.0;
-            return;
-        }
-        cf = rho * ic;
-        const double rc = rho * (ic * (p[n] - p[o]) + nof);
-        const size_t in = size_t(slot_n[f]) * nc + n;
-        s_phi[in] = -ph;
-        s_rc[io] = -rc;
-        s_rc[in] = rc;
-        s_coeff[io] = cf;
-        s_coeff[in] = cf;
-    } else {
-        const uint32_t pp = patch[f];
-        if (pp < npatch && pbt[pp] == 1) {
-            const D3 dv = sub3(fc.get(f), cc.get(o));
-            const D3 Sf = fs.get(f);
-            const D3 dAU = d3(vol[o] * rAU[o], vol[o] * rAU[nc + o], vol[o] * rAU[n2 + o]);
-            double bc = 0.0, def = 0.0;
-            const D3 gp = d3(grad[o], grad[nc + o], grad[n2 + o]);
-            if (!ortho_coeff(Sf, dv, dAU, bc) || !nonortho_flux(Sf, dv, dAU, gp, def)) {
-                err[0] = 3;
-            } else {
-                cf = rho * bc;
-                bs = rho * (bc * (pbv[pp] - p[o]) + def);
-            }
-        }
-    }
-    coeff[f] = cf;
-    bsrc[f] = bs;
-}
-
-// Per cell: continuity in cell-face list order (±phiHbyA, ∓RC flux),
-// diagonal = internal coefficients then fixed-pressure boundary
-// coefficients, both in ascending caller face id; rhs = -continuity +
-// boundary sources. Per-face terms come from the cell's slots.
-__global__ __launch_bounds__(kBlock) void pressure_cell_kernel(
-    uint32_t nc, const uint32_t* __restrict__ coff, const uint8_t* __restrict__ slot_sorted, Slots sl,
-    const double* __restrict__ s_phi, const double* __restrict__ s_rc, const double* __restrict__ s_coeff,
-    const double* __restrict__ coeff, const double* __restrict__ bsrc, const uint32_t* __restrict__ patch,
-    uint32_t npatch, const uint8_t* __restrict__ pbt, double* __restrict__ diag, double* __restrict__ rhs) {
-#pragma clang fp contract(off)
+// The cell fields of one assembly as a record a cell, (x, y, z, w), in the
+// internal numbering: read in the caller's order, written as one 32-byte
+// record, so that a permuted mesh costs one scattered access a cell instead of
+// one a field, and a neighbour's fields arrive together. v: 3 x nc.
+__global__ __launch_bounds__(kBlock) void pack_cells_kernel(uint32_t nc, const uint32_t* __restrict__ to,
+                                                           const double* __restrict__ v,
+                                                           const double* __restrict__ w, double4* __restrict__ rec) {
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= nc) return;
-    const uint32_t deg = coff[c + 1] - coff[c];
-    double cont = 0.0;
-    for (uint32_t q = 0; q < deg; ++q) {
-        const size_t idx = size_t(q) * nc + c;
-        cont += s_phi[idx];
-        if (sl.other[idx] >= 0) cont += s_rc[idx];
-    }
-    double d = 0.0;
-    for (uint32_t k = 0; k < deg; ++k) {
-        const size_t idx = size_t(slot_sorted[size_t(k) * nc + c]) * nc + c;
-        if (sl.other[idx] >= 0) d += s_coeff[idx];
-    }
-    double dd = 0.0 + d;
-    double b = -cont;
-    for (uint32_t k = 0; k < deg; ++k) {
-        const size_t idx = size_t(slot_sorted[size_t(k) * nc + c]) * nc + c;
-        if (sl.other[idx] >= 0) continue;
-        const uint32_t f = sl.face[idx];
-        if (patch[f] < npatch && pbt[patch[f]] == 1) {
-            dd += coeff[f];
-            b += bsrc[f];
-        }
-    }
-    diag[c] = dd;
-    rhs[c] = b;
+    rec[to ? to[c] : c] = make_double4(v[c], v[size_t(nc) + c], v[2 * size_t(nc) + c], w[c]);
 }
 
-// CSR values of the full system: diagonal from diag[], off-diagonals
-// 0 - coeff(f1) - coeff(f2) ... over the faces joining the pair. With src,
-// output k takes the full system's nonzero src[k] (the reduced system of a
-// reference-cell elimination, written without a full-size copy).
-__global__ __launch_bounds__(kBlock) void csr_values_kernel(uint64_t nnz, const uint32_t* __restrict__ src,
-                                                           const uint32_t* __restrict__ nz_row_diag,
+// Where the rows of an assembled matrix go: internal cell c fills the entries
+// from start[c] (~0: the row is left out) and right-hand side entry row[c];
+// rank[k * nc + c] is the entry, counted from the row's start, of the cell's
+// k-th slot in ascending caller face id (kNoEntry: boundary face or column
+// left out), diag[c] that of the diagonal. shared: some pair of cells is
+// joined by several faces, whose entries coincide.
+constexpr uint16_t kNoEntry = 0xffffu;
+struct RowMap {
+    const uint32_t *start, *row;
+    const uint16_t *rank, *diag;
+    int shared;
+};
+
+// A wave's rows from LDS to the matrix: row i of the wave (its length len and
+// first nonzero start held by lane i) lies at rows + i * stride. Eight lanes
+// share a row, so that a row of a randomly numbered mesh is written in one or
+// two requests rather than one a value: those go to memory in 32-byte pieces.
+__device__ __forceinline__ void store_rows(const double* rows, uint32_t stride, uint32_t start, uint32_t len,
+                                           double* __restrict__ vals) {
+    const uint32_t lane = threadIdx.x & 63u, e = lane & 7u;
+#pragma unroll
+    for (uint32_t r0 = 0; r0 < 64; r0 += 8) {
+        const uint32_t r = r0 + (lane >> 3);
+        const uint32_t at = __shfl(start, r), n = __shfl(len, r);
+        for (uint32_t k = e; k < n; k += 8) vals[size_t(at) + k] = rows[r * stride + k];
+    }
+}
+
+// The block's own records in LDS: on the curve most neighbours of a cell lie in
+// its block, and gathers through L1 bound the kernels that take all of a
+// neighbour's fields from memory.
+struct Near {
+    double2* at;  // [half][kBlock]
+    uint32_t first;
+
+    __device__ __forceinline__ void put(uint32_t k, double4 v) const {
+        at[2 * k * kBlock + threadIdx.x] = make_double2(v.x, v.y);
+        at[(2 * k + 1) * kBlock + threadIdx.x] = make_double2(v.z, v.w);
+    }
+    __device__ __forceinline__ bool has(uint32_t c) const { return c - first < uint32_t(kBlock); }
+    __device__ __forceinline__ double4 get(uint32_t k, uint32_t c) const {
+        const double2 a = at[2 * k * kBlock + (c - first)], b = at[(2 * k + 1) * kBlock + (c - first)];
+        return make_double4(a.x, a.y, b.x, b.y);
+    }
+};
+
+// LDS of a workgroup that assembles rows of up to D + 1 entries beside nrec
+// staged records: the rows take the records' place once those are read.
+// Hexahedra (6 slots) take 36 KB and polyhedra up to kRowSlots 48 KB, so three
+// or more workgroups, what the registers allow, share a CU's 160 KB.
+constexpr uint32_t kRowSlots = 12;
+inline size_t row_lds(uint32_t D, uint32_t nrec) {
+    return size_t(kBlock) * 8 * (D + std::max(4 * nrec, D + 1));
+}
+
+// One row of the pressure system per thread (internal cell c): continuity in
+// cell-face list order (+-phiHbyA, -+Rhie-Chow flux of the pressure), the
+// diagonal = internal coefficients then fixed-pressure boundary coefficients,
+// both in ascending caller face id, off-diagonals 0 - coefficient of each
+// joining face, rhs = -continuity + boundary sources; weights are the default
+// w = 1/2. Every face is evaluated from both of its cells: its flux changes
+// sign and its coefficient is the same to the last bit from either side
+// (differences, the area vector and so the unit vector negate exactly, and the
+// weighted sums commute), so nothing has to pass between the cells. Bound by
+// memory: 36 bytes of stencil a slot, three 32-byte records a cell that its
+// neighbours share, the row's values; the arithmetic is free beside it (taking
+// it out changed nothing). kLds: the slots' coefficients wait for the second
+// order in LDS, the block's records are staged and the rows leave by
+// store_rows; else (many slots a cell) coefficients wait in sbuf and values
+// are written one by one. On a 128^3 box of randomly numbered cells: 312 us;
+// 587 with values written one by one and all neighbours' records read from
+// memory (294 of it the writes, 125 the gathers); 762 as a pass over faces
+// that scattered its terms to the cells, one over cells and one over nonzeros.
+template <bool kLds>
+__global__ __launch_bounds__(kBlock) void pressure_row_kernel(
+    uint32_t nc, uint32_t D, const uint32_t* __restrict__ coff, const uint8_t* __restrict__ slot_sorted, Slots sl,
+    const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ pbt,
+    const double* __restrict__ pbv, double rho, Soa3 fc, const double4* __restrict__ cell,
+    const double4* __restrict__ fields, const double4* __restrict__ grad, const double* __restrict__ phi,
+    double* __restrict__ sbuf, RowMap rm, double* __restrict__ vals, double* __restrict__ rhs,
+    int* __restrict__ err) {
+#pragma clang fp contract(off)
+    extern __shared__ double2 row_shared[];
+    const uint32_t first = xcd_block() * kBlock;
+    const bool live = first + threadIdx.x < nc;
+    const uint32_t c = live ? first + threadIdx.x : nc - 1;  // the last block's spare threads only keep step
+    double* lds = reinterpret_cast<double*>(row_shared);
+    double* cbuf = kLds ? lds + threadIdx.x : sbuf + c;
+    const size_t cs = kLds ? size_t(kBlock) : size_t(nc);
+    const Near near{reinterpret_cast<double2*>(lds + size_t(D) * kBlock), first};
+    const uint32_t deg = live ? coff[c + 1] - coff[c] : 0;
+    const double4 C = cell[c], A = fields[c], G = grad[c];
+    if (kLds) {
+        near.put(0, C);
+        near.put(1, A);
+        near.put(2, G);
+        __syncthreads();
+    }
+    const double wh = 0.5;
+    const D3 ra = d3(wh * C.w * A.x, wh * C.w * A.y, wh * C.w * A.z);
+    const D3 gh = d3(wh * G.x, wh * G.y, wh * G.z);
+    double cont = 0.0;
+    bool fixed = false;
+    for (uint32_t q0 = 0; q0 < D; q0 += kRowBatch) {
+        int32_t o[kRowBatch];
+        uint32_t f[kRowBatch];
+        double ph[kRowBatch];
+        D3 S[kRowBatch];
+        double4 Cn[kRowBatch], An[kRowBatch], Gn[kRowBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kRowBatch; ++j) {
+            const size_t idx = size_t(min(q0 + j, D - 1)) * nc + c;
+            o[j] = q0 + j < deg ? sl.other[idx] : -3;
+            f[j] = sl.face[idx];
+            S[j] = sl.s.get(idx);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kRowBatch; ++j) {
+            const uint32_t n = o[j] >= 0 ? uint32_t(o[j]) : c;
+            ph[j] = phi[f[j] & ~kFaceReversed];
+            if (kLds && near.has(n)) {
+                Cn[j] = near.get(0, n);
+                An[j] = near.get(1, n);
+                Gn[j] = near.get(2, n);
+            } else {
+                Cn[j] = cell[n];
+                An[j] = fields[n];
+                Gn[j] = grad[n];
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kRowBatch; ++j) {
+            if (o[j] == -3) continue;
+            double cf = 0.0;
+            cont += f[j] & kFaceReversed ? -ph[j] : ph[j];
+            if (o[j] >= 0) {
+                const D3 dAU = add3(ra, d3(wh * Cn[j].w * An[j].x, wh * Cn[j].w * An[j].y, wh * Cn[j].w * An[j].z));
+                const D3 gp = add3(gh, d3(wh * Gn[j].x, wh * Gn[j].y, wh * Gn[j].z));
+                const D3 dv = d3(Cn[j].x - C.x, Cn[j].y - C.y, Cn[j].z - C.z);
+                double ic = 0.0, nof = 0.0;
+                if (!face_pressure_terms(S[j], dv, dAU, gp, ic, nof)) err[0] = 3;
+                cf = rho * ic;
+                cont -= rho * (ic * (An[j].w - A.w) + nof);
+            } else {
+                const uint32_t pp = patch[f[j]];
+                fixed |= pp < npatch && pbt[pp] == 1;
+            }
+            cbuf[(q0 + j) * cs] = cf;
+        }
+    }
+    if (kLds) __syncthreads();  // the rows take the records' place
+    const uint32_t start = rm.start[c], stride = D + 1;
+    double* row = kLds ? lds + size_t(D) * kBlock + threadIdx.x * stride : vals + size_t(start);
+    double d = 0.0;
+    uint32_t len = 0;
+    for (uint32_t k = 0; k < deg; ++k) {
+        const double cf = cbuf[slot_sorted[size_t(k) * nc + c] * cs];
+        d += cf;
+        const uint16_t r = rm.rank[size_t(k) * nc + c];
+        if (r == kNoEntry) continue;
+        len = max(len, uint32_t(r) + 1u);
+        if (!rm.shared) row[r] = 0.0 - cf;
+    }
+    if (rm.shared) {
+        // Entries of faces that join one pair: summed at the first of them.
+        for (uint32_t k = 0; k < deg; ++k) {
+            const uint16_t r = rm.rank[size_t(k) * nc + c];
+            bool fresh = r != kNoEntry;
+            for (uint32_t j = 0; j < k && fresh; ++j) fresh = rm.rank[size_t(j) * nc + c] != r;
+            if (!fresh) continue;
+            double v = 0.0;
+            for (uint32_t j = k; j < deg; ++j)
+                if (rm.rank[size_t(j) * nc + c] == r) v -= cbuf[slot_sorted[size_t(j) * nc + c] * cs];
+            row[r] = v;
+        }
+    }
+    double b = -cont;
+    if (fixed) {
+        const D3 dAU = d3(C.w * A.x, C.w * A.y, C.w * A.z);
+        for (uint32_t k = 0; k < deg; ++k) {
+            const size_t idx = size_t(slot_sorted[size_t(k) * nc + c]) * nc + c;
+            if (sl.other[idx] >= 0) continue;
+            const uint32_t f = sl.face[idx];
+            const uint32_t pp = patch[f];
+            if (!(pp < npatch && pbt[pp] == 1)) continue;
+            double bc = 0.0, def = 0.0;
+            if (!face_pressure_terms(sl.s.get(idx), sub3(fc.get(f), d3(C.x, C.y, C.z)), dAU, d3(G.x, G.y, G.z), bc,
+                                     def)) {
+                err[0] = 3;
+                continue;
+            }
+            d += rho * bc;
+            b += rho * (bc * (pbv[pp] - A.w) + def);
+        }
+    }
+    const bool kept = live && start != 0xffffffffu;
+    if (kept) {
+        const uint32_t r = rm.diag[c];
+        row[r] = d;
+        len = max(len, r + 1u);
+        rhs[rm.row[c]] = b;
+    }
+    if (kLds) {
+        wave_fence();
+        store_rows(lds + size_t(D) * kBlock + (threadIdx.x & ~63u) * stride, stride, start, kept ? len : 0, vals);
+    }
+}
+
+// CSR values of the diffusion system: diagonal from diag[], off-diagonals
+// 0 - coeff(f1) - coeff(f2) ... over the faces joining the pair.
+__global__ __launch_bounds__(kBlock) void csr_values_kernel(uint64_t nnz, const uint32_t* __restrict__ nz_row_diag,
                                                            const uint32_t* __restrict__ nzf_off,
                                                            const uint32_t* __restrict__ nzf,
                                                            const double* __restrict__ diag,
@@ -452,14 +594,13 @@ __global__ __launch_bounds__(kBlock) void csr_values_kernel(uint64_t nnz, const 
 #pragma clang fp contract(off)
     const uint64_t k = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
     if (k >= nnz) return;
-    const uint64_t j = src ? src[k] : k;
-    const uint32_t dr = nz_row_diag[j];
+    const uint32_t dr = nz_row_diag[k];
     if (dr != 0xffffffffu) {
         vals[k] = diag[dr];
         return;
     }
     double v = 0.0;
-    for (uint32_t q = nzf_off[j]; q < nzf_off[j + 1]; ++q) v -= coeff[nzf[q]];
+    for (uint32_t q = nzf_off[k]; q < nzf_off[k + 1]; ++q) v -= coeff[nzf[q]];
     vals[k] = v;
 }
 
@@ -1264,7 +1405,7 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
     const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ kind,
     const uint8_t* __restrict__ vbt, const double* __restrict__ vbv, const uint8_t* __restrict__ pbt,
     const double* __restrict__ pbv, double rho, Soa3 fc, Soa3 fs, Soa3 cc, const double* __restrict__ vol,
-    const double* __restrict__ H, const double* __restrict__ p, const double* __restrict__ grad,
+    const double* __restrict__ H, const double* __restrict__ p, const double4* __restrict__ grad,
     const double* __restrict__ rAU, double* __restrict__ phi, int* __restrict__ err) {
 #pragma clang fp contract(off)
     const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
@@ -1282,11 +1423,11 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
         const D3 dAU = d3(wo * vol[o] * rAU[o] + wn * vol[n] * rAU[n],
                           wo * vol[o] * rAU[nc + o] + wn * vol[n] * rAU[nc + n],
                           wo * vol[o] * rAU[n2 + o] + wn * vol[n] * rAU[n2 + n]);
-        const D3 gp = d3(wo * grad[o] + wn * grad[n], wo * grad[nc + o] + wn * grad[nc + n],
-                         wo * grad[n2 + o] + wn * grad[n2 + n]);
+        const double4 go = grad[o], gn = grad[n];
+        const D3 gp = d3(wo * go.x + wn * gn.x, wo * go.y + wn * gn.y, wo * go.z + wn * gn.z);
         const D3 dv = sub3(cc.get(n), cc.get(o));
         double ic = 0.0, nofl = 0.0;
-        if (!ortho_coeff(Sf, dv, dAU, ic) || !nonortho_flux(Sf, dv, dAU, gp, nofl)) {
+        if (!face_pressure_terms(Sf, dv, dAU, gp, ic, nofl)) {
             err[0] = 52;
             return;
         }
@@ -1306,10 +1447,11 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
                     err[0] = 52;
                     return;
                 }
-                const D3 gp = d3(grad[o], grad[nc + o], grad[n2 + o]);
+                const double4 go = grad[o];
+                const D3 gp = d3(go.x, go.y, go.z);
                 const D3 dAU = d3(vol[o] * rAU[o], vol[o] * rAU[nc + o], vol[o] * rAU[n2 + o]);
                 double ic = 0.0, def = 0.0;
-                if (!ortho_coeff(Sf, dv, dAU, ic) || !nonortho_flux(Sf, dv, dAU, gp, def)) {
+                if (!face_pressure_terms(Sf, dv, dAU, gp, ic, def)) {
                     err[0] = 52;
                     return;
                 }
@@ -1327,8 +1469,8 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
 // Internal numbering. A caller's cells may be numbered without locality (the
 // benchmark boxes are a random permutation), and a kernel that gathers cell or
 // face data through such ids reads a whole cache line per 8-byte value. The
-// handle therefore keeps the mesh in its own order: cells in reverse
-// Cuthill-McKee order of the cell graph, faces grouped by owner in that order
+// handle therefore keeps the mesh in its own order: cells along a Hilbert
+// curve through their centres, faces grouped by owner in that order
 // (caller order within an owner). Every kernel runs on the internal arrays;
 // the public methods take and return caller-ordered fields and permute them
 // once on the way in and out. Each cell keeps its caller face list order
@@ -1336,6 +1478,91 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
 // accumulates in face order (cfaces_sorted), so every value is unchanged.
 
 namespace {
+
+// Hilbert index of a point of the 2^16 cube (J. Skilling, Programming the
+// Hilbert curve, AIP Conf. Proc. 707, 2004): the axes' bits are turned into
+// the curve's transposed index from the top bit down, then interleaved.
+uint64_t hilbert_key(uint32_t x, uint32_t y, uint32_t z) {
+    uint32_t a[3] = {x, y, z};
+    for (uint32_t q = 1u << 15; q > 1; q >>= 1) {
+        const uint32_t low = q - 1;
+        for (int i = 0; i < 3; ++i) {
+            if (a[i] & q) {
+                a[0] ^= low;
+            } else {
+                const uint32_t t = (a[0] ^ a[i]) & low;
+                a[0] ^= t;
+                a[i] ^= t;
+            }
+        }
+    }
+    a[1] ^= a[0];
+    a[2] ^= a[1];
+    uint32_t t = 0;
+    for (uint32_t q = 1u << 15; q > 1; q >>= 1)
+        if (a[2] & q) t ^= q - 1;
+    uint64_t key = 0;
+    for (int b = 15; b >= 0; --b)
+        for (int i = 0; i < 3; ++i) key = (key << 1) | (((a[i] ^ t) >> b) & 1u);
+    return key;
+}
+
+// Cells in the order of a Hilbert curve through their vertices' means, each
+// axis scaled by the distribution of the cells along it (grids are stretched
+// towards walls by factors of a thousand: equal steps of the key then hold
+// equally many cells). Ties keep the caller's order. The order only sets where
+// values lie: it needs no accuracy, and takes any coordinates.
+void curve_ordering(uint32_t nc, const uint32_t* coff, const uint32_t* cf, const uint32_t* foff,
+                    const uint32_t* fvtx, const double* px, const double* py, const double* pz,
+                    std::vector<uint32_t>& order) {
+    constexpr uint32_t kBins = 1u << 16;
+    std::vector<double> centre[3];
+    for (auto& v : centre) v.resize(nc);
+    parallel_for(nc, 0, [&](uint64_t c) {
+        double s[3] = {0.0, 0.0, 0.0};
+        uint32_t n = 0;
+        for (uint32_t k = coff[c]; k < coff[c + 1]; ++k)
+            for (uint32_t q = foff[cf[k]]; q < foff[cf[k] + 1]; ++q, ++n) {
+                s[0] += px[fvtx[q]];
+                s[1] += py[fvtx[q]];
+                s[2] += pz[fvtx[q]];
+            }
+        for (int d = 0; d < 3; ++d) centre[d][c] = n ? s[d] / n : 0.0;
+    });
+    std::vector<uint16_t> axis[3];
+    for (int d = 0; d < 3; ++d) {
+        axis[d].resize(nc);
+        double lo = INFINITY, hi = -INFINITY;
+        for (double v : centre[d])
+            if (std::isfinite(v)) lo = std::min(lo, v), hi = std::max(hi, v);
+        const double scale = hi > lo ? (kBins - 1) / (hi - lo) : 0.0;
+        std::vector<uint64_t> below(kBins + 1, 0);
+        auto bin = [&](double v) {
+            const double b = (v - lo) * scale;
+            return b >= 0.0 && b <= kBins - 1 ? uint32_t(b) : 0u;
+        };
+        for (double v : centre[d]) ++below[bin(v) + 1];
+        for (uint32_t b = 0; b < kBins; ++b) below[b + 1] += below[b];
+        parallel_for(nc, 0, [&](uint64_t c) {
+            const uint32_t b = bin(centre[d][c]);
+            axis[d][c] = uint16_t((below[b] + below[b + 1]) / 2 * (kBins - 1) / nc);
+        });
+    }
+    std::vector<uint64_t> key(nc);
+    parallel_for(nc, 0, [&](uint64_t c) { key[c] = hilbert_key(axis[0][c], axis[1][c], axis[2][c]); });
+    // Counting sort by 12 bits at a time, stable.
+    order.resize(nc);
+    std::iota(order.begin(), order.end(), 0u);
+    std::vector<uint32_t> next(nc);
+    for (int shift = 0; shift < 48; shift += 12) {
+        std::vector<uint32_t> at(4097, 0);
+        for (uint32_t c = 0; c < nc; ++c) ++at[((key[c] >> shift) & 4095u) + 1];
+        for (int b = 0; b < 4096; ++b) at[b + 1] += at[b];
+        for (uint32_t i = 0; i < nc; ++i) next[at[(key[order[i]] >> shift) & 4095u]++] = order[i];
+        order.swap(next);
+    }
+}
+
 Slots slots_of(const FvMesh& m) {
     return Slots{m.slot_other, m.slot_face, m.slot_w, Soa3{m.slot_sx, m.slot_sy, m.slot_sz}};
 }
@@ -1343,6 +1570,11 @@ WlsCache wls_of(const FvMesh& m) {
     return WlsCache{m.wls_a0, m.wls_a1, m.wls_a2, m.wls_fac, m.wls_nd, m.wls_sig, m.wls_V, m.wls_cond, m.wls_meta};
 }
 }  // namespace
+
+void PressurePlan::release() {
+    for (uint32_t** p : {&rowp, &cols, &nz_row_diag, &nzf_off, &nzf, &row_start, &row_of}) dfree(*p);
+    for (uint16_t** p : {&slot_rank, &diag_rank}) dfree(*p);
+}
 
 FvMesh::~FvMesh() { release(); }
 
@@ -1359,6 +1591,7 @@ void FvMesh::release() {
     scratch.clear();
     dfree(scratch_u8);
     dfree(slot_other);
+    dfree(cell_rec);
     dfree(face_slot_o);
     dfree(face_slot_n);
     dfree(slot_sorted);
@@ -1369,12 +1602,39 @@ void FvMesh::release() {
     dfree(err);
     dfree(mom_flags);
     dfree(bc_u8);
-    for (auto* pl : {&pressure_full, &pressure_red})
-        for (uint32_t** p : {&pl->rowp, &pl->cols, &pl->nz_row_diag, &pl->nzf_off, &pl->nzf, &pl->red_src,
-                             &pl->red_rhs_src})
-            dfree(*p);
+    pressure_full.release();
+    pressure_red.release();
     dfree(pbc_u8);
     dfree(pbc_f64);
+}
+
+// Lines of 16 values that the neighbours and the faces of 64 consecutive cells
+// lie in, summed over up to 1024 such windows spread over the mesh: cells in
+// the order `at` (cell of each place), places cell_place and face_place.
+uint64_t FvMesh::touched_lines(const std::vector<uint32_t>& at, const std::vector<uint32_t>& cell_place,
+                               const std::vector<uint32_t>& face_place) const {
+    const uint32_t windows = (nc + 63) / 64, taken = std::min<uint32_t>(windows, 1024);
+    std::vector<uint32_t> cells, faces;
+    uint64_t lines = 0;
+    for (uint32_t s = 0; s < taken; ++s) {
+        const uint64_t first = uint64_t(s) * windows / taken * 64;
+        cells.clear();
+        faces.clear();
+        for (uint64_t i = first; i < std::min<uint64_t>(first + 64, nc); ++i) {
+            const uint32_t c = at[i];
+            for (uint32_t k = h_coff[c]; k < h_coff[c + 1]; ++k) {
+                const uint32_t f = h_cf[k];
+                faces.push_back(face_place[f] / 16);
+                if (h_neigh[f] >= 0)
+                    cells.push_back(cell_place[h_owner[f] == c ? uint32_t(h_neigh[f]) : h_owner[f]] / 16);
+            }
+        }
+        for (auto* v : {&cells, &faces}) {
+            std::sort(v->begin(), v->end());
+            lines += std::unique(v->begin(), v->end()) - v->begin();
+        }
+    }
+    return lines;
 }
 
 void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy, const double* hz, uint64_t nf_,
@@ -1404,49 +1664,11 @@ void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy
         if (h_cf[k] >= nf) throw std::invalid_argument("cell face index out of range");
     for (uint32_t k = 0; k < hfoff[nf]; ++k)
         if (hfvtx[k] >= np) throw std::invalid_argument("face vertex out of range");
-    // Cell order: reverse Cuthill-McKee of the cell graph.
-    std::vector<uint32_t> cnew, cold(nc), fnew(nf), fold(nf);
+    std::vector<uint32_t> cold(nc), cnew(nc), fnew(nf), fold(nf);
+    // Cells along the curve, faces by internal owner, caller order within one.
+    curve_ordering(nc, h_coff.data(), h_cf.data(), hfoff, hfvtx, hx, hy, hz, cold);
+    for (uint32_t i = 0; i < nc; ++i) cnew[cold[i]] = i;
     {
-        HCsr g;
-        g.n = g.ncols = nc;
-        g.rowp.assign(uint64_t(nc) + 1, 0);
-        for (uint32_t c = 0; c < nc; ++c) {
-            uint32_t d = 0;
-            for (uint32_t k = h_coff[c]; k < h_coff[c + 1]; ++k) d += h_neigh[h_cf[k]] >= 0;
-            g.rowp[c + 1] = g.rowp[c] + d;
-        }
-        g.cols.resize(g.rowp[nc]);
-        parallel_for(nc, 0, [&](uint64_t c) {
-            uint32_t w = g.rowp[c];
-            for (uint32_t k = h_coff[c]; k < h_coff[c + 1]; ++k) {
-                const uint32_t f = h_cf[k];
-                if (h_neigh[f] < 0) continue;
-                g.cols[w++] = h_owner[f] == c ? uint32_t(h_neigh[f]) : h_owner[f];
-            }
-        });
-        cnew = rcm_ordering(g);
-    }
-    // Keep the caller's numbering when it is about as local as RCM (bandwidth
-    // within a factor of two): then no field is permuted at all.
-    {
-        uint64_t bw_caller = 0, bw_rcm = 0;
-        for (uint32_t f = 0; f < nf; ++f) {
-            if (h_neigh[f] < 0) continue;
-            const uint32_t o = h_owner[f], n = uint32_t(h_neigh[f]);
-            bw_caller = std::max<uint64_t>(bw_caller, o > n ? o - n : n - o);
-            const uint32_t a = cnew[o], b = cnew[n];
-            bw_rcm = std::max<uint64_t>(bw_rcm, a > b ? a - b : b - a);
-        }
-        identity_order = bw_caller <= 2 * bw_rcm;
-        if (identity_order) std::iota(cnew.begin(), cnew.end(), 0u);
-    }
-    for (uint32_t c = 0; c < nc; ++c) cold[cnew[c]] = c;
-    // Face order: by internal owner, caller order within an owner (the
-    // caller's order when the cell numbering is kept).
-    if (identity_order) {
-        std::iota(fold.begin(), fold.end(), 0u);
-        std::iota(fnew.begin(), fnew.end(), 0u);
-    } else {
         std::vector<uint32_t> cnt(uint64_t(nc) + 1, 0);
         for (uint32_t f = 0; f < nf; ++f) ++cnt[cnew[h_owner[f]] + 1];
         for (uint32_t c = 0; c < nc; ++c) cnt[c + 1] += cnt[c];
@@ -1454,6 +1676,26 @@ void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy
             const uint32_t pos = cnt[cnew[h_owner[f]]]++;
             fold[pos] = f;
             fnew[f] = pos;
+        }
+    }
+    // Keep the caller's numbering when the accesses of 64 consecutive cells
+    // touch about as few lines in it as on the curve (at most half as many
+    // again): then no field is permuted at all.
+    // Lexicographic numberings of boxes and channels touch 1.05 times the
+    // curve's lines, random ones 9 times. A 222k-cell channel kept as numbered
+    // assembles its pressure in 98 us, moved to another local order in 112 (its
+    // six fields pass through a gather); a random 128^3 box assembled as
+    // numbered would fetch a line for each of its 66M values.
+    {
+        std::vector<uint32_t> same(std::max(nc, nf));
+        std::iota(same.begin(), same.end(), 0u);
+        const uint64_t curve = touched_lines(cold, cnew, fnew), caller = touched_lines(same, same, same);
+        identity_order = 2 * caller <= 3 * curve;
+        if (identity_order) {
+            std::iota(cnew.begin(), cnew.end(), 0u);
+            std::iota(cold.begin(), cold.end(), 0u);
+            std::iota(fold.begin(), fold.end(), 0u);
+            std::iota(fnew.begin(), fnew.end(), 0u);
         }
     }
     // Internal arrays.
@@ -1629,7 +1871,7 @@ void FvMesh::ensure_work() {
     work_phi = dalloc<double>(nf);
     work_diag = dalloc<double>(nc);
     work_rhs = dalloc<double>(nc);
-    work_grad = dalloc<double>(3 * uint64_t(nc));
+    work_grad = dalloc<double>(4 * uint64_t(nc));
     pbc_u8 = dalloc<uint8_t>(std::max<uint32_t>(npatch, 1));
     pbc_f64 = dalloc<double>(std::max<uint32_t>(npatch, 1));
 }
@@ -1642,6 +1884,7 @@ void FvMesh::ensure_slots() {
     if (D > 255) throw std::invalid_argument("cells with more than 255 faces are not supported");
     slot_D = D;
     const uint64_t m = uint64_t(D) * nc;
+    cell_rec = dalloc<double4>(nc);
     slot_other = dalloc<int32_t>(m);
     slot_face = dalloc<uint32_t>(m);
     slot_w = dalloc<double>(m);
@@ -1675,7 +1918,7 @@ void FvMesh::ensure_slots() {
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
     slot_build_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, D, coff, cfaces, owner, neigh, patch, npatch,
-                                                           patch_kind, fc, fs, cc, slots_of(*this), err);
+                                                           patch_kind, fc, fs, cc, vol, cell_rec, slots_of(*this), err);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("cell stencils: degenerate face distances");
 }
@@ -1716,17 +1959,21 @@ void FvMesh::ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt) {
     wls_key = key;
 }
 
-void FvMesh::gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p_i, double* grad_i) {
+// Records (gx, gy, gz, 0) per internal cell of the field p[i * ps].
+void FvMesh::gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps) {
     ensure_slots();
-    const Soa3 fc{fcx, fcy, fcz}, cc{ccx, ccy, ccz};
-    gauss_gradient_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, slots_of(*this), patch, npatch, d_bct, d_bcv, fc, cc,
-                                                               vol, p_i, grad_i);
+    gauss_gradient_kernel<true><<<grid_for(nc), kBlock, 0, stream>>>(
+        nc, slot_D, slots_of(*this), patch, npatch, d_bct, d_bcv, Soa3{fcx, fcy, fcz},
+        Soa3{ccx, ccy, ccz}, vol, p, ps, work_grad);
 }
 
 void FvMesh::gauss_gradient_device(const uint8_t* d_bct, const double* d_bcv, const double* d_p, double* d_grad) {
     const double* p_i = cin(d_p, 9, 1);
     double* g_i = cout_buf(d_grad, 8, 3);
-    gauss_gradient_internal(d_bct, d_bcv, p_i, g_i);
+    ensure_slots();
+    gauss_gradient_kernel<false><<<grid_for(nc), kBlock, 0, stream>>>(
+        nc, slot_D, slots_of(*this), patch, npatch, d_bct, d_bcv, Soa3{fcx, fcy, fcz},
+        Soa3{ccx, ccy, ccz}, vol, p_i, 1, g_i);
     cells_out(g_i, d_grad, 3);
 }
 
@@ -1812,34 +2059,73 @@ const PressurePlan& FvMesh::pressure_plan(bool eliminate, uint32_t ref) {
         full.nz_row_diag = upload(rdiag.data(), rdiag.size());
         full.nzf_off = upload(nzf_off.data(), nzf_off.size());
         full.nzf = upload(nzf.data(), nzf.size());
+        full.shared_pairs = nnz != uint64_t(nc) + fcnt[nc];
+        map_rows(full, 0xffffffffu);
     }
     if (!eliminate) return full;
     PressurePlan& red = pressure_red;
     if (!red.rowp || red.ref != ref) {
-        for (uint32_t** p : {&red.rowp, &red.cols, &red.red_src, &red.red_rhs_src}) dfree(*p);
-        std::vector<uint32_t> rowp{0}, cols, src, rsrc;
+        red.release();
+        std::vector<uint32_t> rowp{0}, cols;
+        rowp.reserve(nc);
+        cols.reserve(full.nnz);
         for (uint32_t c = 0; c < nc; ++c) {
             if (c == ref) continue;
-            rsrc.push_back(h_cell_new[c]);
             for (uint32_t k = full.h_rowp[c]; k < full.h_rowp[c + 1]; ++k) {
                 const uint32_t j = full.h_cols[k];
-                if (j == ref) continue;
-                cols.push_back(j < ref ? j : j - 1);
-                src.push_back(k);
+                if (j != ref) cols.push_back(j < ref ? j : j - 1);
             }
             rowp.push_back(uint32_t(cols.size()));
         }
         red.n = nc - 1;
         red.nnz = cols.size();
         red.ref = ref;
-        red.h_rowp = rowp;
-        red.h_cols = cols;
-        red.rowp = upload(rowp.data(), rowp.size());
-        red.cols = upload(cols.data(), cols.size());
-        red.red_src = upload(src.data(), src.size());
-        red.red_rhs_src = upload(rsrc.data(), rsrc.size());
+        red.h_rowp = std::move(rowp);
+        red.h_cols = std::move(cols);
+        red.shared_pairs = full.shared_pairs;
+        red.rowp = upload(red.h_rowp.data(), red.h_rowp.size());
+        red.cols = upload(red.h_cols.data(), red.h_cols.size());
+        map_rows(red, ref);
     }
     return red;
+}
+
+// Where each internal cell's slots land in the rows of plan (row and column
+// ref left out; ~0: none).
+void FvMesh::map_rows(PressurePlan& plan, uint32_t ref) {
+    ensure_slots();
+    std::vector<uint32_t> start(nc), row(nc), cold(nc);
+    std::vector<uint16_t> rank(uint64_t(slot_D) * nc, kNoEntry), diag(nc, kNoEntry);
+    for (uint32_t c = 0; c < nc; ++c) cold[h_cell_new[c]] = c;
+    auto moved = [&](uint32_t c) { return c > ref ? c - 1 : c; };
+    parallel_chunks(nc, 0, [&](uint64_t b, uint64_t e, uint32_t) {
+        std::vector<uint32_t> faces;
+        for (uint64_t i = b; i < e; ++i) {
+            const uint32_t c = cold[i];
+            if (c == ref) {
+                start[i] = row[i] = 0xffffffffu;
+                continue;
+            }
+            const uint32_t r = moved(c);
+            start[i] = plan.h_rowp[r];
+            row[i] = r;
+            const uint32_t* lo = plan.h_cols.data() + plan.h_rowp[r];
+            const uint32_t* hi = plan.h_cols.data() + plan.h_rowp[r + 1];
+            diag[i] = uint16_t(std::lower_bound(lo, hi, r) - lo);
+            faces.assign(h_cf.begin() + h_coff[c], h_cf.begin() + h_coff[c + 1]);
+            std::sort(faces.begin(), faces.end());
+            for (size_t k = 0; k < faces.size(); ++k) {
+                const uint32_t f = faces[k];
+                if (h_neigh[f] < 0) continue;
+                const uint32_t other = h_owner[f] == c ? uint32_t(h_neigh[f]) : h_owner[f];
+                if (other != ref) rank[k * nc + i] = uint16_t(std::lower_bound(lo, hi, moved(other)) - lo);
+            }
+        }
+    });
+    plan.row_start = upload(start.data(), nc);
+    plan.row_of = upload(row.data(), nc);
+    plan.slot_rank = upload(rank.data(), rank.size());
+    plan.diag_rank = upload(diag.data(), nc);
 }
 
 bool FvMesh::has_fixed_pressure(const uint8_t* h_pbt) const {
@@ -1862,26 +2148,23 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
         HIP_OK(hipMemcpyAsync(d_pbv, h_pbv, size_t(npatch) * 8, hipMemcpyHostToDevice, stream));
     }
     HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
-    const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
-    const double* rau_i = cin(d_rAU, 5, 3);
+    const Soa3 fc{fcx, fcy, fcz};
+    double4* rec = reinterpret_cast<double4*>(scr(5, 4 * uint64_t(nc)));
+    pack_cells_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, d_rAU, d_p, rec);
     const double* phi_i = fin(d_phi, 4);
-    const double* p_i = cin(d_p, 9, 1);
-    gauss_gradient_internal(d_pbt, d_pbv, p_i, work_grad);
-    ensure_slot_terms();
-    pressure_face_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, nc, owner, neigh, patch, npatch, d_pbt, d_pbv, rho,
-                                                              fc, fs, cc, vol, rau_i, p_i, work_grad, work_coeff,
-                                                              work_bsrc, phi_i, face_slot_o, face_slot_n,
-                                                              mom_sdiv, mom_sd0, mom_sdiag, err);
-    pressure_cell_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, slot_sorted, slots_of(*this), mom_sdiv,
-                                                              mom_sd0, mom_sdiag, work_coeff, work_bsrc, patch,
-                                                              npatch, d_pbt, work_diag, work_rhs);
-    csr_values_kernel<<<grid_for(plan.nnz), kBlock, 0, stream>>>(
-        plan.nnz, eliminate ? plan.red_src : nullptr, pressure_full.nz_row_diag, pressure_full.nzf_off,
-        pressure_full.nzf, work_diag, work_coeff, d_vals);
-    if (!eliminate)
-        cells_out(work_rhs, d_rhs, 1);
-    else
-        gather_u32idx_kernel<<<grid_for(plan.n), kBlock, 0, stream>>>(plan.n, plan.red_rhs_src, work_rhs, d_rhs);
+    gauss_gradient_internal(d_pbt, d_pbv, &rec->w, 4);
+    const RowMap rm{plan.row_start, plan.row_of, plan.slot_rank, plan.diag_rank, plan.shared_pairs ? 1 : 0};
+    const double4* grad = reinterpret_cast<const double4*>(work_grad);
+    if (slot_D <= kRowSlots) {
+        pressure_row_kernel<true><<<grid_for(nc), kBlock, row_lds(slot_D, 3), stream>>>(
+            nc, slot_D, coff, slot_sorted, slots_of(*this), patch, npatch, d_pbt, d_pbv, rho, fc, cell_rec, rec, grad,
+            phi_i, nullptr, rm, d_vals, d_rhs, err);
+    } else {
+        ensure_slot_terms();
+        pressure_row_kernel<false><<<grid_for(nc), kBlock, 0, stream>>>(
+            nc, slot_D, coff, slot_sorted, slots_of(*this), patch, npatch, d_pbt, d_pbv, rho, fc, cell_rec, rec, grad,
+            phi_i, mom_sdiag, rm, d_vals, d_rhs, err);
+    }
     HIP_OK(hipStreamSynchronize(stream));
     check_err("pressure_face_orthogonal_coefficient: invalid face geometry or orientation");
     return plan;
@@ -1906,7 +2189,7 @@ const PressurePlan& FvMesh::diffusion_assemble_device(double gamma, const double
                                                                work_coeff, err);
     diffusion_cell_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, cfaces_sorted, neigh, fs, vol, src_i, fval_i,
                                                                fneu_i, work_coeff, work_diag, rhs_i);
-    csr_values_kernel<<<grid_for(plan.nnz), kBlock, 0, stream>>>(plan.nnz, nullptr, plan.nz_row_diag, plan.nzf_off,
+    csr_values_kernel<<<grid_for(plan.nnz), kBlock, 0, stream>>>(plan.nnz, plan.nz_row_diag, plan.nzf_off,
                                                                  plan.nzf, work_diag, work_coeff, d_vals);
     cells_out(rhs_i, d_rhs, 1);
     HIP_OK(hipStreamSynchronize(stream));
@@ -2059,10 +2342,11 @@ void FvMesh::rhie_chow_flux_device(const uint8_t* h_vbt, const double* h_vbv, co
     const double* rau_i = cin(d_rau, 5, 3);
     const double* p_i = cin(d_p, 9, 1);
     double* phi_i = fout_buf(d_phi, 4);
-    gauss_gradient_internal(d_pbt, d_pbv, p_i, work_grad);
+    gauss_gradient_internal(d_pbt, d_pbv, p_i, 1);
     rhie_chow_flux_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, nc, owner, neigh, patch, npatch, patch_kind,
                                                                d_vbt, d_vbv, d_pbt, d_pbv, rho, fc, fs, cc, vol, h_i,
-                                                               p_i, work_grad, rau_i, phi_i, err);
+                                                               p_i, reinterpret_cast<const double4*>(work_grad), rau_i, phi_i,
+                                                               err);
     faces_out(phi_i, d_phi);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("make_rhie_chow_mass_flux: inverse momentum diagonal must be finite and positive, or invalid face");

@@ -22,9 +22,14 @@ struct PressurePlan {
     uint32_t* nz_row_diag = nullptr;
     uint32_t* nzf_off = nullptr;
     uint32_t* nzf = nullptr;
-    // reduced system only: source nonzero / source row in the full system
-    uint32_t* red_src = nullptr;
-    uint32_t* red_rhs_src = nullptr;
+    // Per internal cell: its row's first nonzero and its row (~0: left out), and
+    // the places in that row of its slots' neighbours, slot-major in ascending
+    // caller face id, and of the diagonal (0xffff: none).
+    uint32_t *row_start = nullptr, *row_of = nullptr;
+    uint16_t *slot_rank = nullptr, *diag_rank = nullptr;
+    bool shared_pairs = false;  // some pair of cells is joined by several faces
+
+    void release();
 };
 
 struct FvMesh {
@@ -76,6 +81,7 @@ struct FvMesh {
     uint8_t *face_slot_o = nullptr, *face_slot_n = nullptr;  // slot of each face on either side
     uint8_t* slot_sorted = nullptr;  // per cell, its slots in ascending caller face id
     int32_t* slot_other = nullptr;
+    double4* cell_rec = nullptr;  // (centre, volume) per cell
     uint32_t* slot_face = nullptr;
     double *slot_w = nullptr, *slot_sx = nullptr, *slot_sy = nullptr, *slot_sz = nullptr;
     double *wls_a0 = nullptr, *wls_a1 = nullptr, *wls_a2 = nullptr, *wls_fac = nullptr, *wls_nd = nullptr;
@@ -136,7 +142,10 @@ struct FvMesh {
     void ensure_slots();
     void ensure_slot_terms();
     void ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt);
-    void gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p_i, double* grad_i);
+    void gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps);
+    void map_rows(PressurePlan& plan, uint32_t ref);
+    uint64_t touched_lines(const std::vector<uint32_t>& at, const std::vector<uint32_t>& cell_place,
+                           const std::vector<uint32_t>& face_place) const;
     void check_err(const char* what);
     void release();
 };
