@@ -375,12 +375,46 @@ __global__ __launch_bounds__(kBlock) void pack_cells_kernel(uint32_t nc, const u
     rec[to ? to[c] : c] = make_double4(v[c], v[size_t(nc) + c], v[2 * size_t(nc) + c], w[c]);
 }
 
+// The momentum predictor's fields: (U, mu) and (body - grad p, 0) a cell.
+// Viscosity must be finite and non-negative; flags[0] = 1 when any is positive
+// (diffusion active).
+__global__ __launch_bounds__(kBlock) void pack_momentum_kernel(
+    uint32_t nc, const uint32_t* __restrict__ to, const double* __restrict__ U, const double* __restrict__ mu,
+    const double* __restrict__ gradp, const double* __restrict__ body, double4* __restrict__ rec,
+    double4* __restrict__ source, int* __restrict__ flags, int* __restrict__ err) {
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= nc) return;
+    const size_t n1 = nc;
+    const uint32_t i = to ? to[c] : c;
+    const double m = mu[c];
+    if (!(m >= 0.0) || !isfinite(m)) err[0] = 40;
+    if (m > 0.0) flags[0] = 1;
+    double s[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s[k] = (body ? body[k * n1 + c] : 0.0) - gradp[k * n1 + c];
+    rec[i] = make_double4(U[c], U[n1 + c], U[2 * n1 + c], m);
+    source[i] = make_double4(s[0], s[1], s[2], 0.0);
+}
+
+// Records (x, y, z, w) a cell out to the caller's order: v 3 x nc, w nc.
+__global__ __launch_bounds__(kBlock) void unpack_cells_kernel(uint32_t nc, const uint32_t* __restrict__ from,
+                                                             const double4* __restrict__ rec,
+                                                             double* __restrict__ v, double* __restrict__ w) {
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= nc) return;
+    const double4 r = rec[from ? from[c] : c];
+    v[c] = r.x;
+    v[size_t(nc) + c] = r.y;
+    v[2 * size_t(nc) + c] = r.z;
+    w[c] = r.w;
+}
+
 // Where the rows of an assembled matrix go: internal cell c fills the entries
 // from start[c] (~0: the row is left out) and right-hand side entry row[c];
 // rank[k * nc + c] is the entry, counted from the row's start, of the cell's
 // k-th slot in ascending caller face id (kNoEntry: boundary face or column
-// left out), diag[c] that of the diagonal. shared: some pair of cells is
-// joined by several faces, whose entries coincide.
+// left out; equal for faces that join one pair, of which there are some when
+// shared), diag[c] that of the diagonal.
 constexpr uint16_t kNoEntry = 0xffffu;
 struct RowMap {
     const uint32_t *start, *row;
@@ -426,6 +460,7 @@ struct Near {
 // Hexahedra (6 slots) take 36 KB and polyhedra up to kRowSlots 48 KB, so three
 // or more workgroups, what the registers allow, share a CU's 160 KB.
 constexpr uint32_t kRowSlots = 12;
+constexpr uint32_t kMomNear = 2;  // records a momentum row stages: cell, fields
 inline size_t row_lds(uint32_t D, uint32_t nrec) {
     return size_t(kBlock) * 8 * (D + std::max(4 * nrec, D + 1));
 }
@@ -530,26 +565,19 @@ __global__ __launch_bounds__(kBlock) void pressure_row_kernel(
     double* row = kLds ? lds + size_t(D) * kBlock + threadIdx.x * stride : vals + size_t(start);
     double d = 0.0;
     uint32_t len = 0;
+    if (rm.shared && start != 0xffffffffu) {
+        for (uint32_t k = 0; k < deg; ++k) {
+            const uint16_t r = rm.rank[size_t(k) * nc + c];
+            if (r != kNoEntry) row[r] = 0.0;
+        }
+    }
     for (uint32_t k = 0; k < deg; ++k) {
         const double cf = cbuf[slot_sorted[size_t(k) * nc + c] * cs];
         d += cf;
         const uint16_t r = rm.rank[size_t(k) * nc + c];
         if (r == kNoEntry) continue;
         len = max(len, uint32_t(r) + 1u);
-        if (!rm.shared) row[r] = 0.0 - cf;
-    }
-    if (rm.shared) {
-        // Entries of faces that join one pair: summed at the first of them.
-        for (uint32_t k = 0; k < deg; ++k) {
-            const uint16_t r = rm.rank[size_t(k) * nc + c];
-            bool fresh = r != kNoEntry;
-            for (uint32_t j = 0; j < k && fresh; ++j) fresh = rm.rank[size_t(j) * nc + c] != r;
-            if (!fresh) continue;
-            double v = 0.0;
-            for (uint32_t j = k; j < deg; ++j)
-                if (rm.rank[size_t(j) * nc + c] == r) v -= cbuf[slot_sorted[size_t(j) * nc + c] * cs];
-            row[r] = v;
-        }
+        row[r] = (rm.shared ? row[r] : 0.0) - cf;
     }
     double b = -cont;
     if (fixed) {
@@ -919,8 +947,14 @@ __global__ __launch_bounds__(kBlock) void wls_build_kernel(uint32_t nc, const ui
 // boundary-aware Green-Gauss gradient (compute_scalar_gradient_with_boundary),
 // replaced by the cached WLS fit where it is certified. Field k's boundary
 // value at patch p is bcv[p * bstride + k]; bct: 0 zero-gradient, 1 fixed
-// value, 2 fixed gradient. gate (momentum path): skip the whole pass unless
-// diffusion is active and a face is non-orthogonal.
+// value, 2 fixed gradient. K = 1: one field, its gradient as three arrays; the
+// Green-Gauss pass comes first for every cell, for the errors it raises on
+// fixed gradients. K = 3: velocity records (u, v, w, .) and gradients as three
+// records a cell; boundary types are 0 and 1, for which finite samples make a
+// finite Green-Gauss sum, so only cells whose fit is refused take that pass and
+// the others read neither area vectors nor weights: bound by the 36 bytes of
+// fit a slot (80^3 cells: 72 us; 136 with both passes and gathers from memory). gate: skip the whole pass unless
+// diffusion is active.
 template <int K>
 __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
     uint32_t nc, const uint32_t* __restrict__ coff, Slots sl, const uint32_t* __restrict__ patch, uint32_t npatch,
@@ -928,18 +962,46 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
     const double* __restrict__ vol, int dim, double limit, WlsCache wc, const double* __restrict__ field,
     double* __restrict__ grad, uint8_t* __restrict__ fallback, const int* __restrict__ gate, int* __restrict__ err) {
 #pragma clang fp contract(off)
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= nc) return;
-    if (gate && !(gate[0] && gate[1])) return;
-    const size_t n1 = nc, n3 = 3 * size_t(nc);
-    const uint32_t deg = coff[c + 1] - coff[c];
-    const D3 centre = cc.get(c);
-    const double V = vol[c];
+    static_assert(K == 1 || K == 3);
+    __shared__ double2 near_lds[K == 3 ? 2 * kBlock : 1];
+    if (gate && !gate[0]) return;
+    const uint32_t first = xcd_block() * kBlock, c = first + threadIdx.x;
+    const Near near{near_lds, first};
+    const double4* rec = reinterpret_cast<const double4*>(field);
     double value[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) value[k] = field[k * n1 + c];
+    if constexpr (K == 3) {
+        if (c < nc) {
+            const double4 r = rec[c];
+            near.put(0, r);
+            value[0] = r.x;
+            value[1] = r.y;
+            value[2] = r.z;
+        }
+        __syncthreads();
+    }
+    if (c >= nc) return;
+    if constexpr (K == 1) value[0] = field[c];
+    auto sample = [&](uint32_t i, double* v) {
+        if constexpr (K == 3) {
+            const double4 r = near.has(i) ? near.get(0, i) : rec[i];
+            v[0] = r.x;
+            v[1] = r.y;
+            v[2] = r.z;
+        } else {
+            v[0] = field[i];
+        }
+    };
+    const size_t n1 = nc;
+    const uint32_t deg = coff[c + 1] - coff[c];
+    const double V = vol[c];
+    if (K == 3 && (!(V > 0.0) || !isfinite(V))) {
+        err[0] = 33;
+        return;
+    }
+    D3 g[K];
     // Green-Gauss with boundary values (compute_scalar_gradient_with_boundary).
-    {
+    auto green_gauss = [&]() {
+        const D3 centre = cc.get(c);
         D3 sum[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) sum[k] = d3(0.0, 0.0, 0.0);
@@ -951,8 +1013,10 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
             double fv[K];
             if (o >= 0) {
                 const double w = sl.w[idx];
+                double other[K];
+                sample(uint32_t(o), other);
 #pragma unroll
-                for (int k = 0; k < K; ++k) fv[k] = w * value[k] + (1.0 - w) * field[k * n1 + uint32_t(o)];
+                for (int k = 0; k < K; ++k) fv[k] = w * value[k] + (1.0 - w) * other[k];
             } else {
                 const uint32_t f = sl.face[idx];
                 const uint32_t pp = patch[f];
@@ -960,7 +1024,7 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
                 double dn = 0.0;
                 if (t == 2 && !boundary_normal_distance(fs.get(f), fc.get(f), centre, V, dn)) {
                     err[0] = 31;
-                    return;
+                    return false;
                 }
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
@@ -973,35 +1037,36 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
             for (int k = 0; k < K; ++k) {
                 if (!isfinite(fv[k])) {
                     err[0] = 32;
-                    return;
+                    return false;
                 }
                 sum[k] = add3(sum[k], mul3(Sf, fv[k]));
             }
         }
         if (!(V > 0.0) || !isfinite(V)) {
             err[0] = 33;
-            return;
+            return false;
         }
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            grad[k * n3 + c] = sum[k].x / V;
-            grad[k * n3 + n1 + c] = sum[k].y / V;
-            grad[k * n3 + 2 * n1 + c] = sum[k].z / V;
-        }
-    }
+        for (int k = 0; k < K; ++k) g[k] = d3(sum[k].x / V, sum[k].y / V, sum[k].z / V);
+        return true;
+    };
+    if (K == 1 && !green_gauss()) return;
     // The cached WLS fit: rhs_i = fac_i (value_i - value); proj_j = sum_i
     // a_ij rhs_i (sample order); g += V e_j proj_j / sigma_j^2 (descending).
     const uint32_t meta = wc.meta[c];
     const double cond = wc.cond[c];
     const bool certified = (meta & 1u) && (meta & 2u) && isfinite(cond) && cond <= limit;
     bool any_fallback = !certified;
+    bool use[K];
+    D3 fit[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) use[k] = false;
     if (certified) {
         const int o0 = int((meta >> 2) & 3u), o1 = int((meta >> 4) & 3u), o2 = int((meta >> 6) & 3u);
-        bool ok[K];
         double proj[K][3];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            ok[k] = isfinite(value[k]);
+            use[k] = isfinite(value[k]);
             proj[k][0] = proj[k][1] = proj[k][2] = 0.0;
         }
         for (uint32_t q = 0; q < deg; ++q) {
@@ -1013,22 +1078,23 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
             const double aj0 = o0 == 0 ? a[0] : (o0 == 1 ? a[1] : a[2]);
             const double aj1 = o1 == 0 ? a[0] : (o1 == 1 ? a[1] : a[2]);
             const double aj2 = o2 == 0 ? a[0] : (o2 == 1 ? a[1] : a[2]);
-            uint8_t t = 0;
-            uint32_t pp = 0;
-            double nd = 0.0;
-            if (o < 0) {
-                pp = patch[sl.face[idx]];
-                t = pp < npatch ? bct[pp] : 0;
-                nd = wc.nd[idx];
+            double sv[K];
+            if (o >= 0) {
+                sample(uint32_t(o), sv);
+            } else {
+                const uint32_t pp = patch[sl.face[idx]];
+                const uint8_t t = pp < npatch ? bct[pp] : 0;
+                const double nd = wc.nd[idx];
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    if (t == 1) sv[k] = bcv[size_t(pp) * bstride + k];
+                    else sv[k] = value[k] + nd * (t == 2 ? bcv[size_t(pp) * bstride + k] : 0.0);
+                }
             }
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                double sv;
-                if (o >= 0) sv = field[k * n1 + uint32_t(o)];
-                else if (t == 1) sv = bcv[size_t(pp) * bstride + k];
-                else sv = value[k] + nd * (t == 2 ? bcv[size_t(pp) * bstride + k] : 0.0);
-                const double dv = sv - value[k];
-                if (!isfinite(dv)) ok[k] = false;
+                const double dv = sv[k] - value[k];
+                if (!isfinite(dv)) use[k] = false;
                 const double rhs = fac * dv;
                 proj[k][0] += aj0 * rhs;
                 proj[k][1] += aj1 * rhs;
@@ -1038,58 +1104,55 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
         const int ord[3] = {o0, o1, o2};
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            bool use = ok[k];
-            double g[3] = {0.0, 0.0, 0.0};
-            if (use) {
+            double x[3] = {0.0, 0.0, 0.0};
+            if (use[k]) {
                 for (int oi = 0; oi < dim; ++oi) {
                     const int j = ord[oi];
                     const double sj = wc.sig[j * n1 + c];
                     const double coeff = proj[k][oi] / (sj * sj);
 #pragma unroll
-                    for (int r = 0; r < 3; ++r) g[r] += wc.V[(3 * r + j) * n1 + c] * coeff;
+                    for (int r = 0; r < 3; ++r) x[r] += wc.V[(3 * r + j) * n1 + c] * coeff;
                 }
-                use = isfinite(g[0]) && isfinite(g[1]) && isfinite(g[2]);
+                use[k] = isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]);
             }
-            if (use) {
-                grad[k * n3 + c] = g[0];
-                grad[k * n3 + n1 + c] = g[1];
-                grad[k * n3 + 2 * n1 + c] = g[2];
-            } else {
-                any_fallback = true;
-            }
+            fit[k] = d3(x[0], x[1], x[2]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) any_fallback |= !use[k];
+    if (K == 3 && any_fallback && !green_gauss()) return;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const D3 r = use[k] ? fit[k] : g[k];
+        if constexpr (K == 3) {
+            reinterpret_cast<double4*>(grad)[3 * size_t(c) + k] = make_double4(r.x, r.y, r.z, 0.0);
+        } else {
+            grad[c] = r.x;
+            grad[n1 + c] = r.y;
+            grad[2 * n1 + c] = r.z;
         }
     }
     if (fallback) fallback[c] = any_fallback ? 1 : 0;
 }
 
-// Cell viscosity must be finite and non-negative; flags[0] = 1 when any is
-// positive (diffusion active).
-__global__ __launch_bounds__(kBlock) void viscosity_check_kernel(uint32_t nc, const double* __restrict__ mu,
-                                                                int* __restrict__ flags, int* __restrict__ err) {
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= nc) return;
-    const double m = mu[c];
-    if (!(m >= 0.0) || !isfinite(m)) err[0] = 40;
-    if (m > 0.0) flags[0] = 1;
-}
-
-// needs_nonorthogonal_gradient scan (finite_volume_transport.h:987-1021):
-// flags[1] = 1 when an internal or fixed-value boundary face has a
-// tangential part above 1e-12 |S_f|.
+// needs_nonorthogonal_gradient scan (finite_volume_transport.h:987-1021) of the
+// geometry: an internal or boundary face with a tangential part above 1e-12
+// |S_f| sets flags[its patch] (internal: flags[npatch]), one whose geometry
+// does not define it flags[npatch + 1 + its patch]. Boundary faces count only
+// where the patch's velocity is fixed, which the caller looks up.
 __global__ __launch_bounds__(kBlock) void nonorth_scan_kernel(uint32_t nf, const uint32_t* __restrict__ owner,
                                                              const int32_t* __restrict__ neigh,
                                                              const uint32_t* __restrict__ patch, uint32_t npatch,
-                                                             const uint8_t* __restrict__ kind,
-                                                             const uint8_t* __restrict__ vbt, Soa3 fc, Soa3 fs,
-                                                             Soa3 cc, int* __restrict__ flags, int* __restrict__ err) {
+                                                             const uint8_t* __restrict__ kind, Soa3 fc, Soa3 fs,
+                                                             Soa3 cc, int* __restrict__ flags) {
 #pragma clang fp contract(off)
     const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
     if (f >= nf) return;
     const int32_t nr = neigh[f];
+    uint32_t pp = npatch;
     if (nr < 0) {
-        const uint32_t pp = patch[f];
-        if (pp < npatch && kind[pp] == 1) return;
-        if (!(pp < npatch && vbt[pp] == 1)) return;
+        pp = patch[f];
+        if (pp >= npatch || kind[pp] == 1) return;
     }
     const uint32_t o = owner[f];
     const D3 sf = fs.get(f);
@@ -1098,244 +1161,190 @@ __global__ __launch_bounds__(kBlock) void nonorth_scan_kernel(uint32_t nf, const
     const double sd = dot3(sf, d);
     const double d2 = dot3(d, d);
     if (!(area > 0.0) || !(sd > 0.0) || !(d2 > 0.0) || !isfinite(area) || !isfinite(sd) || !isfinite(d2)) {
-        err[0] = 41;
+        flags[npatch + 1 + pp] = 1;
         return;
     }
     const double alpha = area * area / sd;
     const D3 tangential = sub3(sf, mul3(d, alpha));
-    if (mag3(tangential) > 1e-12 * area) flags[1] = 1;
+    if (mag3(tangential) > 1e-12 * area) flags[pp] = 1;
 }
 
-// Per-slot momentum terms (slot-major): the face's diagonal coefficient for
-// this cell, its signed flux, its signed tangential fluxes of the three
-// components.
-struct MomSlots {
-    double *diag, *div, *d0, *d1, *d2;
-};
-
-// Per face: the upwind/diffusion coefficients the face adds to the owner's
-// diagonal (aon) and to the neighbour's diagonal, or for a fixed-value
-// boundary face the coefficient of the boundary value (ano); with needs, the
-// tangential diffusion flux of each velocity component (nof, 3 x nf) from
-// the components' WLS gradients ugrad (3 components x 3 x nc).
-__global__ __launch_bounds__(kBlock) void momentum_face_kernel(
-    uint32_t nf, uint32_t nc, const uint32_t* __restrict__ owner, const int32_t* __restrict__ neigh,
-    const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ kind,
-    const uint8_t* __restrict__ vbt, Soa3 fc, Soa3 fs, Soa3 cc, const double* __restrict__ vol,
-    const double* __restrict__ mu, const double* __restrict__ phi, const double* __restrict__ ugrad, int bounded,
-    const int* __restrict__ flags, const uint8_t* __restrict__ slot_o, const uint8_t* __restrict__ slot_n,
-    double* __restrict__ aon, double* __restrict__ ano, MomSlots ms, int* __restrict__ err) {
+// One momentum row per thread (internal cell c), its faces in ascending caller
+// face id (the reference's face loop order): the upwind/diffusion coefficient
+// of each face on the diagonal and on the row's entry, flux divergence,
+// tangential diffusion fluxes (needs) and boundary sources; then the
+// bounded-convection correction, sources and the equation relaxation
+// (relax: alpha < 1). As in the pressure rows every face is evaluated from both
+// of its cells: conductances and interpolation weights come out the same to the
+// last bit and fluxes negated, as long as the one quantity that is not
+// symmetric, the weight along the line from the owner, is taken from the
+// owner's side. out: (rhs, relaxed diagonal) a cell. On 80^3 jittered cells,
+// randomly numbered: 155 us; 162 with the gradients staged as well (LDS then
+// leaves two workgroups a CU instead of three), 162 with the face's data read
+// one slot ahead; 368 as a pass over faces that scattered five terms to the
+// cells' slots, one over cells and one over nonzeros.
+__global__ __launch_bounds__(kBlock) void momentum_row_kernel(
+    uint32_t nc, uint32_t D, const uint32_t* __restrict__ coff, const uint8_t* __restrict__ slot_sorted, Slots sl,
+    const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ vbt,
+    const double* __restrict__ vbv, Soa3 fc, const double4* __restrict__ cell, const double4* __restrict__ fields,
+    const double4* __restrict__ source, const double4* __restrict__ ugrad, const double* __restrict__ phi,
+    int bounded, int nonorthogonal, const int* __restrict__ flags, int relax, double alpha_u, RowMap rm,
+    double* __restrict__ vals, double4* __restrict__ out, int* __restrict__ err) {
 #pragma clang fp contract(off)
-    const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nf) return;
-    const bool needs = flags[0] && flags[1];
-    const size_t n1 = nc, n3 = 3 * size_t(nc);
-    const uint32_t o = owner[f];
-    const double F = phi[f];
-    if (!isfinite(F)) err[0] = 42;
-    double t_on = 0.0, t_no = 0.0;
-    double flux[3] = {0.0, 0.0, 0.0};
-    const D3 Sf = fs.get(f), Cf = fc.get(f), Co = cc.get(o);
-    if (neigh[f] >= 0) {
-        const uint32_t n = uint32_t(neigh[f]);
-        const D3 Cn = cc.get(n);
-        const double distance = mag3(sub3(Cn, Co));
-        const double area = mag3(Sf);
-        if (!(distance > 0.0) || !(area > 0.0)) err[0] = 43;
-        const double d_owner = fabs(dot3(sub3(Cf, Co), Sf)) / area;
-        const double d_neigh = fabs(dot3(sub3(Cn, Cf), Sf)) / area;
-        if (!(d_owner > 0.0) || !(d_neigh > 0.0) || !isfinite(d_owner) || !isfinite(d_neigh)) err[0] = 44;
-        const double go = mu[o], gn = mu[n];
-        double D = 0.0;
-        if (go > 0.0 && gn > 0.0) D = area / (d_owner / go + d_neigh / gn);
-        t_on = D + max0(F);
-        t_no = D + max0(-F);
-        if (needs) {
-            const D3 d = sub3(Cn, Co);
-            const double sd = dot3(Sf, d);
-            const double alpha = area * area / sd;
-            const D3 tangential = sub3(Sf, mul3(d, alpha));
-            if (mag3(tangential) > 1e-12 * area) {
-                const double area_projection = fabs(dot3(Sf, d)) / area;
-                if (!(area_projection > 0.0)) err[0] = 45;
-                double conductance = 0.0;
-                if (go > 0.0 && gn > 0.0) conductance = area / (d_owner / go + d_neigh / gn);
-                const double gamma_face = conductance / alpha;
-                const D3 line = sub3(Cn, Co);
-                const double d2_line = mag2_3(line);
-                if (!(d2_line > 0.0) || !isfinite(d2_line)) err[0] = 46;
-                const double w = 1.0 - clamp01(dot3(sub3(Cf, Co), line) / d2_line);
+    extern __shared__ double2 row_shared[];
+    const uint32_t first = xcd_block() * kBlock;
+    const bool live = first + threadIdx.x < nc;
+    const uint32_t c = live ? first + threadIdx.x : nc - 1;  // the last block's spare threads only keep step
+    const bool needs = nonorthogonal && flags[0];
+    const Near near{row_shared, first};
+    const uint32_t stride = D + 1;
+    double* rows = reinterpret_cast<double*>(row_shared + kMomNear * 2 * kBlock);
+    double* row = rows + threadIdx.x * stride;
+    const uint32_t deg = live ? coff[c + 1] - coff[c] : 0;
+    const double4 C = cell[c], A = fields[c];
+    double4 G[3];
+    near.put(0, C);
+    near.put(1, A);
+    if (needs) {
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const double* g = ugrad + k * n3;
-                    const D3 go3 = d3(g[o], g[n1 + o], g[2 * n1 + o]);
-                    const D3 gn3 = d3(g[n], g[n1 + n], g[2 * n1 + n]);
-                    const D3 gf = add3(mul3(go3, w), mul3(gn3, 1.0 - w));
-                    flux[k] = gamma_face * dot3(gf, tangential);
-                    if (!isfinite(flux[k])) err[0] = 47;
+        for (int k = 0; k < 3; ++k) {
+            G[k] = ugrad[3 * size_t(c) + k];
+        }
+    }
+    __syncthreads();
+    const D3 Cc = d3(C.x, C.y, C.z);
+    if (rm.shared)
+        for (uint32_t k = 0; k < stride; ++k) row[k] = 0.0;
+    double diag = 0.0, div = 0.0;
+    double rhs[3] = {0.0, 0.0, 0.0}, def[3] = {0.0, 0.0, 0.0};
+    uint32_t len = 0;
+    // A slot's place, then its ids, then the face's and the neighbour's data
+    // depend on each other: the first two are read ahead.
+    auto place = [&](uint32_t k) {
+        return k < deg ? size_t(slot_sorted[size_t(k) * nc + c]) * nc + c : size_t(c);
+    };
+    size_t idx = place(0), idx1 = place(1);
+    int32_t o1 = sl.other[idx];
+    uint32_t f1 = sl.face[idx];
+    for (uint32_t k = 0; k < deg; ++k) {
+        const size_t at = idx;
+        const int32_t o = o1;
+        const uint32_t fr = f1, f = fr & ~kFaceReversed;
+        const bool reversed = fr != f;
+        const double Fo = phi[f];
+        const D3 Sf = sl.s.get(at), Cf = fc.get(f);
+        idx = idx1;
+        o1 = sl.other[idx];
+        f1 = sl.face[idx];
+        idx1 = place(k + 2);
+        if (!isfinite(Fo)) err[0] = 42;
+        if (o == -2) continue;
+        const double F = reversed ? -Fo : Fo;
+        const double area = mag3(Sf);
+        if (o >= 0) {
+            const uint32_t n = uint32_t(o);
+            const bool in = near.has(n);
+            const double4 Nn = in ? near.get(0, n) : cell[n];
+            const double gn = in ? near.get(1, n).w : fields[n].w, go = A.w;
+            const D3 Cn = d3(Nn.x, Nn.y, Nn.z);
+            const D3 line = sub3(Cn, Cc);
+            const double distance = mag3(line);
+            if (!(distance > 0.0) || !(area > 0.0)) err[0] = 43;
+            const double d_own = fabs(dot3(sub3(Cf, Cc), Sf)) / area;
+            const double d_oth = fabs(dot3(sub3(Cn, Cf), Sf)) / area;
+            if (!(d_own > 0.0) || !(d_oth > 0.0) || !isfinite(d_own) || !isfinite(d_oth)) err[0] = 44;
+            double Dc = 0.0;
+            if (go > 0.0 && gn > 0.0) Dc = area / (d_own / go + d_oth / gn);
+            if (needs) {
+                const double sd = dot3(Sf, line);
+                const double alpha = area * area / sd;
+                const D3 tangential = sub3(Sf, mul3(line, alpha));
+                if (mag3(tangential) > 1e-12 * area) {
+                    const double area_projection = fabs(sd) / area;
+                    if (!(area_projection > 0.0)) err[0] = 45;
+                    const double gamma_face = Dc / alpha;
+                    const double d2_line = mag2_3(line);
+                    if (!(d2_line > 0.0) || !isfinite(d2_line)) err[0] = 46;
+                    const double along =
+                        reversed ? dot3(sub3(Cf, Cn), sub3(Cc, Cn)) : dot3(sub3(Cf, Cc), line);
+                    const double w = 1.0 - clamp01(along / d2_line);
+                    const double wc = reversed ? 1.0 - w : w, wn = reversed ? w : 1.0 - w;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        const double4 N = ugrad[3 * size_t(n) + q];
+                        const D3 gf = add3(mul3(d3(G[q].x, G[q].y, G[q].z), wc), mul3(d3(N.x, N.y, N.z), wn));
+                        const double flux = gamma_face * dot3(gf, tangential);
+                        if (!isfinite(flux)) err[0] = 47;
+                        def[q] += flux;
+                    }
                 }
             }
-        }
-    } else {
-        const uint32_t pp = patch[f];
-        if (!(pp < npatch && kind[pp] == 1)) {
+            diag += Dc + max0(F);
+            div += F;
+            const uint16_t r = rm.rank[size_t(k) * nc + c];
+            len = max(len, uint32_t(r) + 1u);
+            row[r] = (rm.shared ? row[r] : 0.0) - (Dc + max0(-F));
+        } else {
+            const uint32_t pp = patch[f];
             const bool fixed = pp < npatch && vbt[pp] == 1;
-            const double area = mag3(Sf);
             double distance = 0.0;
-            if (!boundary_normal_distance(Sf, Cf, Co, vol[o], distance) || !(distance > 0.0) || !(area > 0.0))
+            if (!boundary_normal_distance(Sf, Cf, Cc, C.w, distance) || !(distance > 0.0) || !(area > 0.0))
                 err[0] = 48;
             if (fixed) {
-                const double D = mu[o] * area / distance;
-                t_on = D + max0(F);
-                t_no = D + max0(-F);
+                const double Dc = A.w * area / distance;
                 if (needs) {
-                    const D3 d = sub3(Cf, Co);
+                    const D3 d = sub3(Cf, Cc);
                     const double sd = dot3(Sf, d);
                     const double alpha = area * area / sd;
                     const D3 tangential = sub3(Sf, mul3(d, alpha));
                     if (mag3(tangential) > 1e-12 * area) {
-                        const double gamma_face = mu[o];
 #pragma unroll
-                        for (int k = 0; k < 3; ++k) {
-                            const double* g = ugrad + k * n3;
-                            const D3 gf = d3(g[o], g[n1 + o], g[2 * n1 + o]);
-                            flux[k] = gamma_face * dot3(gf, tangential);
-                            if (!isfinite(flux[k])) err[0] = 47;
+                        for (int q = 0; q < 3; ++q) {
+                            const double flux = A.w * dot3(d3(G[q].x, G[q].y, G[q].z), tangential);
+                            if (!isfinite(flux)) err[0] = 47;
+                            def[q] += flux;
                         }
                     }
                 }
+                diag += Dc + max0(F);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) rhs[q] += (Dc + max0(-F)) * vbv[3 * size_t(pp) + q];
             } else {
-                t_on = bounded ? F : max0(F);
-            }
-        }
-    }
-    aon[f] = t_on;
-    ano[f] = t_no;
-    // This face's terms in the owner's slot and (internal faces) the
-    // neighbour's slot, signed for that side: x - t is x + (-t) exactly.
-    const size_t io = size_t(slot_o[f]) * nc + o;
-    ms.diag[io] = t_on;
-    ms.div[io] = F;
-    ms.d0[io] = flux[0];
-    ms.d1[io] = flux[1];
-    ms.d2[io] = flux[2];
-    if (neigh[f] >= 0) {
-        const size_t in = size_t(slot_n[f]) * nc + uint32_t(neigh[f]);
-        ms.diag[in] = t_no;
-        ms.div[in] = -F;
-        ms.d0[in] = -flux[0];
-        ms.d1[in] = -flux[1];
-        ms.d2[in] = -flux[2];
-    }
-}
-
-// Per cell, faces in ascending caller face id (the reference's face loop
-// order): diagonal, flux divergence, deferred non-orthogonal terms and
-// boundary sources, read from the cell's slots; then the bounded-convection
-// correction, sources and the equation relaxation (alpha < 1). diag: the
-// relaxed diagonal (shared by the three components); rhs: 3 x nc.
-__global__ __launch_bounds__(kBlock) void momentum_cell_kernel(
-    uint32_t nc, const uint32_t* __restrict__ coff, const uint8_t* __restrict__ slot_sorted, Slots sl,
-    MomSlots ms, const uint32_t* __restrict__ patch, uint32_t npatch, const uint8_t* __restrict__ vbt,
-    const double* __restrict__ vbv, const double* __restrict__ vol, const double* __restrict__ phi,
-    const double* __restrict__ ano, const double* __restrict__ gradp, const double* __restrict__ body,
-    const double* __restrict__ U, int bounded, const int* __restrict__ flags, int relax, double alpha,
-    double* __restrict__ diag_out, double* __restrict__ rhs_out, int* __restrict__ err) {
-#pragma clang fp contract(off)
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= nc) return;
-    const bool needs = flags[0] && flags[1];
-    const size_t n1 = nc;
-    const uint32_t deg = coff[c + 1] - coff[c];
-    double diag = 0.0, div = 0.0;
-    double rhs[3] = {0.0, 0.0, 0.0}, def[3] = {0.0, 0.0, 0.0};
-    for (uint32_t k = 0; k < deg; ++k) {
-        const size_t idx = size_t(slot_sorted[size_t(k) * nc + c]) * nc + c;
-        const int32_t o = sl.other[idx];
-        if (o == -2) continue;
-        if (o >= 0) {
-            diag += ms.diag[idx];
-            div += ms.div[idx];
-            if (needs) {
-                def[0] += ms.d0[idx];
-                def[1] += ms.d1[idx];
-                def[2] += ms.d2[idx];
-            }
-        } else {
-            const uint32_t f = sl.face[idx];
-            const uint32_t pp = patch[f];
-            const double F = phi[f];
-            if (needs) {
-                def[0] += ms.d0[idx];
-                def[1] += ms.d1[idx];
-                def[2] += ms.d2[idx];
-            }
-            diag += ms.diag[idx];
-            if (pp < npatch && vbt[pp] == 1) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) rhs[q] += ano[f] * vbv[3 * size_t(pp) + q];
-            } else if (!bounded && F < 0.0) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) def[q] -= F * U[q * n1 + c];
+                diag += bounded ? F : max0(F);
+                if (!bounded && F < 0.0) {
+                    def[0] -= F * A.x;
+                    def[1] -= F * A.y;
+                    def[2] -= F * A.z;
+                }
             }
             div += F;
         }
     }
     if (bounded) diag -= div;
-    const double V = vol[c];
+    const double V = C.w;
     diag -= 0.0 * V;
-    if (!(diag > 0.0) || !isfinite(diag)) err[0] = 49;
+    if (live && (!(diag > 0.0) || !isfinite(diag))) err[0] = 49;
+    const double4 src = source[c];
+    rhs[0] += src.x * V;
+    rhs[1] += src.y * V;
+    rhs[2] += src.z * V;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const double b = body ? body[k * n1 + c] : 0.0;
-        const double source = b - gradp[k * n1 + c];
-        rhs[k] += source * V;
-        rhs[k] += def[k];
-    }
+    for (int q = 0; q < 3; ++q) rhs[q] += def[q];
     if (relax) {
-        const double added = diag * (1.0 / alpha - 1.0);
+        const double added = diag * (1.0 / alpha_u - 1.0);
         diag += added;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) rhs[k] += added * U[k * n1 + c];
+        rhs[0] += added * A.x;
+        rhs[1] += added * A.y;
+        rhs[2] += added * A.z;
     }
-    diag_out[c] = diag;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) rhs_out[k * n1 + c] = rhs[k];
-}
-
-// CSR values of the momentum matrix (caller numbering), one thread per
-// caller row r (internal row rowmap[r]): the diagonal from diag; off-diagonal
-// (r, j) = 0 - the coefficient of each face joining r and j in ascending
-// caller face order (ano when r owns the face, else aon). nzf: internal face
-// ids; owner, diag, aon, ano: internal numbering. (Threads over internal rows
-// were measured slower on a randomly numbered mesh: the caller's CSR
-// metadata and the output then scatter instead.)
-__global__ __launch_bounds__(kBlock) void momentum_values_kernel(uint32_t n, const uint32_t* __restrict__ rowp,
-                                                                const uint32_t* __restrict__ cols,
-                                                                const uint32_t* __restrict__ rowmap,
-                                                                const uint32_t* __restrict__ nzf_off,
-                                                                const uint32_t* __restrict__ nzf,
-                                                                const uint32_t* __restrict__ owner,
-                                                                const double* __restrict__ diag,
-                                                                const double* __restrict__ aon,
-                                                                const double* __restrict__ ano,
-                                                                double* __restrict__ vals) {
-#pragma clang fp contract(off)
-    const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
-    const uint32_t ri = rowmap[r];
-    for (uint32_t k = rowp[r]; k < rowp[r + 1]; ++k) {
-        if (cols[k] == r) {
-            vals[k] = diag[ri];
-            continue;
-        }
-        double v = 0.0;
-        for (uint32_t q = nzf_off[k]; q < nzf_off[k + 1]; ++q) {
-            const uint32_t f = nzf[q];
-            v -= owner[f] == ri ? ano[f] : aon[f];
-        }
-        vals[k] = v;
+    if (live) {
+        const uint32_t r = rm.diag[c];
+        row[r] = diag;
+        len = max(len, r + 1u);
+        out[c] = make_double4(rhs[0], rhs[1], rhs[2], diag);
     }
+    wave_fence();
+    store_rows(rows + (threadIdx.x & ~63u) * stride, stride, rm.start[c], live ? len : 0, vals);
 }
 
 // rAU = 1 / diag and HbyA_k = rAU (rhs_k + grad_p_k V - sum_{j != r} a_rj U_k[j])
@@ -1581,7 +1590,7 @@ FvMesh::~FvMesh() { release(); }
 void FvMesh::release() {
     for (double** p : {&px, &py, &pz, &fcx, &fcy, &fcz, &fsx, &fsy, &fsz, &ccx, &ccy, &ccz, &vol, &vol_caller,
                        &work_coeff, &work_bsrc, &work_diag, &work_rhs, &work_grad, &work_phi,
-                       &mom_aon, &mom_ano, &mom_ugrad, &bc_f64, &mom_sdiag, &mom_sdiv, &mom_sd0, &mom_sd1, &mom_sd2, &slot_w, &slot_sx, &slot_sy, &slot_sz,
+                       &mom_ugrad, &bc_f64, &slot_coeff, &slot_w, &slot_sx, &slot_sy, &slot_sz,
                        &wls_a0, &wls_a1, &wls_a2, &wls_fac, &wls_nd, &wls_sig, &wls_V, &wls_cond})
         dfree(*p);
     for (uint32_t** p : {&foff, &fvtx, &owner, &coff, &cfaces, &cfaces_sorted, &patch, &cell_new, &cell_old,
@@ -1592,8 +1601,6 @@ void FvMesh::release() {
     dfree(scratch_u8);
     dfree(slot_other);
     dfree(cell_rec);
-    dfree(face_slot_o);
-    dfree(face_slot_n);
     dfree(slot_sorted);
     dfree(slot_face);
     dfree(wls_meta);
@@ -1891,28 +1898,21 @@ void FvMesh::ensure_slots() {
     slot_sx = dalloc<double>(m);
     slot_sy = dalloc<double>(m);
     slot_sz = dalloc<double>(m);
-    // Slot of each face on its owner's and neighbour's side, and each cell's
-    // slots in ascending caller face id (the order of the reference's face
-    // loop accumulations).
+    // Each cell's slots in ascending caller face id (the order of the
+    // reference's face loop accumulations).
     {
-        std::vector<uint8_t> so(nf, 0), sn(nf, 0), sorted(m, 0);
+        std::vector<uint8_t> sorted(m, 0);
         std::vector<uint32_t> cold(nc);
         for (uint32_t c = 0; c < nc; ++c) cold[h_cell_new[c]] = c;
         parallel_for(nc, 0, [&](uint64_t i) {
             const uint32_t c = cold[i];
             const uint32_t b = h_coff[c], deg = h_coff[c + 1] - b;
             uint32_t order[256];
-            for (uint32_t q = 0; q < deg && q < 256; ++q) {
-                const uint32_t f = h_cf[b + q];
-                (h_owner[f] == c ? so : sn)[h_face_new[f]] = uint8_t(q);
-                order[q] = q;
-            }
+            for (uint32_t q = 0; q < deg && q < 256; ++q) order[q] = q;
             std::sort(order, order + std::min<uint32_t>(deg, 256),
                       [&](uint32_t x, uint32_t y) { return h_cf[b + x] < h_cf[b + y]; });
             for (uint32_t k = 0; k < deg && k < 256; ++k) sorted[uint64_t(k) * nc + i] = uint8_t(order[k]);
         });
-        face_slot_o = upload(so.data(), nf);
-        face_slot_n = upload(sn.data(), nf);
         slot_sorted = upload(sorted.data(), m);
     }
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
@@ -1921,15 +1921,6 @@ void FvMesh::ensure_slots() {
                                                            patch_kind, fc, fs, cc, vol, cell_rec, slots_of(*this), err);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("cell stencils: degenerate face distances");
-}
-
-// Per-slot terms written by the face kernels (shared by the momentum and the
-// pressure assembly; scratch within one call).
-void FvMesh::ensure_slot_terms() {
-    ensure_slots();
-    if (mom_sdiag) return;
-    const uint64_t m = uint64_t(slot_D) * nc;
-    for (double** p : {&mom_sdiag, &mom_sdiv, &mom_sd0, &mom_sd1, &mom_sd2}) *p = dalloc<double>(m);
 }
 
 // WLS fit cache for one set of boundary types (fixed value or not, per patch).
@@ -2160,10 +2151,10 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
             nc, slot_D, coff, slot_sorted, slots_of(*this), patch, npatch, d_pbt, d_pbv, rho, fc, cell_rec, rec, grad,
             phi_i, nullptr, rm, d_vals, d_rhs, err);
     } else {
-        ensure_slot_terms();
+        if (!slot_coeff) slot_coeff = dalloc<double>(uint64_t(slot_D) * nc);
         pressure_row_kernel<false><<<grid_for(nc), kBlock, 0, stream>>>(
             nc, slot_D, coff, slot_sorted, slots_of(*this), patch, npatch, d_pbt, d_pbv, rho, fc, cell_rec, rec, grad,
-            phi_i, mom_sdiag, rm, d_vals, d_rhs, err);
+            phi_i, slot_coeff, rm, d_vals, d_rhs, err);
     }
     HIP_OK(hipStreamSynchronize(stream));
     check_err("pressure_face_orthogonal_coefficient: invalid face geometry or orientation");
@@ -2200,15 +2191,24 @@ const PressurePlan& FvMesh::diffusion_assemble_device(double gamma, const double
 // ============================================================ momentum side
 
 void FvMesh::ensure_momentum_work() {
-    if (mom_aon) return;
-    ensure_slot_terms();
-    mom_aon = dalloc<double>(nf);
-    mom_ano = dalloc<double>(nf);
-    mom_ugrad = dalloc<double>(9 * uint64_t(nc));
-    mom_flags = dalloc<int>(4);
+    if (mom_flags) return;
+    ensure_slots();
+    mom_ugrad = dalloc<double>(12 * uint64_t(nc));
     const uint32_t npp = std::max<uint32_t>(npatch, 1);
     bc_u8 = dalloc<uint8_t>(2 * uint64_t(npp));
     bc_f64 = dalloc<double>(4 * uint64_t(npp));
+    // Which patches (last: the internal faces) hold non-orthogonal faces, and
+    // which ones faces that do not say: geometry, so found once.
+    const uint32_t nflag = 2 * (npatch + 1);
+    int* flags = dalloc<int>(std::max<uint32_t>(nflag, 4));
+    h_nonorth.assign(nflag, 0);
+    HIP_OK(hipMemsetAsync(flags, 0, nflag * sizeof(int), stream));
+    nonorth_scan_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, owner, neigh, patch, npatch, patch_kind,
+                                                             Soa3{fcx, fcy, fcz}, Soa3{fsx, fsy, fsz},
+                                                             Soa3{ccx, ccy, ccz}, flags);
+    HIP_OK(hipStreamSynchronize(stream));
+    download(h_nonorth.data(), flags, nflag);
+    mom_flags = flags;
 }
 
 // Boundary data per patch into the persistent device buffers (no allocation
@@ -2277,35 +2277,35 @@ const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const
     const double* d_vbv = bc_f64;
     ensure_wls_cache(h_bc_u8.data(), d_vbt);
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
-    const double* u_i = cin(d_U, 0, 3);
-    const double* gp_i = cin(d_gradp, 1, 3);
-    const double* body_i = d_body ? cin(d_body, 2, 3) : nullptr;
-    const double* mu_i = cin(d_mu, 3, 1);
+    bool nonorthogonal = h_nonorth[npatch], undefined = h_nonorth[2 * npatch + 1];
+    for (uint32_t p = 0; p < npatch; ++p) {
+        if (h_bc_u8[p] != 1) continue;
+        nonorthogonal = nonorthogonal || h_nonorth[p];
+        undefined = undefined || h_nonorth[npatch + 1 + p];
+    }
+    auto records = [&](size_t slot) { return reinterpret_cast<double4*>(scr(slot, 4 * uint64_t(nc))); };
+    double4 *rec = records(0), *source = records(1), *out = records(2);
     const double* phi_i = fin(d_phi, 4);
-    double* rhs_i = cout_buf(d_rhs, 8, 3);
-    double* diag_i = cout_buf(d_diag, 9, 1);
     HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
     HIP_OK(hipMemsetAsync(mom_flags, 0, 4 * sizeof(int), stream));
-    viscosity_check_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, mu_i, mom_flags, err);
-    nonorth_scan_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, owner, neigh, patch, npatch, patch_kind, d_vbt, fc,
-                                                             fs, cc, mom_flags, err);
-    wls_gradient_kernel<3><<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, slots_of(*this), patch, npatch, d_vbt, d_vbv, 3, fc,
-                                                                fs, cc, vol, stencil_dimension(), 1.e8, wls_of(*this), u_i,
-                                                                mom_ugrad, nullptr, mom_flags, err);
-    const MomSlots ms{mom_sdiag, mom_sdiv, mom_sd0, mom_sd1, mom_sd2};
-    momentum_face_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, nc, owner, neigh, patch, npatch, patch_kind, d_vbt,
-                                                              fc, fs, cc, vol, mu_i, phi_i, mom_ugrad,
-                                                              bounded ? 1 : 0, mom_flags, face_slot_o, face_slot_n,
-                                                              mom_aon, mom_ano, ms, err);
-    momentum_cell_kernel<<<grid_for(nc), kBlock, 0, stream>>>(
-        nc, coff, slot_sorted, slots_of(*this), ms, patch, npatch, d_vbt, d_vbv, vol, phi_i, mom_ano, gp_i, body_i,
-        u_i, bounded ? 1 : 0, mom_flags, alpha != 1.0 ? 1 : 0, alpha, diag_i, rhs_i, err);
-    momentum_values_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, plan.rowp, plan.cols, cell_new, plan.nzf_off,
-                                                                plan.nzf, owner, diag_i, mom_aon, mom_ano, d_vals);
-    cells_out(diag_i, d_diag, 1);
-    cells_out(rhs_i, d_rhs, 3);
+    pack_momentum_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, d_U, d_mu,
+                                                              d_gradp, d_body, rec, source, mom_flags, err);
+    if (nonorthogonal)
+        wls_gradient_kernel<3><<<grid_for(nc), kBlock, 0, stream>>>(
+            nc, coff, slots_of(*this), patch, npatch, d_vbt, d_vbv, 3, fc, fs, cc, vol, stencil_dimension(), 1.e8,
+            wls_of(*this), &rec->x, mom_ugrad, nullptr, mom_flags, err);
+    const RowMap rm{plan.row_start, plan.row_of, plan.slot_rank, plan.diag_rank, plan.shared_pairs ? 1 : 0};
+    momentum_row_kernel<<<grid_for(nc), kBlock, size_t(kBlock) * 8 * (4 * kMomNear + slot_D + 1), stream>>>(
+        nc, slot_D, coff, slot_sorted, slots_of(*this), patch, npatch, d_vbt, d_vbv, fc, cell_rec, rec, source,
+        reinterpret_cast<const double4*>(mom_ugrad), phi_i, bounded ? 1 : 0, nonorthogonal ? 1 : 0, mom_flags,
+        alpha != 1.0 ? 1 : 0, alpha, rm, d_vals, out, err);
+    unpack_cells_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, out, d_rhs,
+                                                             d_diag);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("assemble_momentum_component: invalid viscosity, flux or geometry, or non-positive diagonal");
+    if (undefined)
+        throw std::domain_error("assemble_momentum_component: invalid viscosity, flux or geometry, or non-positive "
+                                "diagonal (code 41)");
     return plan;
 }
 

@@ -59,12 +59,13 @@ struct FvMesh {
     // pressure boundary types / values per patch, refreshed by each assembly
     uint8_t* pbc_u8 = nullptr;
     double* pbc_f64 = nullptr;
-    // momentum side: per-face upwind/diffusion coefficients, tangential
-    // fluxes (3 x nf), velocity WLS gradients (3 x 3 x nc), flags
-    double *mom_aon = nullptr, *mom_ano = nullptr, *mom_ugrad = nullptr;
-    // per-slot momentum terms (slot-major): diagonal, signed flux, signed tangential fluxes
-    double *mom_sdiag = nullptr, *mom_sdiv = nullptr, *mom_sd0 = nullptr, *mom_sd1 = nullptr, *mom_sd2 = nullptr;
+    // momentum side: velocity WLS gradients (three records a cell), flags, and
+    // per patch (last: internal faces) whether faces are non-orthogonal, then
+    // whether their geometry leaves that undefined
+    double* mom_ugrad = nullptr;
     int* mom_flags = nullptr;
+    std::vector<int> h_nonorth;
+    double* slot_coeff = nullptr;  // coefficients per slot, where they do not fit LDS
     // per-patch boundary data of the momentum-side calls (persistent)
     uint8_t* bc_u8 = nullptr;
     double* bc_f64 = nullptr;
@@ -78,7 +79,6 @@ struct FvMesh {
     std::vector<uint8_t> h_patch_boundary;  // per patch: owns at least one boundary face
     // slot stencils (slot-major, slot_D slots per cell) and the WLS fit cache
     uint32_t slot_D = 0;
-    uint8_t *face_slot_o = nullptr, *face_slot_n = nullptr;  // slot of each face on either side
     uint8_t* slot_sorted = nullptr;  // per cell, its slots in ascending caller face id
     int32_t* slot_other = nullptr;
     double4* cell_rec = nullptr;  // (centre, volume) per cell
@@ -140,7 +140,6 @@ struct FvMesh {
     double* cout_buf(double* caller, size_t slot, int comps);
     double* fout_buf(double* caller, size_t slot);
     void ensure_slots();
-    void ensure_slot_terms();
     void ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt);
     void gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps);
     void map_rows(PressurePlan& plan, uint32_t ref);

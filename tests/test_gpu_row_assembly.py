@@ -1,5 +1,5 @@
-"""Pressure assembly by rows, one thread a cell, against the oracle bit for bit
-where its bookkeeping branches: pairs of cells joined by one, two or four faces
+"""Pressure and momentum assembly by rows, one thread a cell, against the oracle bit for bit
+where the bookkeeping branches: pairs of cells joined by one, two or four faces
 (every quad whole, halved, or a fan of triangles, in shuffled face order), up to
 24 slots a cell (more than LDS holds the coefficients of), cells short of, at
 and past a workgroup, and the row and column of a reference cell left out at
@@ -12,15 +12,15 @@ import cfdx_dev_amd as cx
 pytestmark = pytest.mark.gpu
 
 
-def split_faces(m, pieces, seed):
-    """m with every quad in `pieces` faces, internal faces first, each group shuffled."""
+def split_faces(m, pieces, seed, inner_only=False):
+    """m with every quad (or the internal ones) in `pieces` faces, internal faces first, each group shuffled."""
     rng = np.random.default_rng(seed)
     fo, fv = m.face_offsets.astype(int), m.face_vertices.astype(int)
     pts = [list(a) for a in (m.px, m.py, m.pz)]
     faces, parent = [], []
     for f in range(m.n_faces):
         v = list(fv[fo[f]:fo[f + 1]])
-        if pieces == 1:
+        if pieces == 1 or (inner_only and m.neighbour[f] < 0):
             parts = [v]
         elif pieces == 2:
             parts = [[v[0], v[1], v[2]], [v[0], v[2], v[3]]]
@@ -95,3 +95,30 @@ def test_empty_and_stepped(oracle):
     same(oracle, cx.generate_mesh("extruded2d", 20, 15, 1), 7, False)
     same(oracle, cx.generate_mesh("channel_step", 24, 12, 4, lx=3.0, jitter=0.05, permute=True, seed=9,
                                   step_height_fraction=1.0 / 3.0, step_length_fraction=0.25), 0, True)
+
+
+@pytest.mark.parametrize("pieces", [1, 2])
+@pytest.mark.parametrize("dims", [(8, 8, 4), (11, 8, 3)])
+@pytest.mark.parametrize("jitter", [0.0, 0.05])  # orthogonal or not: without or with velocity gradients
+@pytest.mark.parametrize("bounded", [True, False])
+def test_momentum_rows(oracle, dims, pieces, jitter, bounded):
+    m = cx.generate_mesh("box", *dims, jitter=jitter, permute=True, seed=6)
+    if pieces > 1:  # wall faces stay whole: ten faces a cell at the most
+        m = cx.generate_mesh("extruded2d", dims[0], dims[1] * dims[2], 1, jitter=jitter, permute=True, seed=6)
+        m = split_faces(m, pieces, 9, inner_only=True)
+    g = oracle.geometry(m)
+    rng = np.random.default_rng(5)
+    nc = m.n_cells
+    U, gp, body = (rng.normal(size=3 * nc) for _ in range(3))
+    mu = np.exp(rng.normal(size=nc)) * (rng.uniform(size=nc) > 0.1)
+    vt = np.zeros(m.n_patches, np.uint8)
+    vt[0] = vt[1] = 1
+    vv = rng.normal(size=3 * m.n_patches)
+    phi = 0.01 * oracle.mass_flux(m, g, vt, vv, 1.0, U)
+    mu += 1.0  # keeps the diagonal positive
+    want = oracle.momentum_assemble(m, g, vt, vv, mu, phi, gp, body, U, bounded, 0.7)
+    got = cx.FvMesh(m).momentum_assemble(vt, vv, mu, phi, gp, body, U, bounded=bounded, alpha=0.7)
+    assert np.array_equal(got[0], want["rowp"]) and np.array_equal(got[1], want["cols"])
+    assert np.array_equal(got[2], want["vals"][0])
+    assert np.array_equal(got[3], want["rhs"].ravel())
+    assert np.array_equal(got[4], want["diag"][0])
