@@ -16,6 +16,7 @@
 #include "device_amg.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <array>
 #include <chrono>
 #include <cmath>
@@ -402,7 +403,14 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
         if (has32_) cns_r32_ = dalloc<float>(lv_[0].n);
     }
     scal_ = dalloc<double>(kScalars);
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_scal_), kScalars * sizeof(double), hipHostMallocDefault));
+    HIP_OK(hipMemset(scal_, 0, kScalars * sizeof(double)));
+    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_scal_), kScalars * sizeof(double), hipHostMallocMapped));
+    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&scal_host_), h_scal_, 0));
+    std::fill_n(h_scal_, kScalars, 0.0);
+    // The last slots but one: the polled tickets.
+    h_done_ = reinterpret_cast<unsigned long long*>(h_scal_ + kScalars - 16);
+    done_ = reinterpret_cast<unsigned long long*>(scal_host_ + kScalars - 16);
+    ticket_ = 0;
     (void)n0;
     HIP_OK(hipStreamSynchronize(stream_));
     phase("coarsest factors, work arrays");
@@ -902,7 +910,7 @@ template <class T>
 void DeviceAmg::remove_mean(T* v, uint32_t n) {
     const uint32_t gs = grid_stride(n);
     sum_partial_kernel<T><<<gs, kBlock, 0, stream_>>>(n, v, aux_part_);
-    reduce_partials_kernel<<<1, 1024, 0, stream_>>>(aux_part_, gs, gs, 1, scal_ + 450);
+    reduce_partials_kernel<<<1, 1024, 0, stream_>>>(aux_part_, gs, gs, scal_ + 450, nullptr);
     subtract_mean_kernel<T><<<grid_for(n), kBlock, 0, stream_>>>(n, v, scal_ + 450, double(n));
 }
 
@@ -912,7 +920,7 @@ void DeviceAmg::project_out(const double* modes, uint32_t count, double* v) {
     for (uint32_t q = 0; q < count; ++q) {
         const double* m = modes + size_t(q) * n;
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, v, m, aux_part_);
-        reduce_partials_kernel<<<1, 1024, 0, stream_>>>(aux_part_, gs, gs, 1, scal_ + 460);
+        reduce_partials_kernel<<<1, 1024, 0, stream_>>>(aux_part_, gs, gs, scal_ + 460, nullptr);
         remove_mode_kernel<<<grid_for(n), kBlock, 0, stream_>>>(n, v, m, scal_ + 460);
     }
 }
@@ -956,15 +964,37 @@ bool DeviceAmg::vcycle32(const float* r, float* z) {
 
 // ------------------------------------------------------------ helpers --
 
-void DeviceAmg::reduce(const double* partials, uint32_t n, uint32_t count, double* out, uint64_t stride) {
-    reduce_partials_kernel<<<1, 1024, 0, stream_>>>(partials, n, uint32_t(stride ? stride : partial_stride_), count,
-                                                    out);
+// out: a slot of base, whose sums the same slots of h_scal_ receive as well
+// (null: they stay on the device).
+void DeviceAmg::reduce(const double* partials, uint32_t n, uint32_t count, double* out, uint64_t stride,
+                       const double* base) {
+    reduce_partials_kernel<<<count, 1024, 0, stream_>>>(partials, n, uint32_t(stride ? stride : partial_stride_), out,
+                                                        base ? scal_host_ + (out - base) : nullptr);
 }
 
-bool DeviceAmg::fetch_scalars(uint32_t count, const double* src) {
-    HIP_OK(hipMemcpyAsync(h_scal_, src ? src : scal_, count * sizeof(double), hipMemcpyDeviceToHost, stream_));
+// Waits for the reduced scalars of slots first..first + count and leaves them at
+// the start of h_scal_.
+bool DeviceAmg::fetch_scalars(uint32_t count, uint32_t first) {
     HIP_OK(hipStreamSynchronize(stream_));
+    if (first) std::copy_n(h_scal_ + first, count, h_scal_);
     return true;
+}
+
+// Waits until the first `count` workgroups of the kernel launched last have
+// signalled ticket_. Polling pinned memory sees them sooner than a stream synchronisation
+// (17 FGMRES steps on 75k rows: 3780 us so, 3890 that way); a launch that takes
+// longer than some milliseconds, or fails, is left to the runtime.
+void DeviceAmg::await(int count) {
+    const volatile unsigned long long* done = h_done_;
+    for (int k = 0; k < count; ++k)
+        for (uint32_t spin = 0; done[k] != ticket_; ++spin) {
+            if (spin > 200000u) {
+                HIP_OK(hipStreamSynchronize(stream_));
+                break;
+            }
+            __builtin_ia32_pause();
+        }
+    std::atomic_thread_fence(std::memory_order_acquire);
 }
 
 static double* need_vec(std::vector<double*>& pool, size_t idx, uint32_t n) {
@@ -979,10 +1009,36 @@ static float* need_vec32(std::vector<float*>& pool, size_t idx, uint32_t n) {
 // -------------------------------------------------------- device apply --
 
 namespace {
-__global__ __launch_bounds__(kBlock) void nonfinite_flag_kernel(uint32_t n, const double* __restrict__ v,
-                                                                int* __restrict__ flag) {
+// An application's residual into the solve order. A non-finite entry marks the
+// call (the host's flag, and the call's number for apply_out_kernel) and enters
+// as zero, so that it reaches no workspace.
+template <class T>
+__global__ __launch_bounds__(kBlock) void apply_in_kernel(uint32_t n, const uint32_t* __restrict__ new_of_old,
+                                                         const double* __restrict__ r, T* __restrict__ out,
+                                                         uint32_t call, uint32_t* __restrict__ bad,
+                                                         int* __restrict__ seen) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n && !isfinite(v[i])) *flag = 1;
+    if (i >= n) return;
+    double v = r[i];
+    if (!isfinite(v)) {
+        *bad = call;
+        seen[0] = 1;
+        v = 0.0;
+    }
+    out[new_of_old[i]] = T(v);
+}
+
+// The correction out to the caller's order, unless the call is marked.
+template <class T>
+__global__ __launch_bounds__(kBlock) void apply_out_kernel(uint32_t n, const uint32_t* __restrict__ new_of_old,
+                                                          const T* __restrict__ z, double* __restrict__ out,
+                                                          uint32_t call, const uint32_t* __restrict__ bad,
+                                                          int* __restrict__ seen) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n || *bad == call) return;
+    const double v = double(z[new_of_old[i]]);
+    if (!isfinite(v)) seen[1] = 1;
+    out[i] = v;
 }
 }  // namespace
 
@@ -1008,8 +1064,8 @@ bool DeviceAmg::bounded_action(const double* r, double* z, std::string& err) {
         launch_spmv<double>(lv_[0].A, z, InitZero<double>{}, EpiStore<double>{img}, stream_);
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, img, img, partials_);
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, r, r, partials_ + partial_stride_);
-        reduce(partials_, gs, 2, scal_ + 400);
-        fetch_scalars(2, scal_ + 400);
+        reduce(partials_, gs, 2, scal_ + 400, 0, scal_);
+        fetch_scalars(2, 400);
         const double an = std::sqrt(h_scal_[0]), rn = std::sqrt(h_scal_[1]);
         if (!std::isfinite(an) || !std::isfinite(rn) || !(rn > 0.0) || !(an > 0.0)) return rn == 0.0 && an == 0.0;
         return an / rn <= max_image_ratio;
@@ -1029,58 +1085,71 @@ bool DeviceAmg::apply_caller(const double* r_caller, double* z_caller, bool fp32
         err = fp32 ? "no FP32 hierarchy" : "no FP64 hierarchy";
         return false;
     }
-    int* flag = reinterpret_cast<int*>(scal_ + kScalars - 1);
-    int hflag = 0;
-    HIP_OK(hipMemsetAsync(flag, 0, sizeof(int), stream_));
-    nonfinite_flag_kernel<<<g, kBlock, 0, stream_>>>(n, r_caller, flag);
-    HIP_OK(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, stream_));
-    HIP_OK(hipStreamSynchronize(stream_));
-    if (hflag) {
-        err = "non-finite residual";
-        return false;
-    }
+    // Non-finite entries are seen on the way in and out, so that a good call
+    // waits once; a residual that holds any leaves z as it is. seen: [0] in, [1]
+    // out, read by the host; *bad: the number of the last call that was refused.
+    int* seen = reinterpret_cast<int*>(h_scal_ + kScalars - 1);
+    int* d_seen = reinterpret_cast<int*>(scal_host_ + kScalars - 1);
+    uint32_t* bad = reinterpret_cast<uint32_t*>(scal_ + kScalars - 1);
+    const uint32_t call = ++apply_calls_;
+    const_cast<volatile int*>(seen)[0] = const_cast<volatile int*>(seen)[1] = 0;
+    auto flagged = [&](int k) { return const_cast<volatile int*>(seen)[k] != 0; };
+    const bool bounded = max_image_ratio > 0.0;
     bool ok;
-    if (fp32 && max_image_ratio > 0.0) {
-        // The bounded test works on the FP64 result: convert, test, reorder.
+    if (fp32) {
         float* rs = need_vec32(work32_, 4, n);
         float* zs = need_vec32(work32_, 5, n);
-        double* r64 = need_vec(work_, 13, n);
-        double* z64 = need_vec(work_, 14, n);
-        scatter_perm_kernel<double, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, r64);
-        convert_kernel<double, float><<<g, kBlock, 0, stream_>>>(n, r64, rs);
-        ok = vcycle32(rs, zs);
-        if (ok) {
-            convert_kernel<float, double><<<g, kBlock, 0, stream_>>>(n, zs, z64);
-            if (!bounded_action(r64, z64, err)) return false;
-            gather_perm_kernel<double, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, z64, z_caller);
+        double* r64 = bounded ? need_vec(work_, 13, n) : nullptr;
+        if (bounded) {
+            // The bounded test works on the FP64 result: convert, test, reorder.
+            apply_in_kernel<double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, r64, call, bad, d_seen);
+            convert_kernel<double, float><<<g, kBlock, 0, stream_>>>(n, r64, rs);
+        } else {
+            apply_in_kernel<float><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, rs, call, bad, d_seen);
         }
-    } else if (fp32) {
-        float* rs = need_vec32(work32_, 4, n);
-        float* zs = need_vec32(work32_, 5, n);
-        scatter_perm_kernel<double, float><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, rs);
-        ok = vcycle32(rs, zs);
-        if (ok) gather_perm_kernel<float, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, zs, z_caller);
+        if (cns_) ok = vcycle32(rs, zs);
+        else ok = vcycle_t<float>(0, rs, zs);
+        if (ok && bounded) {
+            double* z64 = need_vec(work_, 14, n);
+            convert_kernel<float, double><<<g, kBlock, 0, stream_>>>(n, zs, z64);
+            if (!apply_bounded(r64, z64, seen, err)) return false;
+            apply_out_kernel<double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, z64, z_caller, call, bad, d_seen);
+        } else if (ok) {
+            apply_out_kernel<float><<<g, kBlock, 0, stream_>>>(n, d_perm0_, zs, z_caller, call, bad, d_seen);
+        }
     } else {
         double* rs = need_vec(work_, 13, n);
         double* zs = need_vec(work_, 14, n);
-        scatter_perm_kernel<double, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, rs);
-        ok = vcycle64(rs, zs);
-        if (ok && !bounded_action(rs, zs, err)) return false;
-        if (ok) gather_perm_kernel<double, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, zs, z_caller);
+        apply_in_kernel<double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, r_caller, rs, call, bad, d_seen);
+        if (cns_) ok = vcycle64(rs, zs);
+        else ok = vcycle_t<double>(0, rs, zs);
+        if (ok && bounded && !apply_bounded(rs, zs, seen, err)) return false;
+        if (ok) apply_out_kernel<double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, zs, z_caller, call, bad, d_seen);
+    }
+    HIP_OK(hipStreamSynchronize(stream_));
+    if (flagged(0)) {
+        err = "non-finite residual";
+        return false;
     }
     if (!ok) {
-        HIP_OK(hipStreamSynchronize(stream_));
         err = "native AMG V-cycle failed: singular coarsest level";
         return false;
     }
-    nonfinite_flag_kernel<<<g, kBlock, 0, stream_>>>(n, z_caller, flag);
-    HIP_OK(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, stream_));
-    HIP_OK(hipStreamSynchronize(stream_));
-    if (hflag) {
+    if (flagged(1)) {
         err = "native AMG V-cycle failed: non-finite correction";
         return false;
     }
     return true;
+}
+
+// The bounded test of an application, unless its residual is refused anyway.
+bool DeviceAmg::apply_bounded(const double* r, double* z, const int* seen, std::string& err) {
+    HIP_OK(hipStreamSynchronize(stream_));
+    if (*const_cast<const volatile int*>(seen)) {
+        err = "non-finite residual";
+        return false;
+    }
+    return bounded_action(r, z, err);
 }
 
 // ---------------------------------------------------------------- PCG --
@@ -1151,16 +1220,16 @@ bool DeviceAmg::pcg_in(const PcgWork& w, const double* b_caller, double* x_calle
     if (ns) project_out(ns_modes, ns_count, x);
     dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, b, b, P0);
     launch_spmv<double>(L0.A, x, InitZero<double>{}, EpiResidual<double, true>{b, rv, P1}, stream_);
-    reduce(P0, gs, 1, scal + 0, stride);
+    reduce(P0, gs, 1, scal + 0, stride, scal);
     if (ns) {
         // the initial residual is projected (cg_solver.h:147-156)
         project_out(ns_modes, ns_count, rv);
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, rv, rv, P1);
-        reduce(P1, gs, 1, scal + 1, stride);
+        reduce(P1, gs, 1, scal + 1, stride, scal);
     } else {
-        reduce(P1, nbA, 1, scal + 1, stride);
+        reduce(P1, nbA, 1, scal + 1, stride, scal);
     }
-    fetch_scalars(2, scal);
+    fetch_scalars(2);
     const double bnorm = std::sqrt(h_scal_[0]);
     const double r0 = std::sqrt(h_scal_[1]);
     const double ref = bnorm > 0.0 ? bnorm : r0;
@@ -1179,8 +1248,8 @@ bool DeviceAmg::pcg_in(const PcgWork& w, const double* b_caller, double* x_calle
     if (on_iterate_) on_iterate_(0, x);
     auto true_residual = [&]() {
         launch_spmv<double>(L0.A, x, InitZero<double>{}, EpiResidual<double, true>{b, rv, P1}, stream_);
-        reduce(P1, nbA, 1, scal + 5, stride);
-        fetch_scalars(6, scal);
+        reduce(P1, nbA, 1, scal + 5, stride, scal);
+        fetch_scalars(6);
         return std::sqrt(h_scal_[5]);
     };
     st.min_true = std::numeric_limits<double>::infinity();
@@ -1196,8 +1265,8 @@ bool DeviceAmg::pcg_in(const PcgWork& w, const double* b_caller, double* x_calle
     if (!precondition()) return finish(3, 0, true_residual());
     HIP_OK(hipMemcpyAsync(p, z, size_t(n) * 8, hipMemcpyDeviceToDevice, stream_));
     dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, r, z, P0);
-    reduce(P0, gs, 1, scal + 4, stride);
-    fetch_scalars(5, scal);
+    reduce(P0, gs, 1, scal + 4, stride, scal);
+    fetch_scalars(5);
     double rsold = h_scal_[4];
     if (!std::isfinite(rsold)) return finish(2, 0, true_residual());
     if (!(rsold > 0.0)) return finish(3, 0, true_residual());
@@ -1224,10 +1293,9 @@ bool DeviceAmg::pcg_in(const PcgWork& w, const double* b_caller, double* x_calle
         }
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, r, z, P0);
         launch_spmv<double>(L0.A, x, InitZero<double>{}, EpiResidual<double, true>{b, rv, P1}, stream_);
-        reduce(P2, gs, 1, scal + 3, stride);
-        reduce(P0, gs, 1, scal + 4, stride);
-        reduce(P1, nbA, 1, scal + 5, stride);
-        fetch_scalars(6, scal);
+        reduce_list_kernel<<<3, 1024, 0, stream_>>>(PartialList{{P2, P0, P1}, {gs, gs, uint32_t(nbA)}}, scal + 3,
+                                                    scal_host_ + 3, done_, ++ticket_);
+        await(3);
         const double pAp = h_scal_[2];
         if (!(pAp > 0.0) || !std::isfinite(pAp)) return finish(3, it, true_residual());
         if (!std::isfinite(rsold / pAp)) return finish(2, it, true_residual());
@@ -1257,8 +1325,8 @@ bool DeviceAmg::pcg_in(const PcgWork& w, const double* b_caller, double* x_calle
             if (ns) project_out(ns_modes, ns_count, r);
             if (!precondition()) return finish(3, it, tr);
             dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, r, z, P0);
-            reduce(P0, gs, 1, scal + 4, stride);
-            fetch_scalars(5, scal);
+            reduce(P0, gs, 1, scal + 4, stride, scal);
+            fetch_scalars(5);
             const double rz = h_scal_[4];
             if (!std::isfinite(rz) || !(rz > 0.0)) return finish(3, it, tr);
             HIP_OK(hipMemcpyAsync(p, z, size_t(n) * 8, hipMemcpyDeviceToDevice, stream_));
@@ -1285,80 +1353,129 @@ namespace {
 // previous step's vector u = V_j and orthogonalises w. Basis vectors are
 // padded to a multiple of 64 entries with zeros and read as pairs.
 constexpr int kGsTile = 12;
+inline uint32_t gs_tiles(uint32_t j) { return j == 0 ? 1u : (j + kGsTile - 1) / kGsTile; }
 
 // Products of step j over row pairs (u = V_j):
 //   partials[k]        = V_k . w    for k < j,  partials[j]      = u . w
 //   partials[j + 1 + k] = V_k . u   for k < j,  partials[2j + 1] = u . u
 //   partials[2j + 2]   = w . w
+// blockIdx.y takes kGsTile basis vectors; the sums of a workgroup are formed by
+// wavefronts, stored, and closed by one thread a sum (one block sum after the
+// other, two barriers each, took 10.9 us a step of 75k rows,
+// averaged over a cycle of 17; 9.1 us so, most of it the loads).
 __global__ __launch_bounds__(kBlock) void gs_dot_kernel(uint32_t npairs, size_t ld, uint32_t j,
                                                        const double* __restrict__ V, const double* __restrict__ w,
                                                        double* __restrict__ partials, uint32_t stride) {
 #pragma clang fp contract(off)
-    __shared__ double red[4];
+    constexpr int kSums = 2 * kGsTile + 3;
+    __shared__ double red[kSums][4];
     const double2* up = reinterpret_cast<const double2*>(V + size_t(j) * ld);
     const double2* wp = reinterpret_cast<const double2*>(w);
-    const uint32_t kend = j == 0 ? 1u : j;
-    for (uint32_t k0 = 0; k0 < kend; k0 += kGsTile) {
-        double aw[kGsTile], au[kGsTile];
+    const uint32_t k0 = blockIdx.y * kGsTile;
+    double aw[kGsTile], au[kGsTile];
 #pragma unroll
-        for (int t = 0; t < kGsTile; ++t) aw[t] = au[t] = 0.0;
-        double uw = 0.0, uu = 0.0, ww = 0.0;
-        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < npairs; i += gridDim.x * kBlock) {
-            const double2 wv = wp[i];
-            const double2 uv = up[i];
-#pragma unroll
-            for (int t = 0; t < kGsTile; ++t) {
-                if (k0 + t < j) {
-                    const double2 v = reinterpret_cast<const double2*>(V + size_t(k0 + t) * ld)[i];
-                    aw[t] += v.x * wv.x;
-                    aw[t] += v.y * wv.y;
-                    au[t] += v.x * uv.x;
-                    au[t] += v.y * uv.y;
-                }
-            }
-            if (k0 == 0) {
-                uw += uv.x * wv.x;
-                uw += uv.y * wv.y;
-                uu += uv.x * uv.x;
-                uu += uv.y * uv.y;
-                ww += wv.x * wv.x;
-                ww += wv.y * wv.y;
-            }
-        }
+    for (int t = 0; t < kGsTile; ++t) aw[t] = au[t] = 0.0;
+    double uw = 0.0, uu = 0.0, ww = 0.0;
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < npairs; i += gridDim.x * kBlock) {
+        const double2 wv = wp[i];
+        const double2 uv = up[i];
 #pragma unroll
         for (int t = 0; t < kGsTile; ++t) {
-            if (k0 + t >= j) break;
-            const double a = block_sum(aw[t], red);
-            const double b = block_sum(au[t], red);
-            if (threadIdx.x == 0) {
-                partials[size_t(k0 + t) * stride + blockIdx.x] = a;
-                partials[size_t(j + 1 + k0 + t) * stride + blockIdx.x] = b;
+            if (k0 + t < j) {
+                const double2 v = reinterpret_cast<const double2*>(V + size_t(k0 + t) * ld)[i];
+                aw[t] += v.x * wv.x;
+                aw[t] += v.y * wv.y;
+                au[t] += v.x * uv.x;
+                au[t] += v.y * uv.y;
             }
         }
         if (k0 == 0) {
-            const double a = block_sum(uw, red), b = block_sum(uu, red), c = block_sum(ww, red);
-            if (threadIdx.x == 0) {
-                partials[size_t(j) * stride + blockIdx.x] = a;
-                partials[size_t(2 * j + 1) * stride + blockIdx.x] = b;
-                partials[size_t(2 * j + 2) * stride + blockIdx.x] = c;
-            }
+            uw += uv.x * wv.x;
+            uw += uv.y * wv.y;
+            uu += uv.x * uv.x;
+            uu += uv.y * uv.y;
+            ww += wv.x * wv.x;
+            ww += wv.y * wv.y;
         }
     }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto close_wave = [&](int slot, double v) {
+        v = wave_sum(v);
+        if (lane == 0) red[slot][wave] = v;
+    };
+#pragma unroll
+    for (int t = 0; t < kGsTile; ++t) {
+        if (k0 + t < j) {
+            close_wave(t, aw[t]);
+            close_wave(kGsTile + t, au[t]);
+        }
+    }
+    if (k0 == 0) {
+        close_wave(2 * kGsTile, uw);
+        close_wave(2 * kGsTile + 1, uu);
+        close_wave(2 * kGsTile + 2, ww);
+    }
+    __syncthreads();
+    const int s = threadIdx.x;
+    if (s >= kSums) return;
+    uint32_t slot;
+    if (s < 2 * kGsTile) {
+        const uint32_t k = k0 + uint32_t(s % kGsTile);
+        if (k >= j) return;
+        slot = s < kGsTile ? k : j + 1 + k;
+    } else {
+        if (k0 != 0) return;
+        slot = s == 2 * kGsTile ? j : 2 * j + uint32_t(s - 2 * kGsTile);
+    }
+    partials[size_t(slot) * stride + blockIdx.x] = ((red[s][0] + red[s][1]) + red[s][2]) + red[s][3];
 }
 
-// Update of step j with coef = [s_0..s_{j-1}, c_0..c_{j-1}, nu, h_jj]:
+// The coefficients of step j's update from its reduced products d = [V_k . w
+// (k <= j), V_k . u (k < j), u . u, w . w], as the host computes them, and a
+// last one that is 0 when the host will end the cycle before the update: so the
+// update follows at once, and the host reads both steps' results in one wait.
+__global__ __launch_bounds__(64) void gs_coef_kernel(uint32_t j, const double* __restrict__ d,
+                                                    double* __restrict__ coef) {
+#pragma clang fp contract(off)
+    const double *c = d, *sv = d + j + 1;
+    const double alpha = d[2 * j + 1], an = sqrt(d[2 * j + 2]);
+    for (uint32_t k = threadIdx.x; k < j; k += 64) {
+        coef[k] = sv[k];
+        coef[j + k] = c[k];
+    }
+    if (threadIdx.x != 0) return;
+    double nu = 1.0, hjj = c[0];
+    bool go = isfinite(an) && isfinite(alpha);
+    if (j > 0) {
+        double ss = 0.0, sc = 0.0;
+        for (uint32_t k = 0; k < j; ++k) {
+            ss += sv[k] * sv[k];
+            sc += sv[k] * c[k];
+        }
+        const double nu2 = alpha - ss;
+        go = go && nu2 > 0.5 * alpha;
+        nu = sqrt(nu2);
+        hjj = (c[j] - sc) / nu;
+    }
+    coef[2 * j] = nu;
+    coef[2 * j + 1] = hjj;
+    coef[2 * j + 2] = go ? 1.0 : 0.0;
+}
+
+// Update of step j with coef = [s_0..s_{j-1}, c_0..c_{j-1}, nu, h_jj, go]:
 //   V_j <- (V_j - sum_k s_k V_k) / nu          (j > 0; V_0 is final)
 //   w   <- w - sum_k c_k V_k - h_jj V_j
 // and the partials of |w|^2.
-constexpr uint32_t kGsCoef = 2 * kRestartMax + 2;
+constexpr uint32_t kGsCoef = 2 * kRestartMax + 3;
 __global__ __launch_bounds__(kBlock) void gs_update_kernel(uint32_t npairs, size_t ld, uint32_t j,
                                                           double* __restrict__ V, const double* __restrict__ coef,
                                                           double* __restrict__ w, double* __restrict__ partials) {
 #pragma clang fp contract(off)
     __shared__ double red[4];
     __shared__ double cs[kGsCoef];
-    for (uint32_t k = threadIdx.x; k < 2 * j + 2; k += kBlock) cs[k] = coef[k];
+    for (uint32_t k = threadIdx.x; k < 2 * j + 3; k += kBlock) cs[k] = coef[k];
     __syncthreads();
+    if (cs[2 * j + 2] == 0.0) return;
     const double nu = cs[2 * j], hjj = cs[2 * j + 1];
     double2* up = reinterpret_cast<double2*>(V + size_t(j) * ld);
     double2* wp = reinterpret_cast<double2*>(w);
@@ -1556,19 +1673,20 @@ bool DeviceAmg::gram_schmidt_seconds(uint32_t j, uint32_t repeat, double& dot_s,
     for (uint32_t k = 0; k < 2 * j; ++k) hc[k] = 1e-3;
     hc[2 * j] = 1.0;
     hc[2 * j + 1] = 1e-3;
-    HIP_OK(hipMemcpyAsync(scal_ + kGsCoefSlot, hc, (2 * j + 2) * sizeof(double), hipMemcpyHostToDevice, stream_));
+    hc[2 * j + 2] = 1.0;
+    HIP_OK(hipMemcpyAsync(scal_ + kGsCoefSlot, hc, (2 * j + 3) * sizeof(double), hipMemcpyHostToDevice, stream_));
     const uint32_t gp = std::min<uint32_t>(grid_stride(npairs), kGsStride);
     hipEvent_t e[3];
     for (auto& ev : e) HIP_OK(hipEventCreate(&ev));
     HIP_OK(hipEventRecord(e[0], stream_));
     for (uint32_t r = 0; r < repeat; ++r) {
-        gs_dot_kernel<<<gp, kBlock, 0, stream_>>>(npairs, ld, j, V, w, partials_, kGsStride);
-        reduce_partials_kernel<<<1, 1024, 0, stream_>>>(partials_, gp, kGsStride, 2 * j + 3, scal_ + 16);
+        gs_dot_kernel<<<dim3(gp, gs_tiles(j)), kBlock, 0, stream_>>>(npairs, ld, j, V, w, partials_, kGsStride);
+        reduce(partials_, gp, 2 * j + 3, scal_ + 16, kGsStride, scal_);
     }
     HIP_OK(hipEventRecord(e[1], stream_));
     for (uint32_t r = 0; r < repeat; ++r) {
         gs_update_kernel<<<gp, kBlock, 0, stream_>>>(npairs, ld, j, V, scal_ + kGsCoefSlot, w, partials_);
-        reduce_partials_kernel<<<1, 1024, 0, stream_>>>(partials_, gp, kGsStride, 1, scal_ + 304);
+        reduce(partials_, gp, 1, scal_ + 304, kGsStride, scal_);
     }
     HIP_OK(hipEventRecord(e[2], stream_));
     HIP_OK(hipStreamSynchronize(stream_));
@@ -1629,7 +1747,7 @@ bool DeviceAmg::fgmres(const double* b_caller, double* x_caller, int restart, ui
     scatter_perm_kernel<double, double><<<g, kBlock, 0, stream_>>>(n, d_perm0_, x_caller, x);
     double* P0 = partials_;
     dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, b, b, P0);
-    reduce(P0, gs, 1, scal_);
+    reduce(P0, gs, 1, scal_, 0, scal_);
     fetch_scalars(1);
     const double bn = std::sqrt(h_scal_[0]);
     auto finish = [&](uint32_t status, uint64_t it, double res) {
@@ -1646,7 +1764,7 @@ bool DeviceAmg::fgmres(const double* b_caller, double* x_caller, int restart, ui
     const double tolv = tol * bn;
     auto true_res = [&]() {
         launch_spmv<double>(L0.A, x, InitZero<double>{}, EpiResidual<double, true>{b, r, P0}, stream_);
-        reduce(P0, nbA, 1, scal_);
+        reduce(P0, nbA, 1, scal_, 0, scal_);
         fetch_scalars(1);
         return std::sqrt(h_scal_[0]);
     };
@@ -1687,7 +1805,7 @@ bool DeviceAmg::fgmres(const double* b_caller, double* x_caller, int restart, ui
             return true;
         }
         dot_partial_kernel<double><<<gs, kBlock, 0, stream_>>>(n, x, x, P0);
-        reduce(P0, gs, 1, scal_);
+        reduce(P0, gs, 1, scal_, 0, scal_);
         fetch_scalars(1);
         const double ref_scale = std::max({std::sqrt(h_scal_[0]), 1.0, 1e-300});
         return done(ax0 <= tol * ref_scale ? 0u : 2u, 0, ax0, ax0 / ref_scale);
@@ -1794,10 +1912,13 @@ bool DeviceAmg::fgmres(const double* b_caller, double* x_caller, int restart, ui
             // w = A z_j
             launch_spmv<double>(L0.A, zj, InitZero<double>{}, EpiStore<double>{w}, stream_);
             const uint32_t cnt = 2 * j + 3;
-            gs_dot_kernel<<<gp, kBlock, 0, stream_>>>(npairs, ld, j, V, w, partials_, kGsStride);
-            reduce_partials_kernel<<<1, 1024, 0, stream_>>>(partials_, gp, kGsStride, cnt, scal_ + 16);
-            HIP_OK(hipMemcpyAsync(h_scal_ + 16, scal_ + 16, cnt * sizeof(double), hipMemcpyDeviceToHost, stream_));
-            HIP_OK(hipStreamSynchronize(stream_));
+            gs_dot_kernel<<<dim3(gp, gs_tiles(j)), kBlock, 0, stream_>>>(npairs, ld, j, V, w, partials_, kGsStride);
+            reduce(partials_, gp, cnt, scal_ + 16, kGsStride);
+            gs_coef_kernel<<<1, 64, 0, stream_>>>(j, scal_ + 16, scal_ + kGsCoefSlot);
+            gs_update_kernel<<<gp, kBlock, 0, stream_>>>(npairs, ld, j, V, scal_ + kGsCoefSlot, w, partials_);
+            reduce_step_kernel<<<1, 1024, 0, stream_>>>(partials_, gp, scal_ + 304, scal_host_ + 304, cnt, scal_ + 16,
+                                                        scal_host_ + 16, done_, ++ticket_);
+            await(1);
             const double* c = h_scal_ + 16;           // V_k . w, k <= j
             const double* sv = h_scal_ + 16 + j + 1;  // V_k . u, k < j
             const double alpha = h_scal_[16 + 2 * j + 1];
@@ -1830,19 +1951,7 @@ bool DeviceAmg::fgmres(const double* b_caller, double* x_caller, int restart, ui
                 close_column(j - 1, pend);
                 hjj = (c[j] - sc) / nu;
             }
-            double* hc = h_scal_ + kGsCoefSlot;
-            for (uint32_t k = 0; k < j; ++k) {
-                hc[k] = sv[k];
-                hc[j + k] = c[k];
-            }
-            hc[2 * j] = nu;
-            hc[2 * j + 1] = hjj;
-            HIP_OK(hipMemcpyAsync(scal_ + kGsCoefSlot, hc, (2 * j + 2) * sizeof(double), hipMemcpyHostToDevice,
-                                  stream_));
-            gs_update_kernel<<<gp, kBlock, 0, stream_>>>(npairs, ld, j, V, scal_ + kGsCoefSlot, w, partials_);
-            reduce_partials_kernel<<<1, 1024, 0, stream_>>>(partials_, gp, kGsStride, 1, scal_ + 304);
-            fetch_scalars(1, scal_ + 304);
-            const double hn = std::sqrt(h_scal_[0]);
+            const double hn = std::sqrt(h_scal_[304]);
             if (!std::isfinite(hn)) {
                 HIP_OK(hipMemcpyAsync(x, bestx, size_t(n) * 8, hipMemcpyDeviceToDevice, stream_));
                 return finish(2, its, best);

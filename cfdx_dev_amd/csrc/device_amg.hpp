@@ -385,8 +385,9 @@ private:
     void release_refresh();
     void release();
     // stride 0: the hierarchy's own partial-sum stride; src null: scal_.
-    void reduce(const double* partials, uint32_t n, uint32_t count, double* out, uint64_t stride = 0);
-    bool fetch_scalars(uint32_t count, const double* src = nullptr);
+    void reduce(const double* partials, uint32_t n, uint32_t count, double* out, uint64_t stride = 0,
+                const double* base = nullptr);
+    bool fetch_scalars(uint32_t count, uint32_t first = 0);
 
     // The FP64 V-cycle's single-launch coarse end (coarse_tail.hpp): its
     // first level (the number of levels: none), the level descriptors on the
@@ -418,6 +419,8 @@ private:
     std::vector<RefreshView> rf_view_host_;
     LanczosState* rf_lz_ = nullptr;
     double* rf_ub_ = nullptr;        // Gershgorin bound per level
+    uint2* rf_long_ = nullptr;     // (level, row) of the levels' long rows, longest first
+    uint32_t rf_nlong_ = 0;
     std::vector<int> rf_host_flags_;
     std::vector<double> rf_host_ub_;
     HCsr rf_coarsest_;               // pattern and fetched values of the coarsest level
@@ -447,6 +450,11 @@ private:
     uint64_t partial_stride_ = 0;
     double* scal_ = nullptr;        // device scalars
     double* h_scal_ = nullptr;      // pinned host mirror
+    unsigned long long *h_done_ = nullptr, *done_ = nullptr, ticket_ = 0;  // tickets of awaited kernels (pinned)
+    void await(int count);
+    uint32_t apply_calls_ = 0;
+    bool apply_bounded(const double* r, double* z, const int* seen, std::string& err);
+    double* scal_host_ = nullptr;  // h_scal_ as the device addresses it
     std::vector<double*> work_;     // generic FP64 n-vectors
     std::vector<float*> work32_;
     std::vector<double*> basis_;    // FGMRES V (m+1), Z (m) and w, padded

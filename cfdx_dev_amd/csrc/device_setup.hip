@@ -627,7 +627,6 @@ __global__ __launch_bounds__(kBlock) void lanczos_scale_kernel(const RefreshView
 
 // w = sq (A u): w_i = sq_i sum_q a_iq (sq_j v_j) in each row's entry order.
 struct EpiScaled {
-    static constexpr bool kPartial = false;
     struct Pre {
         double d;
     };

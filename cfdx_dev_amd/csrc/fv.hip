@@ -241,13 +241,11 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
     }
 }
 
-// The cell block of a launch's workgroup: each XCD takes one contiguous range
-// of cells (workgroups go to the XCDs in turn), so that the records a cell and
-// its neighbours share are fetched into one L2 rather than into most of them.
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t nb = gridDim.x, b = blockIdx.x, x = b & 7u;
-    return x * (nb >> 3) + min(x, nb & 7u) + (b >> 3);
-}
+// Cells go to workgroups by xcd_block: each XCD takes one contiguous range, so
+// that the records a cell and its neighbours share are fetched into one L2
+// rather than into most of them (a 222k-cell channel's pressure rows: 40 us in
+// launch order, 31 so).
+__device__ __forceinline__ uint32_t cell_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 // Slots a thread loads together: the loads of one slot depend on each other
 // (cell id, then that cell's record), so a thread that walks them one by one
@@ -266,7 +264,7 @@ __global__ __launch_bounds__(kBlock) void gauss_gradient_kernel(
     const uint8_t* __restrict__ bct, const double* __restrict__ bcv, Soa3 fc, Soa3 cc, const double* __restrict__ vol,
     const double* __restrict__ p, uint32_t ps, double* __restrict__ grad) {
 #pragma clang fp contract(off)
-    const uint32_t c = xcd_block() * kBlock + threadIdx.x;
+    const uint32_t c = cell_block() * kBlock + threadIdx.x;
     if (c >= nc) return;
     const double pc = p[size_t(c) * ps];
     D3 sum = d3(0.0, 0.0, 0.0);
@@ -396,6 +394,12 @@ __global__ __launch_bounds__(kBlock) void pack_momentum_kernel(
     source[i] = make_double4(s[0], s[1], s[2], 0.0);
 }
 
+__global__ __launch_bounds__(kBlock) void fetch_bcs_kernel(uint32_t words, const double* __restrict__ from,
+                                                          double* __restrict__ to, int* __restrict__ flags) {
+    for (uint32_t i = threadIdx.x; i < words; i += kBlock) to[i] = from[i];
+    if (flags && threadIdx.x < 4) flags[threadIdx.x] = 0;
+}
+
 // Records (x, y, z, w) a cell out to the caller's order: v 3 x nc, w nc.
 __global__ __launch_bounds__(kBlock) void unpack_cells_kernel(uint32_t nc, const uint32_t* __restrict__ from,
                                                              const double4* __restrict__ rec,
@@ -493,7 +497,7 @@ __global__ __launch_bounds__(kBlock) void pressure_row_kernel(
     int* __restrict__ err) {
 #pragma clang fp contract(off)
     extern __shared__ double2 row_shared[];
-    const uint32_t first = xcd_block() * kBlock;
+    const uint32_t first = cell_block() * kBlock;
     const bool live = first + threadIdx.x < nc;
     const uint32_t c = live ? first + threadIdx.x : nc - 1;  // the last block's spare threads only keep step
     double* lds = reinterpret_cast<double*>(row_shared);
@@ -965,7 +969,7 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
     static_assert(K == 1 || K == 3);
     __shared__ double2 near_lds[K == 3 ? 2 * kBlock : 1];
     if (gate && !gate[0]) return;
-    const uint32_t first = xcd_block() * kBlock, c = first + threadIdx.x;
+    const uint32_t first = cell_block() * kBlock, c = first + threadIdx.x;
     const Near near{near_lds, first};
     const double4* rec = reinterpret_cast<const double4*>(field);
     double value[K];
@@ -1192,7 +1196,7 @@ __global__ __launch_bounds__(kBlock) void momentum_row_kernel(
     double* __restrict__ vals, double4* __restrict__ out, int* __restrict__ err) {
 #pragma clang fp contract(off)
     extern __shared__ double2 row_shared[];
-    const uint32_t first = xcd_block() * kBlock;
+    const uint32_t first = cell_block() * kBlock;
     const bool live = first + threadIdx.x < nc;
     const uint32_t c = live ? first + threadIdx.x : nc - 1;  // the last block's spare threads only keep step
     const bool needs = nonorthogonal && flags[0];
@@ -1396,14 +1400,6 @@ __global__ __launch_bounds__(kBlock) void velocity_correct_kernel(uint32_t nc, c
     for (int k = 0; k < 3; ++k) U[k * n1 + c] = hbya[k * n1 + c] - rau[k * n1 + c] * gradp[k * n1 + c] * vol[c];
 }
 
-__global__ __launch_bounds__(kBlock) void positive_check_kernel(uint64_t n, const double* __restrict__ x,
-                                                               int code, int* __restrict__ err) {
-    const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const double v = x[i];
-    if (!isfinite(v) || v <= 0.0) err[0] = code;
-}
-
 // Rhie-Chow face mass flux from HbyA and p (make_rhie_chow_mass_flux,
 // HBYA_PREDICTOR contract, w = 1/2): rho H_f.S_f minus the pressure
 // correction (internal: rhie_chow_pressure_flux_internal; fixed-pressure
@@ -1424,6 +1420,12 @@ __global__ __launch_bounds__(kBlock) void rhie_chow_flux_kernel(
     D3 Hf = d3(H[o], H[nc + o], H[n2 + o]);
     double correction = 0.0;
     const D3 Sf = fs.get(f);
+    // rAU must be finite and positive; every cell is some face's.
+    auto invalid = [&](uint32_t i) {
+        const double a = rAU[i], b = rAU[nc + i], c = rAU[n2 + i];
+        return !(a > 0.0 && b > 0.0 && c > 0.0 && isfinite(a) && isfinite(b) && isfinite(c));
+    };
+    if (invalid(o) || (neigh[f] >= 0 && invalid(uint32_t(neigh[f])))) err[0] = 53;
     if (neigh[f] >= 0) {
         const uint32_t n = uint32_t(neigh[f]);
         const D3 Hn = d3(H[n], H[nc + n], H[n2 + n]);
@@ -1606,13 +1608,13 @@ void FvMesh::release() {
     dfree(wls_meta);
     dfree(neigh);
     dfree(patch_kind);
-    dfree(err);
+    if (h_err) (void)hipHostFree(h_err);
+    h_err = err = nullptr;
+    if (bc_host) (void)hipHostFree(bc_host);
+    bc_host = nullptr;
     dfree(mom_flags);
-    dfree(bc_u8);
     pressure_full.release();
     pressure_red.release();
-    dfree(pbc_u8);
-    dfree(pbc_f64);
 }
 
 // Lines of 16 values that the neighbours and the faces of 64 consecutive cells
@@ -1759,7 +1761,11 @@ void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy
     patch_kind = upload(hkind, npatch);
     for (double** p : {&fcx, &fcy, &fcz, &fsx, &fsy, &fsz}) *p = dalloc<double>(nf);
     for (double** p : {&ccx, &ccy, &ccz, &vol, &vol_caller}) *p = dalloc<double>(nc);
-    err = dalloc<int>(4);
+    // The error flags are host memory that kernels write only when they refuse
+    // something: the host reads and clears them without a copy or a launch.
+    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&h_err), 4 * sizeof(int), hipHostMallocMapped));
+    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&err), h_err, 0));
+    clear_err();
     HIP_OK(hipStreamCreate(&stream));
     compute_geometry();
     gather_u32idx_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, cell_new, vol, vol_caller);
@@ -1836,17 +1842,22 @@ double* FvMesh::cout_buf(double* caller, size_t slot, int comps) {
 }
 double* FvMesh::fout_buf(double* caller, size_t slot) { return identity_order ? caller : scr(slot, nf); }
 
+// Before the first kernel of a call (every call that may raise a flag ends
+// synchronised, so none is in flight).
+void FvMesh::clear_err() {
+    for (int k = 0; k < 4; ++k) const_cast<volatile int*>(h_err)[k] = 0;
+}
+
+// After the call's synchronisation.
 void FvMesh::check_err(const char* what) {
-    int h[4] = {0, 0, 0, 0};
-    HIP_OK(hipMemcpy(h, err, sizeof h, hipMemcpyDeviceToHost));
-    if (h[0] != 0) {
-        HIP_OK(hipMemset(err, 0, 4 * sizeof(int)));
-        throw std::domain_error(std::string(what) + " (code " + std::to_string(h[0]) + ")");
-    }
+    const int code = *const_cast<volatile int*>(h_err);
+    if (code == 0) return;
+    clear_err();
+    throw std::domain_error(std::string(what) + " (code " + std::to_string(code) + ")");
 }
 
 void FvMesh::compute_geometry() {
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     face_geometry_kernel<<<grid_for(nf), kBlock, 0, stream>>>(nf, px, py, pz, foff, fvtx, fc, fs, err);
     cell_centre_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, cfaces, fc, fs, cc);
@@ -1879,8 +1890,6 @@ void FvMesh::ensure_work() {
     work_diag = dalloc<double>(nc);
     work_rhs = dalloc<double>(nc);
     work_grad = dalloc<double>(4 * uint64_t(nc));
-    pbc_u8 = dalloc<uint8_t>(std::max<uint32_t>(npatch, 1));
-    pbc_f64 = dalloc<double>(std::max<uint32_t>(npatch, 1));
 }
 
 // Slot stencils (geometry only): built on first use.
@@ -1916,7 +1925,7 @@ void FvMesh::ensure_slots() {
         slot_sorted = upload(sorted.data(), m);
     }
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     slot_build_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, D, coff, cfaces, owner, neigh, patch, npatch,
                                                            patch_kind, fc, fs, cc, vol, cell_rec, slots_of(*this), err);
     HIP_OK(hipStreamSynchronize(stream));
@@ -1942,7 +1951,7 @@ void FvMesh::ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt) {
     }
     wls_key.clear();
     const Soa3 fc{fcx, fcy, fcz}, cc{ccx, ccy, ccz};
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     wls_build_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, coff, slots_of(*this), patch, npatch, d_bt, fc, cc,
                                                           stencil_dimension(), wls_of(*this), err);
     HIP_OK(hipStreamSynchronize(stream));
@@ -2132,13 +2141,11 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
     const bool fixed = has_fixed_pressure(h_pbt);
     const bool eliminate = !fixed && nc > 1 && ref < nc;
     const PressurePlan& plan = pressure_plan(eliminate, uint32_t(eliminate ? ref : 0));
-    uint8_t* d_pbt = pbc_u8;
-    double* d_pbv = pbc_f64;
-    if (npatch) {
-        HIP_OK(hipMemcpyAsync(d_pbt, h_pbt, npatch, hipMemcpyHostToDevice, stream));
-        HIP_OK(hipMemcpyAsync(d_pbv, h_pbv, size_t(npatch) * 8, hipMemcpyHostToDevice, stream));
-    }
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    upload_bcs(nullptr, nullptr, h_pbt, h_pbv, true, nullptr);
+    const uint32_t npp = std::max<uint32_t>(npatch, 1);
+    const uint8_t* d_pbt = bc_u8 + npp;
+    const double* d_pbv = bc_f64 + 3 * size_t(npp);
+    clear_err();
     const Soa3 fc{fcx, fcy, fcz};
     double4* rec = reinterpret_cast<double4*>(scr(5, 4 * uint64_t(nc)));
     pack_cells_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, d_rAU, d_p, rec);
@@ -2165,7 +2172,7 @@ const PressurePlan& FvMesh::diffusion_assemble_device(double gamma, const double
                                                       const uint8_t* d_fneu, double* d_vals, double* d_rhs) {
     ensure_work();
     const PressurePlan& plan = pressure_plan(false, 0);
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     const double* src_i = cin(d_source, 3, 1);
     const double* fval_i = fin(d_fval, 7);
@@ -2194,9 +2201,6 @@ void FvMesh::ensure_momentum_work() {
     if (mom_flags) return;
     ensure_slots();
     mom_ugrad = dalloc<double>(12 * uint64_t(nc));
-    const uint32_t npp = std::max<uint32_t>(npatch, 1);
-    bc_u8 = dalloc<uint8_t>(2 * uint64_t(npp));
-    bc_f64 = dalloc<double>(4 * uint64_t(npp));
     // Which patches (last: the internal faces) hold non-orthogonal faces, and
     // which ones faces that do not say: geometry, so found once.
     const uint32_t nflag = 2 * (npatch + 1);
@@ -2211,23 +2215,33 @@ void FvMesh::ensure_momentum_work() {
     mom_flags = flags;
 }
 
-// Boundary data per patch into the persistent device buffers (no allocation
-// per call): bc_u8 = [velocity type | pressure type], bc_f64 = [3 velocity
-// values | pressure value]. Types other than 1 read as zero-gradient.
-void FvMesh::upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv) {
-    ensure_momentum_work();
-    const uint32_t npp = std::max<uint32_t>(npatch, 1);
-    h_bc_u8.assign(2 * size_t(npp), 0);
-    h_bc_f64.assign(4 * size_t(npp), 0.0);
+// Boundary data per patch into the persistent device buffer (no allocation per
+// call): bc_f64 = [3 velocity values | pressure value], bc_u8 = [velocity type |
+// pressure type], written by the host into pinned memory and fetched by one
+// small kernel, which also clears the call's device flags. Pressure types other
+// than 1 read as zero-gradient unless raw_pbt. (Two copies of a few
+// bytes and a fill took 10 us of a 222k-cell pressure assembly's 90.)
+void FvMesh::upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv,
+                        bool raw_pbt, int* flags) {
+    const size_t npp = std::max<uint32_t>(npatch, 1);
+    const uint32_t words = uint32_t(4 * npp + (2 * npp + 7) / 8);
+    if (!bc_host) {
+        if (!bc_f64) bc_f64 = dalloc<double>(words);
+        bc_u8 = reinterpret_cast<uint8_t*>(bc_f64 + 4 * npp);
+        HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&bc_host), words * 8, hipHostMallocMapped));
+        h_bc_u8 = reinterpret_cast<uint8_t*>(bc_host + 4 * npp);
+    }
+    std::memset(bc_host, 0, words * 8);
     for (uint32_t p = 0; p < npatch; ++p) {
         if (h_vbt) h_bc_u8[p] = h_vbt[p] == 1 ? 1 : 0;
-        if (h_pbt) h_bc_u8[npp + p] = h_pbt[p] == 1 ? 1 : 0;
+        if (h_pbt) h_bc_u8[npp + p] = raw_pbt ? h_pbt[p] : (h_pbt[p] == 1 ? 1 : 0);
         for (int k = 0; k < 3; ++k)
-            if (h_vbv) h_bc_f64[3 * size_t(p) + k] = h_vbv[3 * size_t(p) + k];
-        if (h_pbv) h_bc_f64[3 * size_t(npp) + p] = h_pbv[p];
+            if (h_vbv) bc_host[3 * size_t(p) + k] = h_vbv[3 * size_t(p) + k];
+        if (h_pbv) bc_host[3 * npp + p] = h_pbv[p];
     }
-    HIP_OK(hipMemcpyAsync(bc_u8, h_bc_u8.data(), h_bc_u8.size(), hipMemcpyHostToDevice, stream));
-    HIP_OK(hipMemcpyAsync(bc_f64, h_bc_f64.data(), h_bc_f64.size() * 8, hipMemcpyHostToDevice, stream));
+    double* from = nullptr;
+    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&from), bc_host, 0));
+    fetch_bcs_kernel<<<1, kBlock, 0, stream>>>(words, from, bc_f64, flags);
 }
 
 int FvMesh::stencil_dimension() const {
@@ -2241,7 +2255,7 @@ void FvMesh::wls_gradient_device(const uint8_t* h_bt, const double* h_bv, double
     if (!(limit >= 1.0) || !std::isfinite(limit)) throw std::invalid_argument("boundary WLS: invalid condition limit");
     uint8_t* d_bt = upload(h_bt, std::max<uint32_t>(npatch, 1));
     double* d_bv = upload(h_bv, std::max<uint32_t>(npatch, 1));
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     double* g_i = cout_buf(d_grad, 8, 3);
     try {
@@ -2272,10 +2286,11 @@ const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const
                                                      double alpha, double* d_vals, double* d_rhs, double* d_diag) {
     if (!(alpha > 0.0 && alpha <= 1.0)) throw std::invalid_argument("relax_momentum_equation: invalid relaxation");
     const PressurePlan& plan = pressure_plan(false, 0);
-    upload_bcs(h_vbt, h_vbv, nullptr, nullptr);
+    ensure_momentum_work();
+    upload_bcs(h_vbt, h_vbv, nullptr, nullptr, false, mom_flags);
     const uint8_t* d_vbt = bc_u8;
     const double* d_vbv = bc_f64;
-    ensure_wls_cache(h_bc_u8.data(), d_vbt);
+    ensure_wls_cache(h_bc_u8, d_vbt);
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     bool nonorthogonal = h_nonorth[npatch], undefined = h_nonorth[2 * npatch + 1];
     for (uint32_t p = 0; p < npatch; ++p) {
@@ -2286,8 +2301,7 @@ const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const
     auto records = [&](size_t slot) { return reinterpret_cast<double4*>(scr(slot, 4 * uint64_t(nc))); };
     double4 *rec = records(0), *source = records(1), *out = records(2);
     const double* phi_i = fin(d_phi, 4);
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
-    HIP_OK(hipMemsetAsync(mom_flags, 0, 4 * sizeof(int), stream));
+    clear_err();
     pack_momentum_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, d_U, d_mu,
                                                               d_gradp, d_body, rec, source, mom_flags, err);
     if (nonorthogonal)
@@ -2312,7 +2326,7 @@ const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const
 void FvMesh::momentum_hbya_device(const double* d_vals, const double* d_rhs, const double* d_diag,
                                   const double* d_gradp, const double* d_U, double* d_rau, double* d_hbya) {
     const PressurePlan& plan = pressure_plan(false, 0);
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
+    clear_err();
     hbya_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, plan.rowp, plan.cols, d_vals, d_rhs, d_diag, d_gradp,
                                                      vol_caller, d_U, d_rau, d_hbya, err);
     HIP_OK(hipStreamSynchronize(stream));
@@ -2329,15 +2343,14 @@ void FvMesh::rhie_chow_flux_device(const uint8_t* h_vbt, const double* h_vbv, co
                                    const double* h_pbv, double rho, const double* d_hbya, const double* d_p,
                                    const double* d_rau, double* d_phi) {
     ensure_work();
-    upload_bcs(h_vbt, h_vbv, h_pbt, h_pbv);
+    upload_bcs(h_vbt, h_vbv, h_pbt, h_pbv, false, nullptr);
     const uint32_t npp = std::max<uint32_t>(npatch, 1);
     const uint8_t* d_vbt = bc_u8;
     const uint8_t* d_pbt = bc_u8 + npp;
     const double* d_vbv = bc_f64;
     const double* d_pbv = bc_f64 + 3 * size_t(npp);
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
-    HIP_OK(hipMemsetAsync(err, 0, 4 * sizeof(int), stream));
-    positive_check_kernel<<<grid_for(3 * uint64_t(nc)), kBlock, 0, stream>>>(3 * uint64_t(nc), d_rau, 53, err);
+    clear_err();
     const double* h_i = cin(d_hbya, 6, 3);
     const double* rau_i = cin(d_rau, 5, 3);
     const double* p_i = cin(d_p, 9, 1);

@@ -52,13 +52,10 @@ struct FvMesh {
     double *ccx = nullptr, *ccy = nullptr, *ccz = nullptr;
     double* vol = nullptr;
     double* vol_caller = nullptr;  // cell volumes in the caller's numbering
-    int* err = nullptr;
+    int *err = nullptr, *h_err = nullptr;  // error flags: device and host address of pinned memory
     // work
     double *work_coeff = nullptr, *work_bsrc = nullptr, *work_diag = nullptr,
            *work_rhs = nullptr, *work_grad = nullptr, *work_phi = nullptr;
-    // pressure boundary types / values per patch, refreshed by each assembly
-    uint8_t* pbc_u8 = nullptr;
-    double* pbc_f64 = nullptr;
     // momentum side: velocity WLS gradients (three records a cell), flags, and
     // per patch (last: internal faces) whether faces are non-orthogonal, then
     // whether their geometry leaves that undefined
@@ -66,11 +63,12 @@ struct FvMesh {
     int* mom_flags = nullptr;
     std::vector<int> h_nonorth;
     double* slot_coeff = nullptr;  // coefficients per slot, where they do not fit LDS
-    // per-patch boundary data of the momentum-side calls (persistent)
+    // per-patch boundary data of a call: device buffer (bc_u8 in its tail) and
+    // its pinned host side
     uint8_t* bc_u8 = nullptr;
     double* bc_f64 = nullptr;
-    std::vector<uint8_t> h_bc_u8;
-    std::vector<double> h_bc_f64;
+    double* bc_host = nullptr;
+    uint8_t* h_bc_u8 = nullptr;
     PressurePlan pressure_full, pressure_red;
     // host copies of the addressing
     std::vector<uint32_t> h_owner, h_coff, h_cf, h_patch;
@@ -127,7 +125,8 @@ struct FvMesh {
                                const double* h_pbv, double rho, const double* d_hbya, const double* d_p,
                                const double* d_rau, double* d_phi);
     void ensure_momentum_work();
-    void upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv);
+    void upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv, bool raw_pbt, int* flags);
+    void clear_err();
     int stencil_dimension() const;
     void ensure_work();
     double* scr(size_t slot, uint64_t count);

@@ -73,26 +73,80 @@ __device__ __forceinline__ T block_sum(T v, T* smem4) {
 }
 
 // Sums `count` partial arrays (each of length n, stride `stride`) into
-// out[slot0 + j]. One workgroup, fixed order: deterministic.
+// out[j], one workgroup an array (of up to 63 in a Gram-Schmidt step, where one
+// workgroup for all took 7.9 us on average), in a fixed order: deterministic.
+// mirror: pinned host memory that receives the sums as well, so that a host
+// that waits for them needs no copy.
+// The write to the host costs a launch about 1.5 us, so only sums that are
+// waited for ask for it.
+__device__ __forceinline__ double sum_partials(const double* __restrict__ p, uint32_t n, double* sm /* 16 */) {
+    double v = 0.0;
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) v += p[i];
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (lane == 0) sm[wid] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < 16; ++w) s += sm[w];
+    return s;
+}
+
 static __global__ __launch_bounds__(1024) void reduce_partials_kernel(const double* __restrict__ partials,
-                                                               uint32_t n, uint32_t stride, uint32_t count,
-                                                               double* __restrict__ out) {
+                                                               uint32_t n, uint32_t stride,
+                                                               double* __restrict__ out,
+                                                               double* __restrict__ mirror) {
     __shared__ double sm[16];
-    for (uint32_t j = 0; j < count; ++j) {
-        const double* p = partials + size_t(j) * stride;
-        double v = 0.0;
-        for (uint32_t i = threadIdx.x; i < n; i += 1024) v += p[i];
-        v = wave_sum(v);
-        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-        if (lane == 0) sm[wid] = v;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double s = 0.0;
-            for (int w = 0; w < 16; ++w) s += sm[w];
-            out[j] = s;
-        }
-        __syncthreads();
-    }
+    const uint32_t j = blockIdx.x;
+    const double s = sum_partials(partials + size_t(j) * stride, n, sm);
+    if (threadIdx.x != 0) return;
+    out[j] = s;
+    if (mirror) mirror[j] = s;
+}
+
+// Tells a host that polls `done` (pinned) that this workgroup's writes to pinned
+// memory, all made by the calling thread, have arrived.
+__device__ __forceinline__ void signal_host(unsigned long long* done, unsigned long long ticket) {
+    __threadfence_system();
+    __hip_atomic_store(done, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The sums that end a PCG iteration, of three arrays of their own lengths, in one
+// launch: out[j] = sum of p[j]; mirror receives them and, in front of them, the
+// scalar that precedes out. done[j]: see signal_host.
+struct PartialList {
+    const double* p[3];
+    uint32_t n[3];
+};
+static __global__ __launch_bounds__(1024) void reduce_list_kernel(PartialList list, double* __restrict__ out,
+                                                                 double* __restrict__ mirror,
+                                                                 unsigned long long* __restrict__ done,
+                                                                 unsigned long long ticket) {
+    __shared__ double sm[16];
+    const uint32_t j = blockIdx.x;
+    const double s = sum_partials(list.p[j], list.n[j], sm);
+    if (threadIdx.x != 0) return;
+    out[j] = mirror[j] = s;
+    if (j == 0) mirror[-1] = out[-1];
+    signal_host(done + j, ticket);
+}
+
+// The sum that ends a Gram-Schmidt step, with the step's `count` products (src)
+// for the host as well: mirror[0..count) and *sum_mirror.
+static __global__ __launch_bounds__(1024) void reduce_step_kernel(const double* __restrict__ partials, uint32_t n,
+                                                                 double* __restrict__ out,
+                                                                 double* __restrict__ sum_mirror, uint32_t count,
+                                                                 const double* __restrict__ src,
+                                                                 double* __restrict__ mirror,
+                                                                 unsigned long long* __restrict__ done,
+                                                                 unsigned long long ticket) {
+    __shared__ double sm[16];
+    for (uint32_t k = threadIdx.x; k < count; k += 1024) mirror[k] = src[k];
+    __threadfence_system();
+    const double s = sum_partials(partials, n, sm);  // a barrier between the copies and the signal
+    if (threadIdx.x != 0) return;
+    *out = *sum_mirror = s;
+    signal_host(done, ticket);
 }
 
 // ------------------------------------------------------------------ SpMV --
@@ -159,7 +213,7 @@ constexpr uint32_t kGroupLanes = CFDX_GROUP_LANES;   // power of two, at most 64
 // FP32 rows of a block that one lane (16 lanes in a block of long rows) would
 // sum for longer than the whole wavefront: the coarse levels mix rows of a few
 // entries with rows that span the level, and such a row summed by one lane
-// kept a launch of seven workgroups waiting 12 us.
+// kept a launch of seven workgroups waiting 12 us (4.5 us so).
 constexpr uint32_t kWaveRowNnz = 24;
 constexpr uint32_t kGroupRowMax = 128;
 
@@ -951,8 +1005,8 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(uint32_t n, const T* __res
 // updates every component at once, each with the operations of the sequential
 // elimination. The back substitution subtracts a row's terms in ascending
 // column order, a chain that only lane ii can follow, so its products are
-// formed by the lanes and read in order. 24 us with one lane and its arrays in
-// scratch memory, see coarse_lu_solve.
+// formed by the lanes and read in order. 10.7 us for n = 16 in a launch of its
+// own; 24 us with one lane and its arrays in scratch memory.
 template <class T>
 __device__ __forceinline__ void coarse_lu_solve(uint32_t n, uint32_t nr, const uint32_t* __restrict__ piv,
                                                 const double* __restrict__ factor, const double* __restrict__ upper,

@@ -19,6 +19,7 @@
 #include <stdexcept>
 
 #include "kernels.hpp"
+#include "parallel.h"
 
 namespace cfdxhip {
 
@@ -792,6 +793,7 @@ Mpnn::~Mpnn() {
     mpnn_free(gm_);
     mpnn_free(gpart_);
     for (auto& t : t_) mpnn_free(t);
+    free_host_vectors();
     mpnn_free(pairs_r);
     mpnn_free(pairs_e);
 }
@@ -812,6 +814,33 @@ void Mpnn::ensure(uint32_t n) {
     for (auto& h : h_) h = mpnn_alloc<uint16_t>(uint64_t(n) * kHid);
     for (auto& t : t_) t = mpnn_alloc<float>(n);
     cap_ = n;
+}
+
+const Mpnn::HostVectors& Mpnn::host_vectors(uint32_t n) {
+    if (n > host_cap_) {
+        MPNN_HIP(hipDeviceSynchronize());
+        free_host_vectors();
+        for (int k = 0; k < 2; ++k) {
+            MPNN_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_.h[k]), n * sizeof(float), hipHostMallocMapped));
+            MPNN_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&host_.d[k]), host_.h[k], 0));
+        }
+        MPNN_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_.hgrad), kMpnnParams * sizeof(float),
+                               hipHostMallocDefault));
+        host_.r = mpnn_alloc<float>(n);
+        host_.g = mpnn_alloc<float>(n);
+        host_.e = mpnn_alloc<float>(n);
+        host_.grad = mpnn_alloc<float>(kMpnnParams);
+        host_cap_ = n;
+    }
+    return host_;
+}
+
+void Mpnn::free_host_vectors() {
+    host_cap_ = 0;
+    for (float* h : {host_.h[0], host_.h[1], host_.hgrad})
+        if (h) (void)hipHostFree(h);
+    host_.h[0] = host_.h[1] = host_.d[0] = host_.d[1] = host_.hgrad = nullptr;
+    for (float** f : {&host_.r, &host_.g, &host_.e, &host_.grad}) mpnn_free(*f);
 }
 
 void Mpnn::reserve_pairs(uint32_t n, uint32_t count) {
@@ -857,7 +886,7 @@ void Mpnn::forward(DeviceAmg& amg, const float* r, float* e, bool keep) {
     if (keep) last_r_ = r;
     const uint32_t rg = red_grid(n);
     scale_kernel<<<rg, kBlock, 0, st>>>(n, r, g.inv_diag, s_, part_);
-    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, 1, scal_);
+    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, scal_, nullptr);
     rho_kernel<<<1, 1, 0, st>>>(scal_, n);
     const uint32_t tiles = tiles_of(n);
     auto wt_of = [&](int l) { return wt_ + l * 2 * kHid * kHid; };
@@ -948,7 +977,7 @@ bool Mpnn::apply(DeviceAmg& amg, const float* r, float* z, std::string& err, dou
     if (network_reduction) {
         const uint32_t rg = red_grid(n);
         sumsq2_kernel<<<rg, kBlock, 0, amg.stream()>>>(n, r, res, part_);
-        reduce_partials_kernel<<<1, 1024, 0, amg.stream()>>>(part_, rg, kMaxPartBlocks, 2, scal_ + 5);
+        reduce_partials_kernel<<<2, 1024, 0, amg.stream()>>>(part_, rg, kMaxPartBlocks, scal_ + 5, nullptr);
         double h[2] = {0.0, 0.0};
         MPNN_HIP(hipMemcpyAsync(h, scal_ + 5, sizeof(h), hipMemcpyDeviceToHost, amg.stream()));
         MPNN_HIP(hipStreamSynchronize(amg.stream()));
@@ -983,9 +1012,9 @@ bool Mpnn::train_step(DeviceAmg& amg, const float* r, const float* e, float lr, 
     axpy_kernel<<<g, kBlock, 0, st>>>(n, u, -1.0f, b, v);    // v = E u
     amg.spmv32(v, a);                                        // a = A v
     dot_partial_kernel<float><<<rg, kBlock, 0, st>>>(n, v, a, part_);
-    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, 1, scal_ + 2);
+    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, scal_ + 2, nullptr);
     dot_partial_kernel<float><<<rg, kBlock, 0, st>>>(n, e, r, part_);
-    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, 1, scal_ + 1);
+    reduce_partials_kernel<<<1, 1024, 0, st>>>(part_, rg, kMaxPartBlocks, scal_ + 1, nullptr);
     if (!amg.vcycle32(a, b)) {                               // b = V A v
         err = "training: V-cycle failed";
         return false;
@@ -1011,35 +1040,48 @@ struct Scoped {
 };
 }  // namespace
 
+// The host-vector entries' vectors stay with the object. The network works in
+// FP32, so the host converts the caller's doubles into pinned memory that the
+// reordering kernels read and write across the bus, and the call waits once, at
+// its end. (Pageable copies of the doubles and a device allocation per vector
+// and call, which waits for the device when it is freed, took 100 of the 445 us
+// of a 75k-node estimate and gradient.)
+namespace {
+template <class S, class D>
+void convert_host(uint32_t n, const S* from, D* to) {
+    auto run = [&](uint64_t b, uint64_t e, uint32_t) {
+        for (uint64_t i = b; i < e; ++i) to[i] = D(from[i]);
+    };
+    if (n < (1u << 20)) run(0, n, 0);  // below a millisecond: cheaper than starting threads
+    else parallel_chunks(n, 0, run);
+}
+}  // namespace
+
 void mpnn_forward_host(Mpnn& m, DeviceAmg& amg, const double* r, double* e) {
     const uint32_t n = amg.level0().n;
     hipStream_t st = amg.stream();
-    Scoped rd(size_t(n) * 8), rs(size_t(n) * 4), es(size_t(n) * 4);
-    MPNN_HIP(hipMemcpy(rd.p, r, size_t(n) * 8, hipMemcpyHostToDevice));
-    scatter_perm_kernel<double, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), rd.as<double>(),
-                                                                     rs.as<float>());
-    m.forward(amg, rs.as<float>(), es.as<float>(), false);
-    gather_perm_kernel<float, double><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), es.as<float>(),
-                                                                    rd.as<double>());
+    const Mpnn::HostVectors& v = m.host_vectors(n);
+    convert_host(n, r, v.h[0]);
+    scatter_perm_kernel<float, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), v.d[0], v.r);
+    m.forward(amg, v.r, v.e, false);
+    gather_perm_kernel<float, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), v.e, v.d[1]);
     MPNN_HIP(hipStreamSynchronize(st));
-    MPNN_HIP(hipMemcpy(e, rd.p, size_t(n) * 8, hipMemcpyDeviceToHost));
+    convert_host(n, v.h[1], e);
 }
 
 void mpnn_vjp_host(Mpnn& m, DeviceAmg& amg, const double* r, const double* ge, float* grad) {
     const uint32_t n = amg.level0().n;
     hipStream_t st = amg.stream();
-    Scoped rd(size_t(n) * 8), rs(size_t(n) * 4), gs(size_t(n) * 4), es(size_t(n) * 4), gd(kMpnnParams * 4);
-    MPNN_HIP(hipMemcpy(rd.p, r, size_t(n) * 8, hipMemcpyHostToDevice));
-    scatter_perm_kernel<double, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), rd.as<double>(),
-                                                                     rs.as<float>());
+    const Mpnn::HostVectors& v = m.host_vectors(n);
+    convert_host(n, r, v.h[0]);
+    scatter_perm_kernel<float, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), v.d[0], v.r);
+    m.forward(amg, v.r, v.e, true);
+    convert_host(n, ge, v.h[1]);
+    scatter_perm_kernel<float, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), v.d[1], v.g);
+    m.backward(amg, v.g, v.grad);
+    MPNN_HIP(hipMemcpyAsync(v.hgrad, v.grad, kMpnnParams * sizeof(float), hipMemcpyDeviceToHost, st));
     MPNN_HIP(hipStreamSynchronize(st));
-    MPNN_HIP(hipMemcpy(rd.p, ge, size_t(n) * 8, hipMemcpyHostToDevice));
-    scatter_perm_kernel<double, float><<<grid_of(n), kBlock, 0, st>>>(n, amg.device_perm0(), rd.as<double>(),
-                                                                     gs.as<float>());
-    m.forward(amg, rs.as<float>(), es.as<float>(), true);
-    m.backward(amg, gs.as<float>(), gd.as<float>());
-    MPNN_HIP(hipStreamSynchronize(st));
-    MPNN_HIP(hipMemcpy(grad, gd.p, kMpnnParams * 4, hipMemcpyDeviceToHost));
+    std::copy_n(v.hgrad, kMpnnParams, grad);
 }
 
 void mpnn_adam_host(Mpnn& m, const float* grad, float lr) {

@@ -46,6 +46,15 @@ public:
 
     int device() const { return device_; }
     // Parameters (flat layout above); setting them resets the Adam state.
+    // What the entries that take host vectors work on, for n nodes: pinned
+    // vectors h (d: their device addresses) and gradient, device vectors.
+    struct HostVectors {
+        float* h[2] = {nullptr, nullptr};
+        float* d[2] = {nullptr, nullptr};
+        float* hgrad = nullptr;
+        float *r = nullptr, *g = nullptr, *e = nullptr, *grad = nullptr;
+    };
+    const HostVectors& host_vectors(uint32_t n);
     void set_params(const float* host);
     void get_params(float* host) const;
 
@@ -78,6 +87,9 @@ private:
     void refresh_bf16(hipStream_t s);
 
     int device_ = 0;
+    HostVectors host_;
+    uint32_t host_cap_ = 0;
+    void free_host_vectors();
     uint32_t cap_ = 0;      // node capacity of the workspace
     const float* last_r_ = nullptr;  // input of the last forward(keep = true)
     // parameters and optimizer state (device, FP32)
