@@ -547,18 +547,24 @@ __global__ __launch_bounds__(kBlock) void decode_bwd_kernel(uint32_t n, const fl
 
 // Layer backward. In: gh = dL/dh_out, the layer's relu mask, h_prev.
 // Out: gh2 = gh + (dL/dX)[:, :32] (residual + self path), gm = (dL/dX)[:, 32:],
-// per-tile partials of dL/dW (X^T gz) and dL/db (sum gz).
+// per-tile partials of dL/dW (X^T gz) and dL/db (sum gz). Bound by the latency
+// of the neighbour gathers, so by the tiles resident: 23 KB of LDS a tile hold
+// six a CU, which takes the 1178 tiles of 75k nodes in one go (47 KB, with
+// dL/dX and the FP32 gz in places of their own, held three: 18.2 us
+// a layer, now 15.5).
 __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
     uint32_t n, const uint32_t* __restrict__ rowp, const uint32_t* __restrict__ cols, const float* __restrict__ vals,
     const float* __restrict__ s, const uint16_t* __restrict__ hprev, const uint32_t* __restrict__ mask,
     const uint16_t* __restrict__ w_g, const float* __restrict__ gh, float* __restrict__ gh2, float* __restrict__ gm,
     float* __restrict__ gpart, uint32_t layer_off) {
-    __shared__ __align__(16) uint16_t XT[2 * kHid * kLd];   // [f][node]
-    __shared__ __align__(16) uint16_t GZ[kTile * kLd32];    // [node][c]
-    __shared__ __align__(16) uint16_t GZT[kHid * kLd];      // [c][node]
+    constexpr int kXt = 2 * kHid * kLd, kGz = kTile * kLd32, kGzt = kHid * kLd, kG = kTile * (2 * kHid + 1);
     __shared__ __align__(16) uint16_t W[2 * kHid * kLd32];  // [f][c]
-    __shared__ float G[kTile * (2 * kHid + 1)];             // dL/dX [node][f]
-    __shared__ float GF[kTile * (kHid + 1)];                // FP32 gz [node][c]
+    __shared__ float GB[4 * kHid];                          // per-wavefront column sums of gz
+    __shared__ __align__(16) uint16_t tile[std::max(kXt + kGz + kGzt, 2 * kG)];
+    uint16_t* XT = tile;                        // [f][node]
+    uint16_t* GZ = tile + kXt;                  // [node][c]
+    uint16_t* GZT = tile + kXt + kGz;           // [c][node]
+    float* G = reinterpret_cast<float*>(tile);  // dL/dX [node][f], in their place once both products are formed
     const int tid = threadIdx.x;
     const uint32_t node0 = blockIdx.x * kTile;
     for (int e = tid; e < 2 * kHid * kHid; e += kBlock) W[(e >> 5) * kLd32 + (e & 31)] = w_g[e];
@@ -575,6 +581,7 @@ __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
         LoadF8{gh, uint32_t(q)}(i, ghv);
         mk = mask[i] >> (8 * q);
     }
+    float gzs[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         const int f = 8 * q + c;
@@ -584,18 +591,24 @@ __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
         const uint16_t gzb = f2bf(gz);
         GZ[il * kLd32 + f] = gzb;
         GZT[f * kLd + il] = gzb;
-        GF[il * (kHid + 1) + f] = gz;
+        gzs[c] = gz;
     }
-    __syncthreads();
     const int wave = tid >> 6, lane = tid & 63;
+    // dL/db: column sums of the FP32 gz, 16 nodes a wavefront, then wavefronts in order.
+#pragma unroll
+    for (int d = 4; d < 64; d <<= 1)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) gzs[c] += __shfl_xor(gzs[c], d);
+    if (lane < 4)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) GB[wave * kHid + 8 * q + c] = gzs[c];
+    __syncthreads();
     // dL/dX = GZ (64 x 32) * W^T (32 x 64): Bt[f][c] = W[f][c].
+    f32x4 dx[4];
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mfma_tile(GZ + wave * 16 * kLd32, kLd32, W + nt * 16 * kLd32, kLd32, kHid, acc);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            G[(wave * 16 + 4 * (lane >> 4) + j) * (2 * kHid + 1) + nt * 16 + (lane & 15)] = acc[j];
+        dx[nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        dx[nt] = mfma_tile(GZ + wave * 16 * kLd32, kLd32, W + nt * 16 * kLd32, kLd32, kHid, dx[nt]);
     }
     // dL/dW = X^T (64 x 64 nodes) * GZ (64 x 32): A = XT rows f, Bt = GZT rows c.
     float* out = gpart + size_t(blockIdx.x) * kMpnnParams + layer_off;
@@ -606,6 +619,13 @@ __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) out[(wave * 16 + 4 * (lane >> 4) + j) * kHid + nt * 16 + (lane & 15)] = acc[j];
     }
+    if (tid < kHid) out[2 * kHid * kHid + tid] = GB[tid] + GB[kHid + tid] + GB[2 * kHid + tid] + GB[3 * kHid + tid];
+    __syncthreads();
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            G[(wave * 16 + 4 * (lane >> 4) + j) * (2 * kHid + 1) + nt * 16 + (lane & 15)] = dx[nt][j];
     __syncthreads();
     if (i < n) {
         const float* gr = G + il * (2 * kHid + 1);
@@ -616,12 +636,6 @@ __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
         float4* om = reinterpret_cast<float4*>(gm + size_t(i) * kHid + 8 * q);
         om[0] = make_float4(gr[kHid + 8 * q], gr[kHid + 8 * q + 1], gr[kHid + 8 * q + 2], gr[kHid + 8 * q + 3]);
         om[1] = make_float4(gr[kHid + 8 * q + 4], gr[kHid + 8 * q + 5], gr[kHid + 8 * q + 6], gr[kHid + 8 * q + 7]);
-    }
-    // dL/db: column sums of the FP32 gz tile in node order.
-    if (tid < kHid) {
-        float tb = 0.0f;
-        for (int r = 0; r < kTile; ++r) tb += GF[r * (kHid + 1) + tid];
-        out[2 * kHid * kHid + tid] = tb;
     }
 }
 
@@ -674,7 +688,7 @@ __global__ __launch_bounds__(kBlock) void encode_bwd_kernel(uint32_t n, const fl
 // in row order. The parameter gradient is reduced in two such stages with a
 // fixed grouping (per = kGradChunk tiles, then all chunk sums), so the sum is
 // deterministic and the reduction has enough parallelism.
-constexpr uint32_t kGradChunk = 64;
+constexpr uint32_t kGradChunk = 24;
 __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(uint32_t rows, uint32_t per,
                                                             const float* __restrict__ gpart,
                                                             float* __restrict__ out) {
