@@ -982,7 +982,7 @@ bool DeviceAmg::fetch_scalars(uint32_t count, uint32_t first) {
 
 // Waits until the first `count` workgroups of the kernel launched last have
 // signalled ticket_. Polling pinned memory sees them sooner than a stream synchronisation
-// (17 FGMRES steps on 75k rows: 3780 us so, 3890 that way); a launch that takes
+// (17 FGMRES steps on 70k rows: 3780 us so, 3890 that way); a launch that takes
 // longer than some milliseconds, or fails, is left to the runtime.
 void DeviceAmg::await(int count) {
     const volatile unsigned long long* done = h_done_;
@@ -1015,7 +1015,8 @@ namespace {
 template <class T>
 __global__ __launch_bounds__(kBlock) void apply_in_kernel(uint32_t n, const uint32_t* __restrict__ new_of_old,
                                                          const double* __restrict__ r, T* __restrict__ out,
-                                                         uint32_t call, uint32_t* __restrict__ bad,
+                                                         unsigned long long call,
+                                                         unsigned long long* __restrict__ bad,
                                                          int* __restrict__ seen) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
@@ -1032,7 +1033,8 @@ __global__ __launch_bounds__(kBlock) void apply_in_kernel(uint32_t n, const uint
 template <class T>
 __global__ __launch_bounds__(kBlock) void apply_out_kernel(uint32_t n, const uint32_t* __restrict__ new_of_old,
                                                           const T* __restrict__ z, double* __restrict__ out,
-                                                          uint32_t call, const uint32_t* __restrict__ bad,
+                                                          unsigned long long call,
+                                                          const unsigned long long* __restrict__ bad,
                                                           int* __restrict__ seen) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n || *bad == call) return;
@@ -1090,8 +1092,8 @@ bool DeviceAmg::apply_caller(const double* r_caller, double* z_caller, bool fp32
     // out, read by the host; *bad: the number of the last call that was refused.
     int* seen = reinterpret_cast<int*>(h_scal_ + kScalars - 1);
     int* d_seen = reinterpret_cast<int*>(scal_host_ + kScalars - 1);
-    uint32_t* bad = reinterpret_cast<uint32_t*>(scal_ + kScalars - 1);
-    const uint32_t call = ++apply_calls_;
+    unsigned long long* bad = reinterpret_cast<unsigned long long*>(scal_ + kScalars - 1);
+    const unsigned long long call = ++apply_calls_;
     const_cast<volatile int*>(seen)[0] = const_cast<volatile int*>(seen)[1] = 0;
     auto flagged = [&](int k) { return const_cast<volatile int*>(seen)[k] != 0; };
     const bool bounded = max_image_ratio > 0.0;
@@ -1361,7 +1363,7 @@ inline uint32_t gs_tiles(uint32_t j) { return j == 0 ? 1u : (j + kGsTile - 1) / 
 //   partials[2j + 2]   = w . w
 // blockIdx.y takes kGsTile basis vectors; the sums of a workgroup are formed by
 // wavefronts, stored, and closed by one thread a sum (one block sum after the
-// other, two barriers each, took 10.9 us a step of 75k rows,
+// other, two barriers each, took 10.9 us a step of 70k rows,
 // averaged over a cycle of 17; 9.1 us so, most of it the loads).
 __global__ __launch_bounds__(kBlock) void gs_dot_kernel(uint32_t npairs, size_t ld, uint32_t j,
                                                        const double* __restrict__ V, const double* __restrict__ w,

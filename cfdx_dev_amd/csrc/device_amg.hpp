@@ -452,7 +452,7 @@ private:
     double* h_scal_ = nullptr;      // pinned host mirror
     unsigned long long *h_done_ = nullptr, *done_ = nullptr, ticket_ = 0;  // tickets of awaited kernels (pinned)
     void await(int count);
-    uint32_t apply_calls_ = 0;
+    unsigned long long apply_calls_ = 0;
     bool apply_bounded(const double* r, double* z, const int* seen, std::string& err);
     double* scal_host_ = nullptr;  // h_scal_ as the device addresses it
     std::vector<double*> work_;     // generic FP64 n-vectors
