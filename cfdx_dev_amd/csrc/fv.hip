@@ -12,11 +12,11 @@
 //   corrector assembly               :8048-8181, CSR + gauge :8599-8652
 //   scalar diffusion assembly        core/solvers/scalar_diffusion.h:39-163
 //
-// Face kernels compute per-face quantities once; cell kernels gather them
-// over the cell->face lists. The reference accumulates the diagonal and the
-// boundary sources in global face order; cells list their faces in ascending
-// face id, so the gather visits them in that same order and every value is
-// bit-identical to the reference (FMA contraction is off). No atomics.
+// The assemblies take one row a thread and evaluate every face from both of its
+// cells. The reference accumulates the diagonal and the boundary sources in
+// global face order; a row visits its cell's faces in ascending face id, so
+// every value is bit-identical to the reference (FMA contraction is off). No
+// atomics.
 
 #include "fv.hpp"
 
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
 
 // Cells go to workgroups by xcd_block: each XCD takes one contiguous range, so
 // that the records a cell and its neighbours share are fetched into one L2
-// rather than into most of them (a 222k-cell channel's pressure rows: 40 us in
+// rather than into most of them (a 232k-cell channel's pressure rows: 40 us in
 // launch order, 31 so).
 __device__ __forceinline__ uint32_t cell_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
@@ -738,9 +738,9 @@ __global__ __launch_bounds__(kBlock) void gather_u8_kernel(uint64_t n, const uin
 // The three velocity components share the flux, the viscosity and the
 // boundary-condition types, so their matrices are identical: one value array
 // (and one diagonal) serves all three, each component keeping its own RHS.
-// Face kernels compute per-face terms once; cell kernels gather them in
-// ascending face order, the order of the reference's global face loop, so the
-// per-cell sums are bit-identical (FMA contraction is off).
+// A row visits its cell's faces in ascending order, the order of the reference's
+// global face loop, so the per-cell sums are bit-identical (FMA contraction is
+// off).
 
 constexpr int kMaxCellFaces = 10;  // WLS stencil: one sample per cell face
 
@@ -957,8 +957,8 @@ __global__ __launch_bounds__(kBlock) void wls_build_kernel(uint32_t nc, const ui
 // records a cell; boundary types are 0 and 1, for which finite samples make a
 // finite Green-Gauss sum, so only cells whose fit is refused take that pass and
 // the others read neither area vectors nor weights: bound by the 36 bytes of
-// fit a slot (80^3 cells: 72 us; 136 with both passes and gathers from memory). gate: skip the whole pass unless
-// diffusion is active.
+// fit a slot (80^3 cells: 72 us; 136 with both passes and gathers from memory).
+// gate: skip the whole pass unless diffusion is active.
 template <int K>
 __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
     uint32_t nc, const uint32_t* __restrict__ coff, Slots sl, const uint32_t* __restrict__ patch, uint32_t npatch,
@@ -1691,7 +1691,7 @@ void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy
     // touch about as few lines in it as on the curve (at most half as many
     // again): then no field is permuted at all.
     // Lexicographic numberings of boxes and channels touch 1.05 times the
-    // curve's lines, random ones 9 times. A 222k-cell channel kept as numbered
+    // curve's lines, random ones 9 times. A 232k-cell channel kept as numbered
     // assembles its pressure in 98 us, moved to another local order in 112 (its
     // six fields pass through a gather); a random 128^3 box assembled as
     // numbered would fetch a line for each of its 66M values.
@@ -2150,7 +2150,10 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
     double4* rec = reinterpret_cast<double4*>(scr(5, 4 * uint64_t(nc)));
     pack_cells_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, identity_order ? nullptr : cell_new, d_rAU, d_p, rec);
     const double* phi_i = fin(d_phi, 4);
-    gauss_gradient_internal(d_pbt, d_pbv, &rec->w, 4);
+    // A kept numbering has p at hand as an array of its own: a quarter of the
+    // lines (256^3 cells in lattice order: 885 us, 1030 from records).
+    if (identity_order) gauss_gradient_internal(d_pbt, d_pbv, d_p, 1);
+    else gauss_gradient_internal(d_pbt, d_pbv, &rec->w, 4);
     const RowMap rm{plan.row_start, plan.row_of, plan.slot_rank, plan.diag_rank, plan.shared_pairs ? 1 : 0};
     const double4* grad = reinterpret_cast<const double4*>(work_grad);
     if (slot_D <= kRowSlots) {
@@ -2220,7 +2223,7 @@ void FvMesh::ensure_momentum_work() {
 // pressure type], written by the host into pinned memory and fetched by one
 // small kernel, which also clears the call's device flags. Pressure types other
 // than 1 read as zero-gradient unless raw_pbt. (Two copies of a few
-// bytes and a fill took 10 us of a 222k-cell pressure assembly's 90.)
+// bytes and a fill took 10 us of a 232k-cell pressure assembly's 90.)
 void FvMesh::upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv,
                         bool raw_pbt, int* flags) {
     const size_t npp = std::max<uint32_t>(npatch, 1);
