@@ -247,6 +247,15 @@ class NativeAMGPreconditioner:
             raise RuntimeError(self.last_error())
         return d.value, u.value
 
+    def coarse_end(self) -> int:
+        """First level that the FP64 V-cycle runs in its single-launch coarse
+        end (num_levels(): none)."""
+        v = C.c_size_t()
+        st = self._lib.cfdxhip_amg_coarse_end(self._h, C.byref(v))
+        if st != 0:
+            raise RuntimeError(f"cfdxhip_amg_coarse_end failed with status {st}")
+        return v.value
+
     def level_spmv_format(self, level: int):
         """(format, stored_entries, slices) of the storage a level's device
         SpMV streams: "csr" (stored_entries = nnz) or "sell64" (slots of

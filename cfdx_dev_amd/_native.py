@@ -171,6 +171,7 @@ def load():
          [vp, C.c_size_t, C.c_uint32, C.c_uint32, C.c_uint32, C.POINTER(C.c_double)])
     _sig(lib, "cfdxhip_amg_gram_schmidt_seconds", st,
          [vp, C.c_uint32, C.c_uint32, C.POINTER(C.c_double), C.POINTER(C.c_double)])
+    _sig(lib, "cfdxhip_amg_coarse_end", st, [vp, C.POINTER(C.c_size_t)])
     _sig(lib, "cfdxhip_amg_level_spmv_format", st,
          [vp, C.c_size_t, C.POINTER(C.c_uint32), C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)])
     _sig(lib, "cfdxhip_amg_level_spmv_bytes", st, [vp, C.c_size_t, C.c_uint32, C.POINTER(C.c_uint64)])

@@ -919,6 +919,13 @@ cfdxhip_status cfdxhip_amg_gram_schmidt_seconds(cfdxhip_amg* h, uint32_t j, uint
     });
 }
 
+cfdxhip_status cfdxhip_amg_coarse_end(const cfdxhip_amg* h, size_t* first_level) {
+    if (!h || !first_level) return CFDXHIP_ERR_INVALID_ARGUMENT;
+    if (!h->ready || !h->dev) return CFDXHIP_ERR_NOT_READY;
+    *first_level = h->dev->coarse_end_level();
+    return CFDXHIP_OK;
+}
+
 cfdxhip_status cfdxhip_amg_level_spmv_format(const cfdxhip_amg* h, size_t level, uint32_t* format,
                                              uint64_t* stored_entries, uint64_t* slices) {
     if (!h || !format || !stored_entries || !slices) return CFDXHIP_ERR_INVALID_ARGUMENT;

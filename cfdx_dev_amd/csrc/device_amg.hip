@@ -248,6 +248,7 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
     post_ = cfg.post;
     has64_ = want64;
     has32_ = want32;
+    cns_ = cfg.constant_null_space;
     smoother64_ = cfg.smoother64;
     smoother32_ = cfg.smoother32;
     cheb_degree_ = cfg.cheb_degree;
@@ -397,7 +398,6 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
     partial_stride_ = std::max<uint64_t>({spmv_groups<double>(lv_[0].A), spmv_groups<float>(lv_[0].A), 4096});
     partials_ = dalloc<double>(std::max<uint64_t>(partial_stride_ * 8, uint64_t(kGsStride) * (2 * kRestartMax + 3)));
     aux_part_ = dalloc<double>(4096);
-    cns_ = cfg.constant_null_space;
     if (cns_) {
         if (has64_) cns_r64_ = dalloc<double>(lv_[0].n);
         if (has32_) cns_r32_ = dalloc<float>(lv_[0].n);

@@ -337,6 +337,9 @@ public:
     // sweep (kind 1) on the level's own buffers (x = b = 1), HIP events.
     size_t num_levels() const { return lv_.size(); }
     const DevCsr& level_matrix(size_t l) const { return lv_[l].A; }
+    // First level of the FP64 V-cycle's single-launch coarse end (the number
+    // of levels: none).
+    uint32_t coarse_end_level() const { return tail_.first; }
     bool level_kernel_seconds(uint32_t level, uint32_t precision, uint32_t kind, uint32_t repeat, double& sec,
                               std::string& err);
     // Seconds per launch of the Gram-Schmidt passes of Arnoldi step j.

@@ -298,6 +298,9 @@ cfdxhip_status cfdxhip_amg_level_kernel_seconds(cfdxhip_amg* h, size_t level, ui
  * basis values. No reference counterpart. */
 cfdxhip_status cfdxhip_amg_gram_schmidt_seconds(cfdxhip_amg* h, uint32_t j, uint32_t repeat, double* dot_seconds,
                                                 double* update_seconds);
+/* First level that the FP64 V-cycle runs in its single-launch coarse end (the
+ * number of levels: none). Diagnostics only. No reference counterpart. */
+cfdxhip_status cfdxhip_amg_coarse_end(const cfdxhip_amg* h, size_t* first_level);
 /* Storage the device SpMV of a level's matrix streams: format 0 = CSR
  * stream (stored_entries = nnz, slices = 0), 1 = SELL-64 (slices of 64 rows,
  * stored_entries = slots including padding). Measurement only: the byte

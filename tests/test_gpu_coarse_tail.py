@@ -8,12 +8,14 @@ for bit, where it can go wrong:
 * a coarsest level without dense factors (24 sweeps), policies of 2 and 6
   sweeps, Chebyshev smoothing with a recurrence;
 * after a numeric refresh (packed values, damping and coefficients renewed).
+A hierarchy with the constant null space, whose mean removals are launches
+between the sweeps, keeps the launches.
 """
 import numpy as np
 import pytest
 
 import cfdx_dev_amd as cx
-from systems import box_mesh, channel_system, pressure_system
+from systems import box_mesh, channel_system, neumann_system, pressure_system
 from test_poisson_mms import mms_system
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +52,11 @@ def test_coarse_end_bit_identical(oracle, name):
         for _ in range(2):
             r = rng.normal(size=s["n"])
             assert np.array_equal(ao.apply(r), ap.apply(r))
+
+
+@pytest.mark.parametrize("method,dims", [("sa", (8, 7, 6)), ("sa", (20, 18, 16)), ("boomer", (14, 12, 11))])
+def test_null_space_keeps_the_launches(oracle, method, dims):
+    s = neumann_system(oracle, box_mesh(*dims, jitter=0.15, seed=6), seed=6)
+    h = cx.NativeAMGPreconditioner(method=method, constant_null_space=True)
+    assert h.setup(s["n"], s["rowp"], s["cols"], s["vals"]), h.last_error()
+    assert h.num_levels() > 2 and h.coarse_end() == h.num_levels()
