@@ -184,9 +184,9 @@ __global__ __launch_bounds__(kBlock) void cell_volume_kernel(uint32_t nc, const 
 // instead of gathering the face and neighbour-cell arrays face by face.
 //   other: the cell across an internal face, -1 for a boundary face, -2 for
 //          an EMPTY face or an unused slot;
-//   face:  the face; the top bit is set on the neighbour's side of an internal
-//          face (a boundary face's entry is the plain id; 2^31 faces are
-//          beyond what the slots of a mesh could be stored for);
+//   face:  the face; the top bit is set on the side of a cell that does not
+//          own it (also where such a cell lists a boundary face, which the
+//          mesh's addressing admits): face_of() makes it an index;
 //   w:     the distance weight dn / (dc + dn) of an internal face (the
 //          Green-Gauss face interpolation);
 //   s:     the face area vector oriented out of the cell.
@@ -196,6 +196,8 @@ struct Slots {
     uint32_t* face;
     double* w;
     Soa3 s;
+
+    __device__ __forceinline__ static uint32_t face_of(uint32_t entry) { return entry & ~kFaceReversed; }
 };
 
 __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_t D, const uint32_t* __restrict__ coff,
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(kBlock) void gauss_gradient_kernel(
             if (o[j] >= 0) {
                 vf = w[j] * pc + (1.0 - w[j]) * po[j];
             } else {
-                const uint32_t f = sl.face[size_t(q0 + j) * nc + c];
+                const uint32_t f = sl.face_of(sl.face[size_t(q0 + j) * nc + c]);
                 const uint32_t pp = patch[f];
                 if (pp < npatch) {
                     if (bct[pp] == 1) {
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(kBlock) void pressure_row_kernel(
 #pragma unroll
         for (uint32_t j = 0; j < kRowBatch; ++j) {
             const uint32_t n = o[j] >= 0 ? uint32_t(o[j]) : c;
-            ph[j] = phi[f[j] & ~kFaceReversed];
+            ph[j] = phi[sl.face_of(f[j])];
             if (kLds && near.has(n)) {
                 Cn[j] = near.get(0, n);
                 An[j] = near.get(1, n);
@@ -558,7 +560,7 @@ __global__ __launch_bounds__(kBlock) void pressure_row_kernel(
                 cf = rho * ic;
                 cont -= rho * (ic * (An[j].w - A.w) + nof);
             } else {
-                const uint32_t pp = patch[f[j]];
+                const uint32_t pp = patch[sl.face_of(f[j])];
                 fixed |= pp < npatch && pbt[pp] == 1;
             }
             cbuf[(q0 + j) * cs] = cf;
@@ -589,7 +591,7 @@ __global__ __launch_bounds__(kBlock) void pressure_row_kernel(
         for (uint32_t k = 0; k < deg; ++k) {
             const size_t idx = size_t(slot_sorted[size_t(k) * nc + c]) * nc + c;
             if (sl.other[idx] >= 0) continue;
-            const uint32_t f = sl.face[idx];
+            const uint32_t f = sl.face_of(sl.face[idx]);
             const uint32_t pp = patch[f];
             if (!(pp < npatch && pbt[pp] == 1)) continue;
             double bc = 0.0, def = 0.0;
@@ -812,7 +814,7 @@ __global__ __launch_bounds__(kBlock) void wls_build_kernel(uint32_t nc, const ui
             pt = cc.get(uint32_t(o));
             wc.nd[idx] = 0.0;
         } else {
-            const uint32_t f = sl.face[idx];
+            const uint32_t f = sl.face_of(sl.face[idx]);
             const uint32_t pp = patch[f];
             const uint8_t t = pp < npatch ? bct[pp] : 0;
             const D3 sf = sl.s.get(idx);
@@ -1022,7 +1024,7 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
 #pragma unroll
                 for (int k = 0; k < K; ++k) fv[k] = w * value[k] + (1.0 - w) * other[k];
             } else {
-                const uint32_t f = sl.face[idx];
+                const uint32_t f = sl.face_of(sl.face[idx]);
                 const uint32_t pp = patch[f];
                 const uint8_t t = pp < npatch ? bct[pp] : 0;
                 double dn = 0.0;
@@ -1086,7 +1088,7 @@ __global__ __launch_bounds__(kBlock) void wls_gradient_kernel(
             if (o >= 0) {
                 sample(uint32_t(o), sv);
             } else {
-                const uint32_t pp = patch[sl.face[idx]];
+                const uint32_t pp = patch[sl.face_of(sl.face[idx])];
                 const uint8_t t = pp < npatch ? bct[pp] : 0;
                 const double nd = wc.nd[idx];
 #pragma unroll
@@ -1233,7 +1235,7 @@ __global__ __launch_bounds__(kBlock) void momentum_row_kernel(
     for (uint32_t k = 0; k < deg; ++k) {
         const size_t at = idx;
         const int32_t o = o1;
-        const uint32_t fr = f1, f = fr & ~kFaceReversed;
+        const uint32_t fr = f1, f = sl.face_of(fr);
         const bool reversed = fr != f;
         const double Fo = phi[f];
         const D3 Sf = sl.s.get(at), Cf = fc.get(f);
@@ -1898,6 +1900,7 @@ void FvMesh::ensure_slots() {
     uint32_t D = 0;
     for (uint32_t c = 0; c < nc; ++c) D = std::max(D, h_coff[c + 1] - h_coff[c]);
     if (D > 255) throw std::invalid_argument("cells with more than 255 faces are not supported");
+    if (nf > kFaceReversed) throw std::invalid_argument("cell stencils: more than 2^31 faces are not supported");
     slot_D = D;
     const uint64_t m = uint64_t(D) * nc;
     cell_rec = dalloc<double4>(nc);
