@@ -1585,7 +1585,12 @@ WlsCache wls_of(const FvMesh& m) {
 }  // namespace
 
 void PressurePlan::release() {
-    for (uint32_t** p : {&rowp, &cols, &nz_row_diag, &nzf_off, &nzf, &row_start, &row_of}) dfree(*p);
+    for (uint32_t** p : {&rowp, &cols, &nz_row_diag, &nzf_off, &nzf}) dfree(*p);
+    release_maps();
+}
+
+void PressurePlan::release_maps() {
+    for (uint32_t** p : {&row_start, &row_of}) dfree(*p);
     for (uint16_t** p : {&slot_rank, &diag_rank}) dfree(*p);
 }
 
@@ -1594,7 +1599,7 @@ FvMesh::~FvMesh() { release(); }
 void FvMesh::release() {
     for (double** p : {&px, &py, &pz, &fcx, &fcy, &fcz, &fsx, &fsy, &fsz, &ccx, &ccy, &ccz, &vol, &vol_caller,
                        &work_coeff, &work_bsrc, &work_diag, &work_rhs, &work_grad, &work_phi,
-                       &mom_ugrad, &bc_f64, &slot_coeff, &slot_w, &slot_sx, &slot_sy, &slot_sz,
+                       &mom_ugrad, &bc_f64, &slot_coeff,
                        &wls_a0, &wls_a1, &wls_a2, &wls_fac, &wls_nd, &wls_sig, &wls_V, &wls_cond})
         dfree(*p);
     for (uint32_t** p : {&foff, &fvtx, &owner, &coff, &cfaces, &cfaces_sorted, &patch, &cell_new, &cell_old,
@@ -1603,10 +1608,7 @@ void FvMesh::release() {
     for (auto& b : scratch) dfree(b.first);
     scratch.clear();
     dfree(scratch_u8);
-    dfree(slot_other);
-    dfree(cell_rec);
-    dfree(slot_sorted);
-    dfree(slot_face);
+    release_slots();
     dfree(wls_meta);
     dfree(neigh);
     dfree(patch_kind);
@@ -1896,13 +1898,14 @@ void FvMesh::ensure_work() {
 
 // Slot stencils (geometry only): built on first use.
 void FvMesh::ensure_slots() {
-    if (slot_other) return;
+    if (slots_built) return;
     uint32_t D = 0;
     for (uint32_t c = 0; c < nc; ++c) D = std::max(D, h_coff[c + 1] - h_coff[c]);
     if (D > 255) throw std::invalid_argument("cells with more than 255 faces are not supported");
     if (nf > kFaceReversed) throw std::invalid_argument("cell stencils: more than 2^31 faces are not supported");
     slot_D = D;
     const uint64_t m = uint64_t(D) * nc;
+    release_slots();  // of an attempt that failed
     cell_rec = dalloc<double4>(nc);
     slot_other = dalloc<int32_t>(m);
     slot_face = dalloc<uint32_t>(m);
@@ -1933,6 +1936,16 @@ void FvMesh::ensure_slots() {
                                                            patch_kind, fc, fs, cc, vol, cell_rec, slots_of(*this), err);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("cell stencils: degenerate face distances");
+    slots_built = true;
+}
+
+void FvMesh::release_slots() {
+    slots_built = false;
+    for (double** p : {&slot_w, &slot_sx, &slot_sy, &slot_sz}) dfree(*p);
+    dfree(slot_other);
+    dfree(slot_face);
+    dfree(slot_sorted);
+    dfree(cell_rec);
 }
 
 // WLS fit cache for one set of boundary types (fixed value or not, per patch).
@@ -1996,6 +2009,7 @@ void FvMesh::mass_flux_device(const uint8_t* d_vbt, const double* d_vbv, double 
 const PressurePlan& FvMesh::pressure_plan(bool eliminate, uint32_t ref) {
     PressurePlan& full = pressure_full;
     if (!full.rowp) {
+        full.release();  // of an attempt that failed
         // Row c: {c} and the other cell of each internal face of c, sorted,
         // duplicates (several faces joining one pair) merged with their faces
         // listed in ascending face id. Two passes over the cell->face lists.
@@ -2057,13 +2071,12 @@ const PressurePlan& FvMesh::pressure_plan(bool eliminate, uint32_t ref) {
         full.nnz = nnz;
         full.h_rowp = std::move(rowp);
         full.h_cols = std::move(cols);
-        full.rowp = upload(full.h_rowp.data(), full.h_rowp.size());
+        full.shared_pairs = nnz != uint64_t(nc) + fcnt[nc];
         full.cols = upload(full.h_cols.data(), full.h_cols.size());
         full.nz_row_diag = upload(rdiag.data(), rdiag.size());
         full.nzf_off = upload(nzf_off.data(), nzf_off.size());
         full.nzf = upload(nzf.data(), nzf.size());
-        full.shared_pairs = nnz != uint64_t(nc) + fcnt[nc];
-        map_rows(full, 0xffffffffu);
+        full.rowp = upload(full.h_rowp.data(), full.h_rowp.size());  // last: the plan is whole
     }
     if (!eliminate) return full;
     PressurePlan& red = pressure_red;
@@ -2086,11 +2099,19 @@ const PressurePlan& FvMesh::pressure_plan(bool eliminate, uint32_t ref) {
         red.h_rowp = std::move(rowp);
         red.h_cols = std::move(cols);
         red.shared_pairs = full.shared_pairs;
-        red.rowp = upload(red.h_rowp.data(), red.h_rowp.size());
         red.cols = upload(red.h_cols.data(), red.h_cols.size());
-        map_rows(red, ref);
+        red.rowp = upload(red.h_rowp.data(), red.h_rowp.size());
     }
     return red;
+}
+
+// The plan with its row maps, which only the assemblies need: the pattern and
+// the calls that read nothing else take meshes that have no slot stencils.
+const PressurePlan& FvMesh::row_plan(bool eliminate, uint32_t ref) {
+    pressure_plan(eliminate, ref);
+    PressurePlan& plan = eliminate ? pressure_red : pressure_full;
+    if (!plan.row_start) map_rows(plan, eliminate ? ref : 0xffffffffu);
+    return plan;
 }
 
 // Where each internal cell's slots land in the rows of plan (row and column
@@ -2125,10 +2146,11 @@ void FvMesh::map_rows(PressurePlan& plan, uint32_t ref) {
             }
         }
     });
-    plan.row_start = upload(start.data(), nc);
+    plan.release_maps();  // of an attempt that failed
     plan.row_of = upload(row.data(), nc);
     plan.slot_rank = upload(rank.data(), rank.size());
     plan.diag_rank = upload(diag.data(), nc);
+    plan.row_start = upload(start.data(), nc);  // last: the maps are whole
 }
 
 bool FvMesh::has_fixed_pressure(const uint8_t* h_pbt) const {
@@ -2143,7 +2165,7 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
     ensure_work();
     const bool fixed = has_fixed_pressure(h_pbt);
     const bool eliminate = !fixed && nc > 1 && ref < nc;
-    const PressurePlan& plan = pressure_plan(eliminate, uint32_t(eliminate ? ref : 0));
+    const PressurePlan& plan = row_plan(eliminate, uint32_t(eliminate ? ref : 0));
     upload_bcs(nullptr, nullptr, h_pbt, h_pbv, true, nullptr);
     const uint32_t npp = std::max<uint32_t>(npatch, 1);
     const uint8_t* d_pbt = bc_u8 + npp;
@@ -2206,7 +2228,7 @@ const PressurePlan& FvMesh::diffusion_assemble_device(double gamma, const double
 void FvMesh::ensure_momentum_work() {
     if (mom_flags) return;
     ensure_slots();
-    mom_ugrad = dalloc<double>(12 * uint64_t(nc));
+    if (!mom_ugrad) mom_ugrad = dalloc<double>(12 * uint64_t(nc));
     // Which patches (last: the internal faces) hold non-orthogonal faces, and
     // which ones faces that do not say: geometry, so found once.
     const uint32_t nflag = 2 * (npatch + 1);
@@ -2291,7 +2313,7 @@ const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const
                                                      const double* d_body, const double* d_U, bool bounded,
                                                      double alpha, double* d_vals, double* d_rhs, double* d_diag) {
     if (!(alpha > 0.0 && alpha <= 1.0)) throw std::invalid_argument("relax_momentum_equation: invalid relaxation");
-    const PressurePlan& plan = pressure_plan(false, 0);
+    const PressurePlan& plan = row_plan(false, 0);
     ensure_momentum_work();
     upload_bcs(h_vbt, h_vbv, nullptr, nullptr, false, mom_flags);
     const uint8_t* d_vbt = bc_u8;

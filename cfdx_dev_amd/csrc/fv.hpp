@@ -30,6 +30,7 @@ struct PressurePlan {
     bool shared_pairs = false;  // some pair of cells is joined by several faces
 
     void release();
+    void release_maps();
 };
 
 struct FvMesh {
@@ -77,6 +78,7 @@ struct FvMesh {
     std::vector<uint8_t> h_patch_boundary;  // per patch: owns at least one boundary face
     // slot stencils (slot-major, slot_D slots per cell) and the WLS fit cache
     uint32_t slot_D = 0;
+    bool slots_built = false;
     uint8_t* slot_sorted = nullptr;  // per cell, its slots in ascending caller face id
     int32_t* slot_other = nullptr;
     double4* cell_rec = nullptr;  // (centre, volume) per cell
@@ -104,6 +106,7 @@ struct FvMesh {
     void gauss_gradient_device(const uint8_t* d_bct, const double* d_bcv, const double* d_p, double* d_grad);
     void mass_flux_device(const uint8_t* d_vbt, const double* d_vbv, double rho, const double* d_U, double* d_phi);
     const PressurePlan& pressure_plan(bool eliminate, uint32_t ref);
+    const PressurePlan& row_plan(bool eliminate, uint32_t ref);
     bool has_fixed_pressure(const uint8_t* h_pbt) const;
     const PressurePlan& pressure_assemble_device(const uint8_t* h_pbt, const double* h_pbv, double rho,
                                                  const double* d_rAU, const double* d_phi, const double* d_p,
@@ -139,6 +142,7 @@ struct FvMesh {
     double* cout_buf(double* caller, size_t slot, int comps);
     double* fout_buf(double* caller, size_t slot);
     void ensure_slots();
+    void release_slots();
     void ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt);
     void gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps);
     void map_rows(PressurePlan& plan, uint32_t ref);
