@@ -774,14 +774,25 @@ cfdxhip_status cfdxhip_amg_set_chebyshev_levels(cfdxhip_amg* h, uint32_t degree,
                     "Chebyshev degree must be in [1, 16], the coarse degree in [0, 16], and ratio > 1");
     if (!h->ready || h->host.lambda_max.empty())
         return fail(h, CFDXHIP_ERR_NOT_READY, "no Chebyshev smoother configured on a set-up hierarchy");
-    h->opt.chebyshev_degree = degree;
-    h->opt.chebyshev_degree_coarse = degree_coarse;
-    h->opt.chebyshev_ratio = ratio;
-    h->cfg.cheb_degree = degree;
-    h->cfg.cheb_degree_coarse = degree_coarse;
-    h->cfg.cheb_ratio = ratio;
-    if (h->dev) h->dev->set_chebyshev_params(h->host, degree, degree_coarse, ratio);
-    return CFDXHIP_OK;
+    return guarded(h, [&]() {
+        if (h->dev) {
+            hip_check(hipSetDevice(h->opt.device), "hipSetDevice");
+            try {
+                h->dev->set_chebyshev_params(h->host, degree, degree_coarse, ratio);
+            } catch (...) {
+                // The device's coefficients may be the old ones.
+                h->ready = false;
+                throw;
+            }
+        }
+        h->opt.chebyshev_degree = degree;
+        h->opt.chebyshev_degree_coarse = degree_coarse;
+        h->opt.chebyshev_ratio = ratio;
+        h->cfg.cheb_degree = degree;
+        h->cfg.cheb_degree_coarse = degree_coarse;
+        h->cfg.cheb_ratio = ratio;
+        return CFDXHIP_OK;
+    });
 }
 
 cfdxhip_status cfdxhip_amg_set_chebyshev(cfdxhip_amg* h, uint32_t degree, double ratio) {
