@@ -2464,7 +2464,7 @@ __device__ __forceinline__ void accumulate_faces(uint64_t nf, uint64_t nc, const
     auto add = [&](uint64_t cell, int c, double v) {
         const uint64_t w = cell - base;
         if (w < width) unsafeAtomicAdd(&win[c][w], v);
-        else unsafeAtomicAdd(out[c] + cell, v);
+        else atomicAdd(out[c] + cell, v);
     };
 #pragma unroll
     for (uint32_t k = 0; k < kFacePer; ++k) {
@@ -2483,7 +2483,7 @@ __device__ __forceinline__ void accumulate_faces(uint64_t nf, uint64_t nc, const
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const double v = win[c][w];
-            if (v != 0.0) unsafeAtomicAdd(out[c] + base + w, v);
+            if (v != 0.0) atomicAdd(out[c] + base + w, v);
         }
 }
 
