@@ -146,8 +146,8 @@ struct FvMesh {
     void ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt);
     void gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps);
     void map_rows(PressurePlan& plan, uint32_t ref);
-    uint64_t touched_lines(const std::vector<uint32_t>& at, const std::vector<uint32_t>& cell_place,
-                           const std::vector<uint32_t>& face_place) const;
+    uint64_t touched_lines(const uint32_t* at, const uint32_t* cell_place, const uint32_t* face_place,
+                           uint64_t* fewest) const;
     void check_err(const char* what);
     void release();
 };
