@@ -219,7 +219,7 @@ void DeviceAmg::release() {
     dfree(lu_.factor);
     dfree(lu_.upper);
     lu_ = DevCoarseLU{};
-    for (void* p : tail_.mem) (void)hipFree(p);
+    dfree(tail_.mem);
     tail_ = Tail{};
     dfree(d_perm0_);
     dfree(partials_);
@@ -303,9 +303,11 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
     phase("orderings");
     // ---- matrices
     std::vector<uint32_t> rowp, cols, src;
+    std::vector<TailPatterns> small(L);  // A, R, P of the levels the coarse end may take
     auto upload_csr = [&](DevCsr& D, const HCsr& H, const std::vector<uint32_t>& rp,
-                          const std::vector<uint32_t>& cp, uint32_t ncols) {
+                          const std::vector<uint32_t>& cp, uint32_t ncols, TailPatterns::Pattern* keep) {
         permute_csr(H, rp, cp, rowp, cols, src);
+        if (keep) *keep = {rowp, cols};
         D.n = H.n;
         D.ncols = ncols;
         D.nnz = H.nnz();
@@ -332,7 +334,8 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
         const HostLevel& H = h.lv[l];
         DevLevel& D = lv_[l];
         D.n = H.A.n;
-        upload_csr(D.A, H.A, D.new_of_old, D.new_of_old, H.A.n);
+        TailPatterns* keep = D.n <= kTailMaxRows ? &small[l] : nullptr;
+        upload_csr(D.A, H.A, D.new_of_old, D.new_of_old, H.A.n, keep ? &keep->m[0] : nullptr);
         std::vector<double> inv(D.n);
         for (uint32_t i = 0; i < D.n; ++i) inv[D.new_of_old[i]] = H.inv_diag[i];
         if (has64_) {
@@ -357,7 +360,7 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
         HIP_OK(hipStreamSynchronize(stream_));
         if (l + 1 < L) {
             const auto& cperm = lv_[l + 1].new_of_old;
-            upload_csr(D.P, H.P, D.new_of_old, cperm, H.P.ncols);
+            upload_csr(D.P, H.P, D.new_of_old, cperm, H.P.ncols, keep ? &keep->m[2] : nullptr);
             // R = P^T in the reference order: coarse row c lists fine rows
             // ascending in the reference numbering.
             HCsr R;
@@ -376,7 +379,7 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
                     R.vals[cur[c]] = H.P.vals[q];
                     ++cur[c];
                 }
-            upload_csr(D.R, R, cperm, D.new_of_old, H.P.n);
+            upload_csr(D.R, R, cperm, D.new_of_old, H.P.n, keep ? &keep->m[1] : nullptr);
         }
     }
     phase("matrices, transfers, SELL copies");
@@ -392,7 +395,7 @@ bool DeviceAmg::build(const HostHierarchy& h, const AmgConfig& cfg, bool reorder
             lu_.upper = upload(lu.upper, stream_);
         }
     }
-    build_tail();
+    build_tail(small);
     const uint32_t n0 = lv_[0].n;
     d_perm0_ = upload(lv_[0].new_of_old, stream_);
     partial_stride_ = std::max<uint64_t>({spmv_groups<double>(lv_[0].A), spmv_groups<float>(lv_[0].A), 4096});
@@ -755,7 +758,7 @@ bool pack_tail(const std::vector<uint32_t>& rowp, const std::vector<uint32_t>& c
 // coarsest, at least two, whose matrices fit its lanes and whose vectors fit
 // LDS (160 KiB). Mean removals of the constant null space are launches
 // between the sweeps: such hierarchies keep the launches.
-void DeviceAmg::build_tail() {
+void DeviceAmg::build_tail(const std::vector<TailPatterns>& small) {
     Tail& t = tail_;
     const uint32_t L = uint32_t(lv_.size());
     t.first = L;
@@ -774,11 +777,8 @@ void DeviceAmg::build_tail() {
         bool ok = true;
         for (int m = 0; ok && m < (t.first == L ? 1 : 3); ++m) {
             const DevCsr& M = m == 0 ? D.A : m == 1 ? D.R : D.P;
-            std::vector<uint32_t> rowp(size_t(M.n) + 1), cols(M.nnz);
-            HIP_OK(hipMemcpyAsync(rowp.data(), M.rowp, rowp.size() * 4, hipMemcpyDeviceToHost, stream_));
-            HIP_OK(hipMemcpyAsync(cols.data(), M.cols, cols.size() * 4, hipMemcpyDeviceToHost, stream_));
-            HIP_OK(hipStreamSynchronize(stream_));
-            ok = pack_tail(rowp, cols, M.ncols, p[m]);
+            const auto& pattern = small[t.first - 1].m[m];
+            ok = pack_tail(pattern.rowp, pattern.cols, M.ncols, p[m]);
         }
         if (!ok) break;
         packs.push_back(std::move(p));
@@ -789,11 +789,30 @@ void DeviceAmg::build_tail() {
         t.first = L;
         return;
     }
+    // One allocation and one copy: the arrays one after the other, then the
+    // values, which a kernel gathers, and the level descriptors.
+    std::vector<unsigned char> image;
     auto put = [&](const auto& v) {
-        auto* d = upload(v, stream_);
-        t.mem.push_back(d);
-        return d;
+        const size_t at = (image.size() + 15) & ~size_t(15);
+        image.resize(at + v.size() * sizeof(v[0]));
+        if (!v.empty()) std::memcpy(image.data() + at, v.data(), v.size() * sizeof(v[0]));
+        return at;
     };
+    struct Places {
+        size_t ctl, cols, groups, lrows, lcols, src, vals;
+    };
+    std::vector<std::array<Places, 3>> places(L - t.first);
+    size_t values = 0;
+    auto matrices = [&](uint32_t k) { return t.first + k + 1 == L ? 1 : 3; };
+    for (uint32_t k = 0; k < places.size(); ++k)
+        for (int m = 0; m < matrices(k); ++m) {
+            const TailPack& p = packs[places.size() - 1 - k][m];
+            places[k][m] = {put(p.ctl), put(p.cols), put(p.groups), put(p.lrows), put(p.lcols), put(p.src), values};
+            values += (p.src.size() + 1) & ~size_t(1);
+        }
+    const size_t first_value = (image.size() + 15) & ~size_t(15), levels = first_value + values * 8;
+    t.mem = dalloc<unsigned char>(levels + places.size() * sizeof(TailLevel));
+    HIP_OK(hipMemcpy(t.mem, image.data(), image.size(), hipMemcpyHostToDevice));
     t.host.resize(L - t.first);
     uint32_t at = 0;
     for (uint32_t k = 0; k < t.host.size(); ++k) {
@@ -805,25 +824,25 @@ void DeviceAmg::build_tail() {
         H.x = at;
         H.b = at + D.n + 1;
         at += 2 * D.n + 2;
-        auto& p = packs[t.host.size() - 1 - k];
-        for (int m = 0; m < (l + 1 == L ? 1 : 3); ++m) {
+        for (int m = 0; m < matrices(k); ++m) {
+            const TailPack& p = packs[t.host.size() - 1 - k][m];
+            const Places& o = places[k][m];
             const DevCsr& M = m == 0 ? D.A : m == 1 ? D.R : D.P;
             TailMat& X = m == 0 ? H.A : m == 1 ? H.R : H.P;
             X.n = M.n;
-            X.ngroups = uint32_t(p[m].groups.size());
-            std::copy(p[m].first, p[m].first + kTailWaves, X.first);
-            std::copy(p[m].count, p[m].count + kTailWaves, X.count);
-            X.ctl = put(p[m].ctl);
-            X.cols = reinterpret_cast<const uint4*>(put(p[m].cols));
-            X.groups = put(p[m].groups);
-            X.lrows = put(p[m].lrows);
-            X.lcols = put(p[m].lcols);
-            double* v = dalloc<double>(p[m].src.size());
-            t.mem.push_back(v);
+            X.ngroups = uint32_t(p.groups.size());
+            std::copy(p.first, p.first + kTailWaves, X.first);
+            std::copy(p.count, p.count + kTailWaves, X.count);
+            X.ctl = reinterpret_cast<const uint32_t*>(t.mem + o.ctl);
+            X.cols = reinterpret_cast<const uint4*>(t.mem + o.cols);
+            X.groups = reinterpret_cast<const uint4*>(t.mem + o.groups);
+            X.lrows = reinterpret_cast<const uint4*>(t.mem + o.lrows);
+            X.lcols = reinterpret_cast<const uint16_t*>(t.mem + o.lcols);
+            double* v = reinterpret_cast<double*>(t.mem + first_value) + o.vals;
             X.vals = v;
-            X.lvals = v + p[m].lane_values;
-            const uint32_t n = uint32_t(p[m].src.size());
-            const uint32_t* src = put(p[m].src);
+            X.lvals = v + p.lane_values;
+            const uint32_t n = uint32_t(p.src.size());
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(t.mem + o.src);
             tail_values_kernel<<<grid_for(n), kBlock, 0, stream_>>>(n, src, M.v64, v);
             if (m == 0) t.refill.push_back({l, n, src, v});
         }
@@ -831,8 +850,7 @@ void DeviceAmg::build_tail() {
     t.cells = at;
     t.stage = at + 3 * (lv_[t.first].n + 1);
     t.lds_bytes = (t.stage + stage_cells) * sizeof(double);
-    t.dev = dalloc<TailLevel>(t.host.size());
-    t.mem.push_back(t.dev);
+    t.dev = reinterpret_cast<TailLevel*>(t.mem + levels);
     for (const auto kernel : {coarse_tail_kernel<false>, coarse_tail_kernel<true>})
         HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    int(kLds)));

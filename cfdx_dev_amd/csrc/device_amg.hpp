@@ -406,9 +406,16 @@ private:
         std::vector<TailLevel> host;
         TailLevel* dev = nullptr;
         std::vector<Refill> refill;
-        std::vector<void*> mem;  // its device arrays
+        unsigned char* mem = nullptr;  // its device arrays
     };
-    void build_tail();
+    // Host patterns of a level's A, R and P in the solve ordering.
+    struct TailPatterns {
+        struct Pattern {
+            std::vector<uint32_t> rowp, cols;
+        };
+        Pattern m[3];
+    };
+    void build_tail(const std::vector<TailPatterns>& small);
     void upload_tail();  // after new Chebyshev coefficients
     void refill_tail();  // after new values of the levels' CSR copies
     Tail tail_;
