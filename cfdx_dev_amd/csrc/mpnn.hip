@@ -686,9 +686,8 @@ __global__ __launch_bounds__(kBlock) void encode_bwd_kernel(uint32_t n, const fl
 
 // out[y][p] = sum of gpart[b][p] over b in [y * per, min((y + 1) * per, rows))
 // in row order. The parameter gradient is reduced in two such stages with a
-// fixed grouping (per = kGradChunk tiles, then all chunk sums), so the sum is
-// deterministic and the reduction has enough parallelism.
-constexpr uint32_t kGradChunk = 24;
+// grouping fixed by the tile count (grad_chunk tiles, then all chunk sums), so
+// the sum is deterministic and the reduction has enough parallelism.
 __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(uint32_t rows, uint32_t per,
                                                             const float* __restrict__ gpart,
                                                             float* __restrict__ out) {
@@ -765,6 +764,18 @@ __global__ void loss_value_kernel(const double* __restrict__ scal, double* __res
 
 inline uint32_t grid_of(uint64_t n) { return uint32_t((n + kBlock - 1) / kBlock); }
 inline uint32_t tiles_of(uint32_t n) { return (n + kTile - 1) / kTile; }
+
+// Tiles a thread of the first reduction stage adds, one after the other; the
+// second adds the chunk sums the same way, so the two serial lengths are kept
+// alike: the square root of the tile count (2.1M nodes: second stage 63 us,
+// 177 with chunks of 64 and 477 with chunks of 24, which suit 70k nodes; the
+// first stage 294, 304 and 309). Up to 24 tiles take one stage.
+inline uint32_t grad_chunk(uint32_t tiles) {
+    uint32_t c = 24;
+    while (uint64_t(c) * c < tiles) ++c;
+    return c;
+}
+inline uint32_t grad_chunks(uint32_t tiles) { return (tiles + grad_chunk(tiles) - 1) / grad_chunk(tiles); }
 inline uint32_t red_grid(uint32_t n) { return std::min<uint32_t>(grid_of(n), kMaxPartBlocks); }
 // Persistent inference grid: 256 CUs x 4 resident workgroups (VGPR-bound).
 constexpr uint32_t kWaveGrid = 256 * 4;
@@ -942,8 +953,9 @@ void Mpnn::backward(DeviceAmg& amg, const float* ge, float* grad_dev) {
         gm_ = mpnn_alloc<float>(uint64_t(cap_) * kHid);
     }
     // tile partials plus one row per chunk of the two-stage reduction
-    const uint64_t cap_tiles = tiles_of(cap_);
-    const uint64_t need = (cap_tiles + (cap_tiles + kGradChunk - 1) / kGradChunk) * kMpnnParams;
+    // (never fewer for more tiles)
+    const uint32_t cap_tiles = tiles_of(cap_);
+    const uint64_t need = (uint64_t(cap_tiles) + grad_chunks(cap_tiles)) * kMpnnParams;
     if (gpart_cap_ < need) {
         MPNN_HIP(hipStreamSynchronize(st));
         mpnn_free(gpart_);
@@ -958,14 +970,14 @@ void Mpnn::backward(DeviceAmg& amg, const float* ge, float* grad_dev) {
         mix_t_kernel<<<grid_of(uint64_t(n) * 4), kBlock, 0, st>>>(n, g.rowp, g.cols, g.vals, s_, gm_, gh2_, gh_);
     }
     encode_bwd_kernel<<<tiles, kBlock, 0, st>>>(n, last_r_, s_, scal_, gh_, mask_[0], gpart_);
-    const uint32_t chunks = (tiles + kGradChunk - 1) / kGradChunk;
+    const uint32_t chunk = grad_chunk(tiles), chunks = grad_chunks(tiles);
     if (chunks <= 1) {
         grad_reduce_kernel<<<grid_of(kMpnnParams), kBlock, 0, st>>>(tiles, tiles, gpart_, grad_dev);
     } else {
         // Chunk sums go to the rows after the tiles' rows (the buffer holds
         // tiles + chunks rows, see the allocation above), then are summed.
         float* csum = gpart_ + size_t(tiles) * kMpnnParams;
-        grad_reduce_kernel<<<dim3(grid_of(kMpnnParams), chunks), kBlock, 0, st>>>(tiles, kGradChunk, gpart_, csum);
+        grad_reduce_kernel<<<dim3(grid_of(kMpnnParams), chunks), kBlock, 0, st>>>(tiles, chunk, gpart_, csum);
         grad_reduce_kernel<<<grid_of(kMpnnParams), kBlock, 0, st>>>(chunks, chunks, csum, grad_dev);
     }
 }
