@@ -160,19 +160,6 @@ void sell_values(DevCsr& D, hipStream_t s, bool first) {
     }
 }
 
-void scatter_d2d(uint32_t n, const uint32_t* perm, const double* src, double* dst, hipStream_t s) {
-    scatter_perm_kernel<double, double><<<grid_for(n), kBlock, 0, s>>>(n, perm, src, dst);
-}
-void gather_d2d(uint32_t n, const uint32_t* perm, const double* src, double* dst, hipStream_t s) {
-    gather_perm_kernel<double, double><<<grid_for(n), kBlock, 0, s>>>(n, perm, src, dst);
-}
-void scatter_d2f(uint32_t n, const uint32_t* perm, const double* src, float* dst, hipStream_t s) {
-    scatter_perm_kernel<double, float><<<grid_for(n), kBlock, 0, s>>>(n, perm, src, dst);
-}
-void gather_f2d(uint32_t n, const uint32_t* perm, const float* src, double* dst, hipStream_t s) {
-    gather_perm_kernel<float, double><<<grid_for(n), kBlock, 0, s>>>(n, perm, src, dst);
-}
-
 DeviceAmg::~DeviceAmg() { release(); }
 
 void DeviceAmg::release() {
@@ -508,10 +495,6 @@ static void launch_spmv(const DevCsr& M, const T* x, Init init, Epi epi, hipStre
     if (nb == 0) return;
     spmv_stream_kernel<T, Init, Epi><<<nb, kBlock, 0, s>>>(sizeof(T) == 8 ? M.blocks : M.blocks32, nb, M.rowp, M.cols,
                                                                   vals_of<T>(M), x, init, epi);
-}
-
-void DeviceAmg::spmv64_level(uint32_t l, const double* x, double* y) {
-    launch_spmv<double>(lv_[l].A, x, InitZero<double>{}, EpiStore<double>{y}, stream_);
 }
 
 template <class T>

@@ -114,12 +114,6 @@ struct SolveStats {
 // SELL copy); first: the padding slots too.
 void sell_values(DevCsr& D, hipStream_t s, bool first);
 
-// Caller <-> solve ordering moves on the device (new_of_old on the device).
-void scatter_d2d(uint32_t n, const uint32_t* perm, const double* src, double* dst, hipStream_t s);
-void gather_d2d(uint32_t n, const uint32_t* perm, const double* src, double* dst, hipStream_t s);
-void scatter_d2f(uint32_t n, const uint32_t* perm, const double* src, float* dst, hipStream_t s);
-void gather_f2d(uint32_t n, const uint32_t* perm, const float* src, double* dst, hipStream_t s);
-
 // Work memory of the allocation-free PCG: a fixed device array of
 // kNoAllocScratchBytes per GPU (file-scope in device_amg.hip), laid out in
 // kNoAllocAlign-byte aligned parts. noalloc_scratch returns its address on
@@ -325,9 +319,6 @@ public:
     bool collect_pairs(const double* b, const std::vector<uint64_t>& iterations, double tol, float* r_out,
                        float* e_out, uint32_t& got, SolveStats& st, std::string& err);
     Level0View level0() const;
-    // y = A x on level l, FP64, solve ordering (each row summed in the
-    // reference's entry order).
-    void spmv64_level(uint32_t l, const double* x, double* y);
     // y = A x on the finest level, FP32, solve ordering.
     void spmv32(const float* x, float* y);
     // r = b - A x on the finest level, FP32, solve ordering.
@@ -357,7 +348,6 @@ public:
     }
 
     hipStream_t stream() const { return stream_; }
-    const std::vector<uint32_t>& perm0() const { return lv_[0].new_of_old; }
 
 private:
     template <class T>

@@ -1636,7 +1636,7 @@ FvMesh::~FvMesh() { release(); }
 
 void FvMesh::release() {
     for (double** p : {&px, &py, &pz, &fcx, &fcy, &fcz, &fsx, &fsy, &fsz, &ccx, &ccy, &ccz, &vol, &vol_caller,
-                       &work_coeff, &work_bsrc, &work_diag, &work_rhs, &work_grad, &work_phi,
+                       &work_coeff, &work_diag, &work_grad,
                        &mom_ugrad, &bc_f64, &slot_coeff,
                        &wls_a0, &wls_a1, &wls_a2, &wls_fac, &wls_nd, &wls_sig, &wls_V, &wls_cond})
         dfree(*p);
@@ -1931,16 +1931,6 @@ void FvMesh::geometry_out(double* fc_aos, double* fs_aos, double* cc_aos, double
     dfree(tmp);
 }
 
-void FvMesh::ensure_work() {
-    if (work_coeff) return;
-    work_coeff = dalloc<double>(nf);
-    work_bsrc = dalloc<double>(nf);
-    work_phi = dalloc<double>(nf);
-    work_diag = dalloc<double>(nc);
-    work_rhs = dalloc<double>(nc);
-    work_grad = dalloc<double>(4 * uint64_t(nc));
-}
-
 // Slot stencils (geometry only): built on first use.
 void FvMesh::ensure_slots() {
     if (slots_built) return;
@@ -2022,6 +2012,7 @@ void FvMesh::ensure_wls_cache(const uint8_t* h_bt, const uint8_t* d_bt) {
 
 // Records (gx, gy, gz, 0) per internal cell of the field p[i * ps].
 void FvMesh::gauss_gradient_internal(const uint8_t* d_bct, const double* d_bcv, const double* p, uint32_t ps) {
+    if (!work_grad) work_grad = dalloc<double>(4 * uint64_t(nc));
     ensure_slots();
     gauss_gradient_kernel<true><<<grid_for(nc), kBlock, 0, stream>>>(
         nc, slot_D, slots_of(*this), patch, npatch, d_bct, d_bcv, Soa3{fcx, fcy, fcz},
@@ -2182,7 +2173,6 @@ bool FvMesh::has_fixed_pressure(const uint8_t* h_pbt) const {
 const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const double* h_pbv, double rho,
                                                      const double* d_rAU, const double* d_phi, const double* d_p,
                                                      uint64_t ref, double* d_vals, double* d_rhs) {
-    ensure_work();
     const bool fixed = has_fixed_pressure(h_pbt);
     const bool eliminate = !fixed && nc > 1 && ref < nc;
     const PressurePlan& plan = row_plan(eliminate, uint32_t(eliminate ? ref : 0));
@@ -2218,7 +2208,8 @@ const PressurePlan& FvMesh::pressure_assemble_device(const uint8_t* h_pbt, const
 
 const PressurePlan& FvMesh::diffusion_assemble_device(double gamma, const double* d_source, const double* d_fval,
                                                       const uint8_t* d_fneu, double* d_vals, double* d_rhs) {
-    ensure_work();
+    if (!work_coeff) work_coeff = dalloc<double>(nf);
+    if (!work_diag) work_diag = dalloc<double>(nc);
     const PressurePlan& plan = pressure_plan(false, 0);
     clear_err();
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
@@ -2390,7 +2381,6 @@ void FvMesh::velocity_correct_device(const double* d_hbya, const double* d_rau, 
 void FvMesh::rhie_chow_flux_device(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt,
                                    const double* h_pbv, double rho, const double* d_hbya, const double* d_p,
                                    const double* d_rau, double* d_phi) {
-    ensure_work();
     upload_bcs(h_vbt, h_vbv, h_pbt, h_pbv, false, nullptr);
     const uint32_t npp = std::max<uint32_t>(npatch, 1);
     const uint8_t* d_vbt = bc_u8;

@@ -55,8 +55,7 @@ struct FvMesh {
     double* vol_caller = nullptr;  // cell volumes in the caller's numbering
     int *err = nullptr, *h_err = nullptr;  // error flags: device and host address of pinned memory
     // work
-    double *work_coeff = nullptr, *work_bsrc = nullptr, *work_diag = nullptr,
-           *work_rhs = nullptr, *work_grad = nullptr, *work_phi = nullptr;
+    double *work_coeff = nullptr, *work_diag = nullptr, *work_grad = nullptr;
     // momentum side: velocity WLS gradients (three records a cell), flags, and
     // per patch (last: internal faces) whether faces are non-orthogonal, then
     // whether their geometry leaves that undefined
@@ -131,7 +130,6 @@ struct FvMesh {
     void upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv, bool raw_pbt, int* flags);
     void clear_err();
     int stencil_dimension() const;
-    void ensure_work();
     double* scr(size_t slot, uint64_t count);
     void cells_in(const double* caller, double* internal, int comps);
     void cells_out(const double* internal, double* caller, int comps);
