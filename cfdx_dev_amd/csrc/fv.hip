@@ -501,7 +501,7 @@ struct Near {
 
 // LDS of a workgroup that assembles rows of up to D + 1 entries beside nrec
 // staged records: the rows take the records' place once those are read.
-// Hexahedra (6 slots) take 36 KB and polyhedra up to kRowSlots 48 KB, so three
+// Hexahedra (6 slots) take 36 KB and polyhedra up to kRowSlots 50 KB, so three
 // or more workgroups, what the registers allow, share a CU's 160 KB.
 constexpr uint32_t kRowSlots = 12;
 constexpr uint32_t kMomNear = 2;  // records a momentum row stages: cell, fields
@@ -2315,10 +2315,10 @@ void FvMesh::wls_gradient_device(const uint8_t* h_bt, const double* h_bv, double
     check_err("boundary WLS gradient: invalid geometry, boundary data or stencil size");
 }
 
-// One stream-ordered pass, synchronised once at the end for the error flag:
-// viscosity check and the non-orthogonality scan set device flags that the
-// gradient, face and cell kernels read (the WLS velocity gradients are only
-// computed when a face is non-orthogonal and diffusion is active).
+// One stream-ordered pass, synchronised once at the end for the error flag. The
+// velocity gradients are only computed when a face that counts is
+// non-orthogonal (geometry and boundary types: known on the host) and diffusion
+// is active (a device flag that the packing kernel sets from the viscosity).
 const PressurePlan& FvMesh::momentum_assemble_device(const uint8_t* h_vbt, const double* h_vbv, const double* d_mu,
                                                      const double* d_phi, const double* d_gradp,
                                                      const double* d_body, const double* d_U, bool bounded,
