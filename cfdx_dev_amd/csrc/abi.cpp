@@ -1145,6 +1145,7 @@ cfdxhip_status cfdxhip_fv_pressure_pattern(cfdxhip_fv* fv, const uint8_t* pbt, s
         const bool fixed = m.npatch ? m.has_fixed_pressure(pbt) : false;
         const bool eliminate = !fixed && m.nc > 1 && ref < m.nc;
         const PressurePlan& pl = m.pressure_plan(eliminate, uint32_t(eliminate ? ref : 0));
+        m.prepare_rows(eliminate, uint32_t(eliminate ? ref : 0));
         *n_rows = pl.n;
         *nnz = pl.nnz;
         if (rowp) std::memcpy(rowp, pl.h_rowp.data(), pl.h_rowp.size() * 4);
@@ -1284,6 +1285,7 @@ cfdxhip_status cfdxhip_fv_momentum_pattern(cfdxhip_fv* fv, size_t* n_rows, size_
     if (!fv || !n_rows || !nnz) return CFDXHIP_ERR_INVALID_ARGUMENT;
     return fv_guarded(fv, [&]() {
         const PressurePlan& pl = fv->mesh.pressure_plan(false, 0);
+        fv->mesh.prepare_rows(false, 0);
         *n_rows = pl.n;
         *nnz = pl.nnz;
         if (rowp) std::memcpy(rowp, pl.h_rowp.data(), pl.h_rowp.size() * 4);

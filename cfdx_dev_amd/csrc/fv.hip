@@ -207,7 +207,9 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
                                                            const uint32_t* __restrict__ patch, uint32_t npatch,
                                                            const uint8_t* __restrict__ kind, Soa3 fc, Soa3 fs,
                                                            Soa3 cc, const double* __restrict__ vol,
+                                                           const uint32_t* __restrict__ face_old,
                                                            double4* __restrict__ cell, Slots sl,
+                                                           uint8_t* __restrict__ slot_sorted,
                                                            int* __restrict__ err) {
 #pragma clang fp contract(off)
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
@@ -225,6 +227,15 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
             continue;
         }
         const uint32_t f = cf[coff[c] + q];
+        // The slot's place in the cell's faces by caller id (a face listed
+        // twice keeps its order).
+        const uint32_t id = face_old[f];
+        uint32_t before = 0;
+        for (uint32_t x = 0; x < deg; ++x) {
+            const uint32_t other = face_old[cf[coff[c] + x]];
+            before += other < id || (other == id && x < q);
+        }
+        slot_sorted[size_t(before) * nc + c] = uint8_t(q);
         const bool own = owner[f] == c;
         sl.face[idx] = own ? f : f | kFaceReversed;
         sl.s.set(idx, own ? fs.get(f) : mul3(fs.get(f), -1.0));
@@ -1950,25 +1961,12 @@ void FvMesh::ensure_slots() {
     slot_sz = dalloc<double>(m);
     // Each cell's slots in ascending caller face id (the order of the
     // reference's face loop accumulations).
-    {
-        std::vector<uint8_t> sorted(m, 0);
-        std::vector<uint32_t> cold(nc);
-        for (uint32_t c = 0; c < nc; ++c) cold[h_cell_new[c]] = c;
-        parallel_for(nc, 0, [&](uint64_t i) {
-            const uint32_t c = cold[i];
-            const uint32_t b = h_coff[c], deg = h_coff[c + 1] - b;
-            uint32_t order[256];
-            for (uint32_t q = 0; q < deg && q < 256; ++q) order[q] = q;
-            std::sort(order, order + std::min<uint32_t>(deg, 256),
-                      [&](uint32_t x, uint32_t y) { return h_cf[b + x] < h_cf[b + y]; });
-            for (uint32_t k = 0; k < deg && k < 256; ++k) sorted[uint64_t(k) * nc + i] = uint8_t(order[k]);
-        });
-        slot_sorted = upload(sorted.data(), m);
-    }
+    slot_sorted = dalloc<uint8_t>(m);
     const Soa3 fc{fcx, fcy, fcz}, fs{fsx, fsy, fsz}, cc{ccx, ccy, ccz};
     clear_err();
     slot_build_kernel<<<grid_for(nc), kBlock, 0, stream>>>(nc, D, coff, cfaces, owner, neigh, patch, npatch,
-                                                           patch_kind, fc, fs, cc, vol, cell_rec, slots_of(*this), err);
+                                                           patch_kind, fc, fs, cc, vol, face_old, cell_rec, slots_of(*this),
+                                                           slot_sorted, err);
     HIP_OK(hipStreamSynchronize(stream));
     check_err("cell stencils: degenerate face distances");
     slots_built = true;
@@ -2141,13 +2139,23 @@ const PressurePlan& FvMesh::pressure_plan(bool eliminate, uint32_t ref) {
     return red;
 }
 
-// The plan with its row maps, which only the assemblies need: the pattern and
-// the calls that read nothing else take meshes that have no slot stencils.
+// The plan with its row maps, which only the assemblies need: the calls that
+// read nothing but the pattern take meshes that have no slot stencils.
 const PressurePlan& FvMesh::row_plan(bool eliminate, uint32_t ref) {
     pressure_plan(eliminate, ref);
     PressurePlan& plan = eliminate ? pressure_red : pressure_full;
     if (!plan.row_start) map_rows(plan, eliminate ? ref : 0xffffffffu);
     return plan;
+}
+
+// A pattern query is followed by assemblies: lays the maps out ahead where the
+// mesh has stencils. What fails here is raised by the assembly that meets it.
+void FvMesh::prepare_rows(bool eliminate, uint32_t ref) {
+    try {
+        row_plan(eliminate, ref);
+    } catch (const std::exception&) {
+        (void)hipGetLastError();
+    }
 }
 
 // Row maps of plan (row and column ref left out; ~0: none).

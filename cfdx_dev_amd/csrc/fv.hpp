@@ -106,6 +106,7 @@ struct FvMesh {
     void mass_flux_device(const uint8_t* d_vbt, const double* d_vbv, double rho, const double* d_U, double* d_phi);
     const PressurePlan& pressure_plan(bool eliminate, uint32_t ref);
     const PressurePlan& row_plan(bool eliminate, uint32_t ref);
+    void prepare_rows(bool eliminate, uint32_t ref);
     bool has_fixed_pressure(const uint8_t* h_pbt) const;
     const PressurePlan& pressure_assemble_device(const uint8_t* h_pbt, const double* h_pbv, double rho,
                                                  const double* d_rAU, const double* d_phi, const double* d_p,
