@@ -6,8 +6,8 @@
 // one down to the coarsest and back up instead. The vectors of those levels
 // live in LDS, the matrix in hand in registers over all sweeps of a smoothing
 // pass, and a phase (a sweep, a residual, a transfer) costs one barrier. On a
-// 12^3 box (1727 + 406 + 57 + 14 rows, 6 + 6 sweeps) the cycle takes 73 us
-// against 45 launches of 4.5 us.
+// 12^3 box (1727 + 406 + 57 + 14 rows, 6 + 6 sweeps) the cycle takes 76 us
+// (under the kernel trace) against 45 launches of 4.5 us.
 //
 // Matrix layout: a row of at most 64 entries belongs to one lane and takes
 // batches of eight slots there; a lane holds at most 8 batches in registers

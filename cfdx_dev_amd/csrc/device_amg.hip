@@ -983,7 +983,7 @@ bool DeviceAmg::fetch_scalars(uint32_t count, uint32_t first) {
 
 // Waits until the first `count` workgroups of the kernel launched last have
 // signalled ticket_. Polling pinned memory sees them sooner than a stream synchronisation
-// (17 FGMRES steps on 70k rows: 3780 us so, 3890 that way); a launch that takes
+// (17 FGMRES steps on 67k rows: 3780 us so, 3890 that way); a launch that takes
 // longer than some milliseconds, or fails, is left to the runtime.
 void DeviceAmg::await(int count) {
     const volatile unsigned long long* done = h_done_;
@@ -1364,7 +1364,7 @@ inline uint32_t gs_tiles(uint32_t j) { return j == 0 ? 1u : (j + kGsTile - 1) / 
 //   partials[2j + 2]   = w . w
 // blockIdx.y takes kGsTile basis vectors; the sums of a workgroup are formed by
 // wavefronts, stored, and closed by one thread a sum (one block sum after the
-// other, two barriers each, took 10.9 us a step of 70k rows,
+// other, two barriers each, took 10.9 us a step of 67k rows,
 // averaged over a cycle of 17; 9.1 us so, most of it the loads).
 __global__ __launch_bounds__(kBlock) void gs_dot_kernel(uint32_t npairs, size_t ld, uint32_t j,
                                                        const double* __restrict__ V, const double* __restrict__ w,

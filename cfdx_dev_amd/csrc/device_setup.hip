@@ -430,7 +430,7 @@ __global__ __launch_bounds__(kBlock) void gershgorin_sd_kernel(const RefreshView
 // Rows above kGershgorinRow entries, listed longest first: one wavefront each, 64
 // terms formed at a time and added in order, a chain of 6 ns an entry. Coarse
 // levels hold their long rows side by side: with the wavefront that holds a row
-// of 64 also summing its long ones, a refresh of 232k cells spent 1204 us here.
+// of 64 also summing its long ones, a refresh of 222k cells spent 1204 us here.
 // With a wavefront each the whole refresh went from 6410 to 5398 us.
 constexpr uint32_t kGershgorinRow = 48;
 __global__ __launch_bounds__(kBlock) void gershgorin_long_kernel(const RefreshView* __restrict__ views, uint32_t slot,

@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void slot_build_kernel(uint32_t nc, uint32_
 
 // Cells go to workgroups by xcd_block: each XCD takes one contiguous range, so
 // that the records a cell and its neighbours share are fetched into one L2
-// rather than into most of them (a 232k-cell channel's pressure rows: 40 us in
+// rather than into most of them (a 222k-cell channel's pressure rows: 40 us in
 // launch order, 31 so).
 __device__ __forceinline__ uint32_t cell_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
@@ -1735,9 +1735,9 @@ void FvMesh::create(int device, uint64_t np_, const double* hx, const double* hy
     // touch about as few lines in it as on the curve (at most half as many
     // again): then no field is permuted at all.
     // Lexicographic numberings of boxes and channels touch 1.05 times the
-    // curve's lines, random ones 9 times. A 232k-cell channel kept as numbered
-    // assembles its pressure in 98 us, moved to another local order in 112 (its
-    // six fields pass through a gather); a random 128^3 box assembled as
+    // curve's lines, random ones 9 times. A 222k-cell channel kept as numbered
+    // assembles its pressure in 71 us, moved onto the curve in 81 (its fields
+    // pass through gathers); a random 128^3 box assembled as
     // numbered would fetch a line for each of its 66M values.
     // The curve itself touches 1.4 to 1.7 times the fewest lines that any
     // order could, so a numbering within twice the fewest (lexicographic ones
@@ -2267,7 +2267,7 @@ void FvMesh::ensure_momentum_work() {
 // pressure type], written by the host into pinned memory and fetched by one
 // small kernel, which also clears the call's device flags. Pressure types other
 // than 1 read as zero-gradient unless raw_pbt. (Two copies of a few
-// bytes and a fill took 10 us of a 232k-cell pressure assembly's 90.)
+// bytes and a fill took 10 us of a 222k-cell pressure assembly's 90.)
 void FvMesh::upload_bcs(const uint8_t* h_vbt, const double* h_vbv, const uint8_t* h_pbt, const double* h_pbv,
                         bool raw_pbt, int* flags) {
     const size_t npp = std::max<uint32_t>(npatch, 1);

@@ -1011,7 +1011,7 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(uint32_t n, const T* __res
 // updates every component at once, each with the operations of the sequential
 // elimination. The back substitution subtracts a row's terms in ascending
 // column order, a chain that only lane ii can follow, so its products are
-// formed by the lanes and read in order, by lane reads: 17 FGMRES steps on 70k
+// formed by the lanes and read in order, by lane reads: 17 FGMRES steps on 67k
 // rows take 3580 us so, 3680 with shuffles (11 us a solve of order 16). One lane
 // with its arrays in scratch memory took 24 us a solve.
 template <class T>

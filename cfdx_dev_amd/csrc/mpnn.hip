@@ -549,7 +549,7 @@ __global__ __launch_bounds__(kBlock) void decode_bwd_kernel(uint32_t n, const fl
 // Out: gh2 = gh + (dL/dX)[:, :32] (residual + self path), gm = (dL/dX)[:, 32:],
 // per-tile partials of dL/dW (X^T gz) and dL/db (sum gz). Bound by the latency
 // of the neighbour gathers, so by the tiles resident: 23 KB of LDS a tile hold
-// six a CU, which takes the 1097 tiles of 70k nodes in one go (47 KB, with
+// six a CU, which takes the 1050 tiles of 67k nodes in one go (47 KB, with
 // dL/dX and the FP32 gz in places of their own, held three: 18.2 us
 // a layer, now 15.5).
 __global__ __launch_bounds__(kBlock) void layer_bwd_kernel(
@@ -768,7 +768,7 @@ inline uint32_t tiles_of(uint32_t n) { return (n + kTile - 1) / kTile; }
 // Tiles a thread of the first reduction stage adds, one after the other; the
 // second adds the chunk sums the same way, so the two serial lengths are kept
 // alike: the square root of the tile count (2.1M nodes: second stage 63 us,
-// 177 with chunks of 64 and 477 with chunks of 24, which suit 70k nodes; the
+// 177 with chunks of 64 and 477 with chunks of 24, which suit 67k nodes; the
 // first stage 294, 304 and 309). Up to 24 tiles take one stage.
 inline uint32_t grad_chunk(uint32_t tiles) {
     uint32_t c = 24;
@@ -1071,7 +1071,7 @@ struct Scoped {
 // reordering kernels read and write across the bus, and the call waits once, at
 // its end. (Pageable copies of the doubles and a device allocation per vector
 // and call, which waits for the device when it is freed, took 100 of the 445 us
-// of a 70k-node estimate and gradient.)
+// of a 67k-node estimate and gradient.)
 namespace {
 template <class S, class D>
 void convert_host(uint32_t n, const S* from, D* to) {
